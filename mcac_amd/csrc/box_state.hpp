@@ -10,15 +10,17 @@ namespace mcac_dev {
 constexpr int kBlock = 256;            // threads per block (4 waves of 64)
 constexpr int kFilterBlocks = 128;     // contact-search filter grid
 constexpr int kSolveBlocks = 256;      // pair-solve grid (one block per CU)
-constexpr long long kChunk = 4096;     // sphere pairs per block the host sizes the grid form's grid by
-constexpr long long kMinChunk = 256;   // minimum sphere pairs per solve chunk (one per thread)
 constexpr int kMaxVisit = 2048;        // visited cells handled with an LDS prefix
 constexpr int kMaxPlan = 4096;         // filtered candidates planned in LDS
 constexpr int kOverlapSlots = 16;      // contacts kept per sphere row (multi-kernel merge)
 constexpr int kSmallMerge = 256;       // merged aggregates up to this size use one fused kernel
 constexpr int kFusedMerge = 512;       // overlap-correction merges up to this size run in one workgroup
 constexpr int kStepCands = 32;         // k_step solves up to this many survivors itself
-constexpr long long kStepPairs = 16384;  // ... holding up to this many sphere pairs
+constexpr long long kStepPairs = 1 << 18;  // ... holding up to this many sphere pairs (with the mover's)
+constexpr long long kStepExactPairs = 1 << 14;  // ... where the move is so long that most pairs take the exact test
+constexpr long long kStepWorst = 1 << 15;  // a mover that may meet more pairs than this in one survivor takes the grid form,
+constexpr int kStepNarrow = 128;       // unless it has at most this many spheres itself,
+constexpr long long kStepNarrowWorst = 1 << 20;  // up to this many pairs
 constexpr int kStepMover = 1024;       // movers up to this size may take k_step
 constexpr int kThreadPairs = 4;        // candidates with this few sphere pairs are solved by one thread
 constexpr int kPendingSolve = -1;      // StepRecord.status: pairs left for k_solve

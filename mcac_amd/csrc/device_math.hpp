@@ -128,4 +128,53 @@ __device__ __forceinline__ double swept_sphere(double p1x, double p1y, double p1
     return res;
 }
 
+// Sound pre-test of swept_sphere.  A finite result means that the sphere of
+// radius r1 at p1, moved along the segment t dir, t in [0, dist], comes within
+// r1 + r2 of an image of sphere 2; with dist / 2 + r1 + r2 below half the box
+// only the image nearest to the segment's middle can.  d is that image's offset
+// from p1; the margin is far above the rounding of box-sized coordinates.  A NaN
+// passes.
+struct SweepTest {
+    double dx, dy, dz, dist, L, inv_L, margin, limit;
+    double hx, hy, hz;  // half the move
+    bool usable;  // unit direction and a forward move (what the bound assumes)
+};
+__device__ __forceinline__ SweepTest sweep_test(const double dir[3], double dist, double L) {
+    SweepTest s;
+    s.dx = dir[0];
+    s.dy = dir[1];
+    s.dz = dir[2];
+    s.dist = dist;
+    s.L = L;
+    s.inv_L = 1.0 / L;
+    s.margin = 4e-9 * L;
+    s.limit = 0.45 * L - 0.5 * dist;  // radius sums up to this keep the nearest image the only one
+    s.hx = 0.5 * dist * s.dx;
+    s.hy = 0.5 * dist * s.dy;
+    s.hz = 0.5 * dist * s.dz;
+    const double n2 = s.dx * s.dx + s.dy * s.dy + s.dz * s.dz;
+    s.usable = __builtin_fabs(n2 - 1.0) <= 1e-9 && dist >= 0.0;
+    return s;
+}
+// Offset of the image nearest to the segment's middle (h: that middle's offset).
+__device__ __forceinline__ double nearest_image(double d, double h, const SweepTest &s) {
+    return d - s.L * __builtin_rint((d - h) * s.inv_L);
+}
+// earliest (when it passes): a bound below the travel to contact.  With t the
+// point of the segment nearest to the image, at distance e, contact at s means
+// s >= t - sqrt(R^2 - e^2) (by sqrt(h + a^2) <= sqrt(h) + a for the part a of
+// the image ahead of the segment's end).
+__device__ __forceinline__ bool sweep_may_touch(const SweepTest &s, double d0, double d1, double d2, double radii,
+                                                double *earliest = nullptr) {
+    double t = d0 * s.dx + d1 * s.dy + d2 * s.dz;
+    t = t < 0.0 ? 0.0 : (t > s.dist ? s.dist : t);
+    const double e0 = d0 - t * s.dx, e1 = d1 - t * s.dy, e2 = d2 - t * s.dz;
+    const double R = radii + s.margin;
+    const double h = R * R - (e0 * e0 + e1 * e1 + e2 * e2);
+    // single precision is enough for a bound: one part in 10^4 of a root below
+    // the radii, on the safe side
+    if (earliest) *earliest = t - 1.0001 * static_cast<double>(__builtin_amdgcn_sqrtf(static_cast<float>(h))) - s.margin;
+    return !(h < 0.0);
+}
+
 }  // namespace mcac_dev

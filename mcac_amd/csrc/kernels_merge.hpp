@@ -95,6 +95,18 @@ __device__ __forceinline__ void publish_merge(const MergeArgs &a, const mcac_mer
 }
 
 // ------------------------------------------------------------------ fused merge (n <= kSmallMerge)
+struct MergeLds {
+    double diffpos[3], refpos[3], r[3];
+    int ok;
+    int sidx[kSmallMerge];
+    double dcs[kSmallMerge], vols[kSmallMerge], rads[kSmallMerge], surfs[kSmallMerge];
+    double rlx[kSmallMerge], rly[kSmallMerge], rlz[kSmallMerge];
+    int nrow[kSmallMerge];
+    double crow[kSmallMerge * 8];
+    double V, svr2;
+    mcac_merge_result res;
+};
+
 // One block merges; thread 0 ends with the result in res_out.  Used by
 // k_merge_small and by the finishing block of a step that found a contact.
 // Global loads are issued in two batches (member indices with the keeper's
@@ -106,16 +118,11 @@ __device__ __forceinline__ void publish_merge(const MergeArgs &a, const mcac_mer
 // merge takes those positions from mover_ref instead of reading them back,
 // and thread q also rewrites that sphere when the mover is the one removed.
 __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeArgs &a, mcac_merge_result &res_out,
-                                                  const double *mover_ref) {
-    __shared__ double diffpos[3], refpos[3], r[3];
-    __shared__ int ok;
-    __shared__ int sidx[kSmallMerge];
-    __shared__ double dcs[kSmallMerge], vols[kSmallMerge], rads[kSmallMerge], surfs[kSmallMerge];
-    __shared__ double rlx[kSmallMerge], rly[kSmallMerge], rlz[kSmallMerge];
-    __shared__ int nrow[kSmallMerge];
-    __shared__ double crow[kSmallMerge * 8];
-    __shared__ double s_V, s_svr2;
-    __shared__ mcac_merge_result s_res;
+                                                  const double *mover_ref, MergeLds &u) {
+    double *const diffpos = u.diffpos, *const refpos = u.refpos, *const r = u.r;
+    int *const sidx = u.sidx, *const nrow = u.nrow;
+    double *const dcs = u.dcs, *const vols = u.vols, *const rads = u.rads, *const surfs = u.surfs;
+    double *const rlx = u.rlx, *const rly = u.rly, *const rlz = u.rlz, *const crow = u.crow;
     const int n = a.n_k + a.n_r;
     const int k = a.keep;
     const bool mover_keeps = a.keep == a.magg;
@@ -175,7 +182,7 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
         // (aggregat_list.cpp:375-378, aggregat.cpp:496-535)
         // contact(moving sphere, other sphere) in the reference's argument order
         const double *p1 = mover_keeps ? m4 : o4, *p2 = mover_keeps ? o4 : m4;
-        ok = contact(p1[0], p1[1], p1[2], p1[3], p2[0], p2[1], p2[2], p2[3], a.L) ? 1 : 0;
+        u.ok = contact(p1[0], p1[1], p1[2], p1[3], p2[0], p2[1], p2[2], p2[3], a.L) ? 1 : 0;
         const double mpos[3] = {m4[0], m4[1], m4[2]}, opos[3] = {o4[0], o4[1], o4[2]};
         for (int l = 0; l < 3; ++l) {
             const double dcontact = periodic_distance(opos[l] - mpos[l], a.L);
@@ -183,7 +190,7 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
         }
     }
     lds_barrier();
-    if (!ok) {
+    if (!u.ok) {
         if (threadIdx.x == 0) {
             mcac_merge_result res{};
             res.keeper = a.keep;
@@ -293,9 +300,9 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
         b.dpcell[dsr] = -1;
         b.cslot[a.rem] = -1;
         for (int l = 0; l < 3; ++l) r[l] = rr[l];
-        s_V = V;
-        s_svr2 = svr2;
-        mcac_merge_result &res = s_res;
+        u.V = V;
+        u.svr2 = svr2;
+        mcac_merge_result &res = u.res;
         res.keeper = k;
         res.removed = a.rem;
         res.n = n;
@@ -339,8 +346,8 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
             rmax = smax(rmax, rads[i] + dcs[i]);       // aggregat.cpp:462
             arg = arg + vols[i] * (dcs[i] * dcs[i]);   // aggregat.cpp:476
         }
-        const double V = s_V;
-        const double rg = __builtin_sqrt(__builtin_fabs((arg + 3. / 5. * s_svr2) / V));  // aggregat.cpp:481
+        const double V = u.V;
+        const double rg = __builtin_sqrt(__builtin_fabs((arg + 3. / 5. * u.svr2) / V));  // aggregat.cpp:481
         b.armax[k] = rmax;
         b.dpr[dsk] = rmax;
         b.arg[k] = rg;
@@ -373,7 +380,7 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
             overlapping /= static_cast<double>(inter);
             coord = static_cast<double>(inter) / static_cast<double>(n);
         }
-        mcac_merge_result res = s_res;
+        mcac_merge_result res = u.res;
         res.rmax = rmax;
         res.rg = rg;
         res.overlapping = overlapping;
@@ -384,7 +391,8 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
 
 __global__ __launch_bounds__(kBlock) void k_merge_small(DevBox b, MergeArgs a) {
     __shared__ mcac_merge_result res;
-    merge_small_block(b, a, res, nullptr);
+    __shared__ MergeLds u;
+    merge_small_block(b, a, res, nullptr, u);
     if (threadIdx.x == 0) publish_merge(a, res);
 }
 

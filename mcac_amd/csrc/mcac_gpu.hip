@@ -457,11 +457,21 @@ int settle_handovers(mcac_box *b) {
     return 0;
 }
 
+// The one-launch form: the finishing block solves the survivors itself.  Its
+// solve takes about 2 us per 256 spheres of survivors and 64 spheres of mover,
+// so a narrow mover may meet large partners; a wide mover among wide partners
+// is spread over a grid (searches of 100-sphere movers among 150-sphere
+// aggregates: 11 us in one block, 24 us as a grid with its barrier; 700 x 700:
+// 109 us as a grid).
+bool fits_one_launch(const mcac_box *b, int n_mov) {
+    const long long worst = static_cast<long long>(n_mov) * b->max_count;
+    return n_mov <= kStepMover && (worst <= kStepWorst || (n_mov <= kStepNarrow && worst <= kStepNarrowWorst));
+}
+
 // A step that one block can take whole: the one-launch form (small mover, few
 // sphere pairs possible), the mover moved by the finishing block, not timed.
 bool one_block_step(const mcac_box *b, int n_mov, bool timed) {
-    const bool fused = n_mov <= kStepMover && static_cast<long long>(n_mov) * b->max_count <= kStepPairs;
-    return fused && n_mov <= 4 * kBlock && !timed;
+    return fits_one_launch(b, n_mov) && n_mov <= 4 * kBlock && !timed;
 }
 
 // Entries a step may have to sweep (cells of a window for a mover of rmax at
@@ -576,7 +586,7 @@ int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, do
     hipEvent_t *ev = b->sev[slot];
     const bool timed = b->timing > 0 && (seq - b->timing_base) % static_cast<unsigned long long>(b->timing) == 0;
     // one launch when the mover is small enough for the finishing block
-    const bool fused = n_mov <= kStepMover && static_cast<long long>(n_mov) * b->max_count <= kStepPairs;
+    const bool fused = fits_one_launch(b, n_mov);
     // filter grid sized to the expected work: entries of the visited cells
     // (1.5x the mean cell occupancy) plus the dirty list, one per thread
     int grid = kFilterBlocks;
@@ -628,13 +638,13 @@ int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, do
         if (timed) hipExtLaunchKernelGGL(k_step, dim3(grid), dim3(kBlock), 0, bstream(b), ev[0], ev[1], 0, b->d, a);
         else hipLaunchKernelGGL(k_step, dim3(grid), dim3(kBlock), 0, bstream(b), b->d, a);
     } else if (b->grid_solve) {
-        // one launch: the filter grid, widened to the solve chunks that a
-        // survivor as large as the largest aggregate would bring, at most
+        // one launch: the filter grid, widened to the sphere tiles that four
+        // survivors as large as the largest aggregate would bring, at most
         // grid_blocks (a block of it holds 81 KB of LDS, one per CU, all of
         // them resident together for its barrier, whose arrivals are atomics
         // on one counter)
-        const double chunks = std::ceil(static_cast<double>(n_mov) * static_cast<double>(b->max_count) / kChunk);
-        const int g2 = std::min(b->grid_blocks, std::max(grid, static_cast<int>(std::min<double>(kFilterBlocks, chunks))));
+        const double tiles = std::ceil(4.0 * static_cast<double>(b->max_count) / 64);
+        const int g2 = std::min(b->grid_blocks, std::max(grid, static_cast<int>(std::min<double>(kFilterBlocks, tiles))));
         if (timed) hipExtLaunchKernelGGL(k_step_grid, dim3(g2), dim3(kBlock), 0, bstream(b), ev[0], ev[1], 0, b->d, a);
         else hipLaunchKernelGGL(k_step_grid, dim3(g2), dim3(kBlock), 0, bstream(b), b->d, a);
     } else if (timed) {
