@@ -15,7 +15,8 @@ constexpr int kMaxPlan = 4096;         // filtered candidates planned in LDS
 constexpr int kOverlapSlots = 16;      // contacts kept per sphere row (multi-kernel merge)
 constexpr int kSmallMerge = 256;       // merged aggregates up to this size use one fused kernel
 constexpr int kFusedMerge = 512;       // overlap-correction merges up to this size run in one workgroup
-constexpr int kStepCands = 32;         // k_step solves up to this many survivors itself
+constexpr int kMaxSteps = 8;           // steps of one box in one launch
+constexpr int kStepCands = 64;         // k_step solves up to this many survivors itself
 constexpr long long kStepPairs = 1 << 18;  // ... holding up to this many sphere pairs (with the mover's)
 constexpr long long kStepExactPairs = 1 << 14;  // ... where the move is so long that most pairs take the exact test
 constexpr long long kStepWorst = 1 << 15;  // a mover that may meet more pairs than this in one survivor takes the grid form,
@@ -37,7 +38,11 @@ struct SearchState {
     int newcell;
     int pad;
     unsigned long long gate;   // seq of a gated step that found a contact (0: open)
-    unsigned long long tick;   // k_step blocks: finished << 56 | appended << 32 | visited
+    // steps of a launch, by number: blocks finished << 56 | survivors << 32 |
+    // visited, and survivors appended; steps whose search is finished
+    unsigned long long step_tick[kMaxSteps];
+    unsigned int step_nfilt[kMaxSteps];
+    unsigned int steps_done, pad2;
     unsigned long long fp32_tested, fp32_kept, fp32_missed;  // FP32 broad-phase accounting
     // persistent step engine (k_step_engine)
     unsigned long long eng_done;      // 2 * last job index completed + 1 if that step closed the gate
@@ -50,15 +55,16 @@ struct SearchState {
     unsigned int grid_bar, grid_fail;
 };
 
-// Record published to pinned host memory by the last block of a search.
+// Record published to pinned host memory by the last block of a search; the
+// part before `merge` is all that a step without a contact fills in.
 struct StepRecord {
     double dist, move;
     long long ms, os, oagg;
     int contact, status;
     unsigned long long nquery, nfilt, npairs;
     int skipped, dirty_count;  // step skipped behind a closed gate; dirty list length after it
-    mcac_merge_result merge;   // merge done in the same launch (merged_inline)
     int merged_inline, m_new_start, m_new_cap, pad;
+    mcac_merge_result merge;   // merge done in the same launch (merged_inline)
     unsigned long long seq;    // written last (system-scope release)
 };
 
@@ -116,19 +122,28 @@ struct DevBox {
     int *walk_n;               // entries of each walk row (alphas only)
     SearchState *ss;
     MergeState *ms;
+    struct StepPick *picks;            // finished searches of a launch of several steps, by step number
+    struct SearchArgs *sargs;          // and their arguments (k_steps_group)
     struct EngineJob *eng_jobs;        // persistent engine: block 0's copy of each queued job, by ring slot
     unsigned long long *eng_closed;    // persistent engine: eng_done's word of each completed job, by ring slot
 };
 
 struct SearchArgs {
+    // what later steps of the same launch take of this one (the moved set): the
+    // move without contact, computed by the host (aggregat.cpp:148-161)
     int src;
+    int nc_cell;               // reference cell after it
+    double srmax;
+    double nc_com[3], nc_ref[3];  // new CoM and CoM - relative CoM
     int n_mov, start;          // mover size and member segment (host mirror)
-    int known;                 // host supplies the mover's CoM, rmax, relative CoM and window
-    double sx, sy, sz, srmax, srx, sry, srz;
+    int known, nc_ok;          // host supplies the mover's CoM, rmax, relative CoM and window; and the move
+    double sx, sy, sz, srx, sry, srz;
     int b1[3], len[3];
     int dirty_n;               // dirty-list length when this step runs
     int dirty_slot;            // dirty-list index this step's move appends, -1 when already listed
     int dirty_pos;             // dirty-list index of the mover after this step
+    int run_dirty;             // dirty-list length when the first step of its launch runs
+    int vg;                    // blocks on this step in a launch of several
     int n_div;
     int cap;
     int n_built;               // items in the CSR cell list
@@ -142,17 +157,14 @@ struct SearchArgs {
     StepRecord *out;           // pinned host record
     unsigned long long seq;
     int gated;                 // pipelined step: closes the gate on contact, skipped behind it
-    unsigned long long released;  // gate values up to this one are open for this step
     int automerge;             // merge in the same launch on contact when small enough
+    unsigned long long released;  // gate values up to this one are open for this step
     int prec;                  // 0 FP64; 1 FP32 capsule prune of cell entries; 2 as 1 plus miss count
     float margin32;            // FP32 prune margin added to the radius sum [m]
     long long pool_used, pool_cap;  // member pool state when this step runs
-    int nc_ok;                 // the host computed the move without contact (known mover):
-    int nc_cell;               //   its reference cell,
-    double nc_com[3], nc_ref[3];  //   new CoM and CoM - relative CoM (aggregat.cpp:148-161)
 };
 
-// Bounds of the visited cells of a batched step, supplied by the host from
+// Bounds of the visited cells of an engine step, supplied by the host from
 // its copy of the cell starts (n = 0: the kernel reads them from cstart).
 struct CellTable {
     int n;

@@ -20,16 +20,60 @@
 
 namespace mcac_dev {
 
-__device__ __forceinline__ void append_candidate(const DevBox &b, const SearchArgs &a, int id, int rank, double d) {
-    unsigned int slot = atomicAdd(&b.ss->nfilt, 1u);
-    if (slot < static_cast<unsigned int>(a.cap)) {
-        b.cand_db[slot] = d;
-        b.cand_rank[slot] = rank;
-        b.cand_id[slot] = id;
-    } else {
-        atomicOr(&b.ss->overflow, 1u);
+// Where a search's survivors go: the box's candidate buffer (the grid forms).
+struct BoxSink {
+    const DevBox &b;
+    int cap;
+    __device__ __forceinline__ void operator()(int id, int rank, double d) const {
+        const unsigned int slot = atomicAdd(&b.ss->nfilt, 1u);
+        if (slot < static_cast<unsigned int>(cap)) {
+            b.cand_db[slot] = d;
+            b.cand_rank[slot] = rank;
+            b.cand_id[slot] = id;
+        } else {
+            atomicOr(&b.ss->overflow, 1u);
+        }
     }
-}
+};
+
+// The moves of a step's predecessors in the same launch, assumed without
+// contact (a step behind a contact is not carried out): the newest one of each
+// mover, in LDS.  The search takes these aggregates from here instead of from
+// the box, where the moves are carried out at the launch's end.  n = 0 and
+// self = -1 for a step that has no predecessor.
+struct Moved {
+    int n;                                   // entries (id -1: superseded by a later one)
+    int self;                                // the step's own mover's entry, -1: it has not moved
+    int id[kMaxSteps], cell[kMaxSteps];
+    double x[kMaxSteps], y[kMaxSteps], z[kMaxSteps], r[kMaxSteps];  // centre of mass and rmax
+    double rx[kMaxSteps], ry[kMaxSteps], rz[kMaxSteps];             // centre - relative centre: its spheres' origin
+};
+
+// Positions of spheres as a step sees them: an aggregate with entry m >= 0 of
+// the moved set has its spheres at that move's origin + relative position, the
+// values its move stores (aggregat.cpp:148-161).
+template <bool kMoved> struct Places {
+    const DevBox &b;
+    const Moved *mv;
+    __device__ __forceinline__ void operator()(int m, int sp, double &x, double &y, double &z) const {
+        if (kMoved && m >= 0) {
+            x = mv->rx[m] + b.srx[sp];
+            y = mv->ry[m] + b.sry[sp];
+            z = mv->rz[m] + b.srz[sp];
+        } else {
+            x = b.sx[sp];
+            y = b.sy[sp];
+            z = b.sz[sp];
+        }
+    }
+    __device__ __forceinline__ int entry(int id) const {
+        int e = -1;
+        if (kMoved)
+            for (int m = 0; m < mv->n; ++m)
+                if (mv->id[m] == id) e = m;
+        return e;
+    }
+};
 
 // FP32 broad phase: can the candidate's bounding sphere (centre c, radius rc)
 // come within the mover's radius rs of the sweep segment p1 + t dir, t in
@@ -107,10 +151,14 @@ struct FilterLds {
 
 // Filter work of block vb of the vg blocks on this step: the aggregates of the
 // reference's visited Verlet cells and the dirty list, bounding sweep,
-// candidate append (shared by k_filter, k_step and k_step_batch).  With skip
-// the work is read-only (a step behind a closed gate appends nothing).
+// survivors to `append` (shared by every form of the search).  With skip the
+// work is read-only (a step behind a closed gate appends nothing).  nd: entries
+// of the dirty list.  kMoved: the aggregates of the moved set are taken from
+// there, by the first block.
+template <bool kMoved, class Sink>
 __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, const SearchArgs &a, unsigned vb,
-                                                           unsigned vg, const CellBounds &cb, bool skip, FilterLds &u) {
+                                                           unsigned vg, const CellBounds &cb, bool skip, FilterLds &u,
+                                                           int nd, const Moved *mv, const Sink &append) {
     int *const pre = u.pre, *const cbeg = u.cbeg;
     const int n = a.n_div;
     int b1i, b1j, b1k, li, lj, lk, V;
@@ -202,10 +250,22 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
         total = pre[V];
     } else {
         total = b.cstart[n * n * n];  // every entry of the build
+        lds_barrier();
     }
     // one index space: cell entries, then the aggregates moved since the build
     // (at their current cell), so that both kinds run side by side
-    const int nd = a.dirty_n;
+    int gone[kMaxSteps];  // the mover and the moved set: not taken from the box
+    int own = a.src;
+    if (kMoved)
+        for (int m = 0; m < kMaxSteps; ++m) gone[m] = m < mv->n ? mv->id[m] : -1;
+    auto elsewhere = [&](int id) {
+        bool e = id == own;
+        if (kMoved) {
+#pragma unroll
+            for (int m = 0; m < kMaxSteps; ++m) e = e || id == gone[m];
+        }
+        return e;
+    };
     unsigned long long n32 = 0, kept32 = 0, miss32 = 0;
     const float fx = static_cast<float>(sx), fy = static_cast<float>(sy), fz = static_cast<float>(sz);
     const float fr = static_cast<float>(sr), fdx = static_cast<float>(a.dir[0]), fdy = static_cast<float>(a.dir[1]);
@@ -220,6 +280,20 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
             return kInf;
         return swept_sphere(sx, sy, sz, sr, x, y, z, r, a.dir[0], a.dir[1], a.dir[2], a.lpm, a.L);
     };
+    if (kMoved && vb == 0u && static_cast<int>(threadIdx.x) < mv->n && mv->id[threadIdx.x] >= 0 &&
+        mv->id[threadIdx.x] != own) {
+        const int m = threadIdx.x, c = mv->cell[m];
+        const int oi = window_offset(c / (n * n), b1i, n), oj = window_offset((c / n) % n, b1j, n),
+                  ok = window_offset(c % n, b1k, n);
+        if (oi < li && oj < lj && ok < lk) {
+            cnt += 1;
+            const double d = bounding(mv->x[m], mv->y[m], mv->z[m], mv->r[m]);
+            if (d < a.lpm && !skip) {
+                append(mv->id[m], (oi * lj + oj) * lk + ok, d);
+                cnt += kAppendOne;
+            }
+        }
+    }
     if (a.prec == 0 && V <= kMaxVisit && total > gstride) {
         // FP64 sweep with several entries per thread (a block that takes a
         // window alone): kSweep entries per pass have their rank searches and
@@ -254,11 +328,11 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
             }
 #pragma unroll
             for (int u = 0; u < kSweep; ++u) {
-                if (rv[u] < 0.0 || idv[u] == a.src) continue;  // past the end, moved since the build, or the mover
+                if (rv[u] < 0.0 || elsewhere(idv[u])) continue;  // past the end, moved since the build, or the mover
                 cnt += 1;
                 const double d = bounding(xv[u], yv[u], zv[u], rv[u]);
                 if (d < a.lpm && !skip) {
-                    append_candidate(b, a, idv[u], rk[u], d);
+                    append(idv[u], rk[u], d);
                     cnt += kAppendOne;
                 }
             }
@@ -266,14 +340,14 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
         for (int i = gtid; i < nd; i += gstride) {  // the dirty list, as below
             const int id = b.dirty_list[i];
             const int c = b.dpcell[i];
-            if (c < 0 || id == a.src) continue;
+            if (c < 0 || elsewhere(id)) continue;
             int oi = window_offset(c / (n * n), b1i, n), oj = window_offset((c / n) % n, b1j, n),
                 ok = window_offset(c % n, b1k, n);
             if (oi >= li || oj >= lj || ok >= lk) continue;
             cnt += 1;
             const double d = bounding(b.dpx[i], b.dpy[i], b.dpz[i], b.dpr[i]);
             if (d < a.lpm && !skip) {
-                append_candidate(b, a, id, (oi * lj + oj) * lk + ok, d);
+                append(id, (oi * lj + oj) * lk + ok, d);
                 cnt += kAppendOne;
             }
         }
@@ -299,7 +373,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
             if (a.prec > 0) {
                 // FP32 broad phase: 16 B per entry; only its survivors read the FP64 row
                 const float4 f = b.cf[pos];
-                if (f.w < 0.f) continue;  // moved since the build
+                if (f.w < 0.f || (kMoved && elsewhere(b.citems[pos]))) continue;  // moved since the build
                 const bool pass = capsule_pass32(fx, fy, fz, fr, f, fdx, fdy, fdz, flpm, fL, a.margin32);
                 n32 += 1;
                 if (!pass) {
@@ -307,7 +381,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
                         const int id2 = b.citems[pos];
                         const double d2 = swept_sphere(sx, sy, sz, sr, b.cpx[pos], b.cpy[pos], b.cpz[pos],
                                                        b.cpr[pos], a.dir[0], a.dir[1], a.dir[2], a.lpm, a.L);
-                        if (id2 != a.src && d2 < a.lpm) miss32 += 1;
+                        if (!elsewhere(id2) && d2 < a.lpm) miss32 += 1;
                     }
                     continue;
                 }
@@ -318,7 +392,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
             y = b.cpy[pos];
             z = b.cpz[pos];
             r = b.cpr[pos];
-            if (r < 0.0 || id == a.src) continue;  // moved since the build, or the mover
+            if (r < 0.0 || elsewhere(id)) continue;  // moved since the build, or the mover
             if (V > kMaxVisit) {
                 const int c = ref_cell(x, y, z, n, a.L);
                 int oi = window_offset(c / (n * n), b1i, n), oj = window_offset((c / n) % n, b1j, n),
@@ -334,7 +408,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
             y = b.dpy[i];
             z = b.dpz[i];
             r = b.dpr[i];
-            if (c < 0 || id == a.src) continue;
+            if (c < 0 || elsewhere(id)) continue;
             int oi = window_offset(c / (n * n), b1i, n), oj = window_offset((c / n) % n, b1j, n),
                 ok = window_offset(c % n, b1k, n);
             if (oi >= li || oj >= lj || ok >= lk) continue;
@@ -343,7 +417,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
         cnt += 1;
         const double d = bounding(x, y, z, r);
         if (d < a.lpm && !skip) {
-            append_candidate(b, a, id, rank, d);
+            append(id, rank, d);
             cnt += kAppendOne;
         }
     }
@@ -364,30 +438,35 @@ __global__ __launch_bounds__(kBlock) void k_filter(DevBox b, SearchArgs a) {
     if (behind_gate(b, a)) return;
     __shared__ FilterLds u;
     const unsigned long long tot =
-        block_sum(filter_phase(b, a, blockIdx.x, gridDim.x, CellBounds{0, 0, 0}, false, u)) & 0xffffffffull;
+        block_sum(filter_phase<false>(b, a, blockIdx.x, gridDim.x, CellBounds{0, 0, 0}, false, u, a.dirty_n, nullptr,
+                                      BoxSink{b, a.cap})) & 0xffffffffull;
     if (threadIdx.x == 0 && tot) atomicAdd(&b.ss->nquery, tot);
 }
 
-// What the last block of a step knows besides the candidates.
-struct StepTotals {
+// A finished search: the contact and the search's counts (aggregat_list.cpp:459-482).
+struct StepPick {
+    double dist;                // distance of the contact, +inf: none
+    long long ms, os, oagg;     // its spheres and other aggregate, -1: none
+    long long tpairs;           // sphere pairs of the survivors
     unsigned long long nquery;  // aggregates of the visited cells tested
     unsigned int nfilt;         // candidates appended (may exceed the capacity)
     int overflow;
     int src_slot;               // packed cell entry of the mover (-1: none)
-    long long tpairs;           // sphere pairs of the survivors
+    int handover;               // survivors left to the grid form: no contact known
 };
 
 // Survivors of a one-launch step (at most kStepCands), kept in LDS by the
 // finishing block: bounding distance, visit rank, label, size and member
-// segment, exact (d, pair) minimum, and the multimap order.
+// segment, moved-set entry, exact (d, pair) minimum, and the multimap order.
 struct StepCands {
     double db[kStepCands], ex[kStepCands];
     long long pair[kStepCands];
-    int rank[kStepCands], id[kStepCands], nk[kStepCands], sk[kStepCands], order[kStepCands];
+    int rank[kStepCands], id[kStepCands], nk[kStepCands], sk[kStepCands], mv[kStepCands], order[kStepCands];
     int pre[kStepCands + 1];  // spheres before each survivor's
+    unsigned int n;           // survivors of a search by one block (may exceed kStepCands)
 };
 
-// Sphere of the mover a thread places in the finishing block, loaded early
+// Sphere of the mover a thread places when it applies a step, loaded early
 // when the mover has at most one sphere per thread.
 struct MoverSphere {
     int loaded;  // the block loaded the mover (uniform)
@@ -459,17 +538,12 @@ union StepLds {
     MergeLds merge;
 };
 
-// Last block of a step: orders the candidates like the reference's multimap,
-// runs its early-exit scan over the exact per-candidate distances (from LDS
-// when lc is given, else cand_exact / cand_pair), moves the aggregate,
-// writes the record (publishing it unless the caller publishes later) and
-// resets the search counters.  Returns (in thread 0) whether the step closed
-// the gate for the steps queued behind it.
-__device__ __forceinline__ bool finish_step(const DevBox &b, const SearchArgs &a, unsigned int F, long long nsrc,
-                                            int ssrc, const StepTotals &t, const MoverSphere &m, StepCands *lc,
-                                            bool publish, MergeLds &u) {
-    bool closed = false;
-    // std::multimap order: (bounding distance, visit rank, label)
+// Orders the F candidates like the reference's std::multimap (bounding
+// distance, visit rank, label) and runs its early-exit scan over the exact
+// distances (from LDS when lc is given, else cand_exact / cand_pair): the
+// contact, in pick, by thread 0.
+__device__ __forceinline__ void scan_candidates(const DevBox &b, unsigned int F, int ssrc, const StepCands *lc,
+                                                int *order, StepPick &pick) {
     if (lc) {
         for (unsigned int c = threadIdx.x; c < F; c += blockDim.x) {
             const double dc = lc->db[c];
@@ -480,7 +554,7 @@ __device__ __forceinline__ bool finish_step(const DevBox &b, const SearchArgs &a
                 const int re = lc->rank[e];
                 pos += (de < dc || (de == dc && (re < rc || (re == rc && lc->id[e] < ic)))) ? 1u : 0u;
             }
-            lc->order[pos] = static_cast<int>(c);
+            order[pos] = static_cast<int>(c);
         }
         if (F > 0) lds_barrier();
     } else {
@@ -493,18 +567,15 @@ __device__ __forceinline__ bool finish_step(const DevBox &b, const SearchArgs &a
                 int re = b.cand_rank[e];
                 pos += (de < dc || (de == dc && (re < rc || (re == rc && b.cand_id[e] < ic)))) ? 1u : 0u;
             }
-            b.order[pos] = static_cast<int>(c);
+            order[pos] = static_cast<int>(c);
         }
         if (F > 0) __syncthreads();  // order and exact distances come from other threads
     }
-    __shared__ double s_ref[3];
-    __shared__ StepRecord srec;  // assembled here, copied to host memory by one wave
-    SearchState *s = b.ss;
     if (threadIdx.x == 0) {
         double closest = kInf;
         int best = -1;
         for (unsigned int pos = 0; pos < F; ++pos) {
-            const int c = lc ? lc->order[pos] : b.order[pos];
+            const int c = order[pos];
             if (closest <= 0.) break;
             if (closest < (lc ? lc->db[c] : b.cand_db[c])) break;
             const double ex = lc ? lc->ex[c] : b.cand_exact[c];
@@ -513,18 +584,37 @@ __device__ __forceinline__ bool finish_step(const DevBox &b, const SearchArgs &a
                 best = c;
             }
         }
-        // every load of this thread comes before its stores (no reloads through global memory)
-        long long ms = -1, os = -1, oagg = -1;
+        pick.dist = closest;
+        pick.ms = pick.os = pick.oagg = -1;
         if (best >= 0) {
             const long long p = lc ? lc->pair[best] : b.cand_pair[best];
             const int k = lc ? lc->id[best] : b.cand_id[best];
             const long long nk = lc ? lc->nk[best] : b.acount[k];
             const int sk = lc ? lc->sk[best] : b.astart[k];
             const long long i = p / nk, j = p - i * nk;
-            ms = b.members[ssrc + i];
-            os = b.members[sk + j];
-            oagg = k;
+            pick.ms = b.members[ssrc + i];
+            pick.os = b.members[sk + j];
+            pick.oagg = k;
         }
+    }
+}
+
+// Carries out a finished search in the box: moves the aggregate, merges on a
+// contact when asked to, writes the record (publishing it unless the caller
+// publishes later) and resets the search counters.  pick is read by thread 0
+// only.  Returns (in thread 0) whether the step closed the gate for the steps
+// queued behind it.
+__device__ __forceinline__ bool apply_step(const DevBox &b, const SearchArgs &a, const StepPick &pick,
+                                           const MoverSphere &m, bool publish, MergeLds &u) {
+    bool closed = false;
+    const long long nsrc = a.n_mov;
+    const int ssrc = a.start;
+    __shared__ double s_ref[3];
+    __shared__ StepRecord srec;  // assembled here, copied to host memory by one wave
+    SearchState *s = b.ss;
+    if (threadIdx.x == 0) {
+        // every load of this thread comes before its stores (no reloads through global memory)
+        const double closest = pick.dist;
         // calcul.cpp:128-130 and aggregat.cpp:148-153
         const int contact = closest <= a.lpm;
         const double move = contact ? closest : a.lpm;
@@ -558,19 +648,18 @@ __device__ __forceinline__ bool finish_step(const DevBox &b, const SearchArgs &a
         StepRecord *o = &srec;
         o->dist = closest;
         o->move = move;
-        o->ms = ms;
-        o->os = os;
-        o->oagg = oagg;
+        o->ms = pick.ms;
+        o->os = pick.os;
+        o->oagg = pick.oagg;
         o->contact = contact;
-        o->status = t.overflow ? MCAC_E_CAPACITY : 0;
-        o->nquery = t.nquery;
-        o->nfilt = t.nfilt;
-        o->npairs = static_cast<unsigned long long>(t.tpairs);
+        o->status = pick.overflow ? MCAC_E_CAPACITY : 0;
+        o->nquery = pick.nquery;
+        o->nfilt = pick.nfilt;
+        o->npairs = static_cast<unsigned long long>(pick.tpairs);
         o->skipped = 0;
         o->merged_inline = 0;
         o->m_new_start = 0;
         o->m_new_cap = 0;
-        o->pad = 0;
         o->dirty_count = a.dirty_n + ((a.apply && a.dirty_slot >= 0) ? 1 : 0);
         for (int l = 0; l < 3; ++l) {
             s->newcom[l] = ncom[l];
@@ -587,9 +676,9 @@ __device__ __forceinline__ bool finish_step(const DevBox &b, const SearchArgs &a
                 b.dirty_list[a.dirty_slot] = a.src;
                 b.dslot[a.src] = a.dirty_slot;
                 s->dirty_count = static_cast<unsigned int>(a.dirty_slot + 1);
-                if (t.src_slot >= 0) {
-                    b.cpr[t.src_slot] = -1.0;
-                    b.cf[t.src_slot].w = -1.f;
+                if (pick.src_slot >= 0) {
+                    b.cpr[pick.src_slot] = -1.0;
+                    b.cf[pick.src_slot].w = -1.f;
                 }
             }
             set_dirty_entry(b, a.dirty_pos, ncom[0], ncom[1], ncom[2], rmax_src, ncell);
@@ -600,7 +689,6 @@ __device__ __forceinline__ bool finish_step(const DevBox &b, const SearchArgs &a
         s->nquery = 0;
         s->overflow = 0;
         s->done_solve = 0;
-        s->tick = 0ull;
         s->grid_bar = 0;
     }
     lds_barrier();  // s_ref
@@ -699,12 +787,15 @@ __device__ __forceinline__ double from_ordered_bits(unsigned long long u) {
 
 // The mover's spheres [i0, i0 + nt) into LDS; returns the radius around centre
 // that holds them (block-uniform).
+template <class Where>
 __device__ __forceinline__ double load_mover_tile(const DevBox &b, SolveLds &u, int ssrc, long long i0, int nt,
-                                                  const double centre[3]) {
+                                                  const double centre[3], int self, const Where &where) {
     double far = 0.0;
     for (int t = threadIdx.x; t < nt; t += blockDim.x) {
         const int sp = b.members[ssrc + i0 + t];
-        const double x = b.sx[sp], y = b.sy[sp], z = b.sz[sp], r = b.sr[sp];
+        double x, y, z;
+        const double r = b.sr[sp];
+        where(self, sp, x, y, z);
         u.mx[t] = x;
         u.my[t] = y;
         u.mz[t] = z;
@@ -725,24 +816,23 @@ __device__ __forceinline__ double load_mover_tile(const DevBox &b, SolveLds &u, 
 }
 
 // One tile: thread t holds sphere number j of candidate cl (counted from the
-// tile's first; cl < 0: no sphere), listed at member slot m, against the nt
-// mover spheres in LDS (numbers i0 ...).  Returns whether some pair of the tile
+// tile's first; cl < 0: no sphere), listed at member slot m, of an aggregate
+// with moved-set entry `entry`, against the nt mover spheres in LDS (numbers i0 ...).  Returns whether some pair of the tile
 // has a finite distance: then u.dmin / u.pmin hold the minima of its ncl (at
 // most kBlock) candidates, candidate cl's for thread cl, where they are at most
 // `best` (thread cl's: the candidate's minimum over earlier tiles; u.pmin stays
 // ~0 where no pair of the tile is).  nk(cl): its size.
-template <class Size>
+template <class Where, class Size>
 __device__ __forceinline__ bool solve_tile(const DevBox &b, const SearchArgs &a, const SweepTest &sw, SolveLds &u,
                                            const double centre[3], double reach, long long i0, int nt, int cl,
-                                           long long j, long long m, int ncl, double best, Size &&nk) {
+                                           long long j, long long m, int entry, const Where &where, int ncl, double best,
+                                           Size &&nk) {
     double x = 0, y = 0, z = 0, r = 0, q0 = 0, q1 = 0, q2 = 0;
     bool keep = false;
     if (cl >= 0) {
         const int sp = b.members[m];
-        x = b.sx[sp];
-        y = b.sy[sp];
-        z = b.sz[sp];
         r = b.sr[sp];
+        where(entry, sp, x, y, z);
         const double d0 = nearest_image(x - centre[0], sw.hx, sw), d1 = nearest_image(y - centre[1], sw.hy, sw),
                      d2 = nearest_image(z - centre[2], sw.hz, sw);
         q0 = centre[0] + d0;
@@ -867,6 +957,7 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
     double centre[3] = {a.sx, a.sy, a.sz};
     if (!a.known) centre[0] = b.ax[a.src], centre[1] = b.ay[a.src], centre[2] = b.az[a.src];
     const SweepTest sw = sweep_test(a.dir, a.lpm, a.L);
+    const Places<false> where{b, nullptr};
     const int n_movers = static_cast<int>((nsrc + kMoverTile - 1) / kMoverTile);
     double reach = 0.0;
     int nt = 0, in_lds = -1;
@@ -875,7 +966,7 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
         lds_barrier();
         nt = static_cast<int>(nsrc - static_cast<long long>(q) * kMoverTile < kMoverTile
                                   ? nsrc - static_cast<long long>(q) * kMoverTile : kMoverTile);
-        reach = load_mover_tile(b, u, ssrc, static_cast<long long>(q) * kMoverTile, nt, centre);
+        reach = load_mover_tile(b, u, ssrc, static_cast<long long>(q) * kMoverTile, nt, centre, -1, where);
         in_lds = q;
     };
     // a few candidates' member segments are loaded once, into LDS
@@ -925,7 +1016,7 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
             for (int q = 0; q < n_movers; ++q) {
                 mover_tile(q);
                 if (solve_tile(b, a, sw, u, centre, reach, static_cast<long long>(q) * kMoverTile, nt, cl, j, m,
-                               c1 - c0 + 1, bd, [&](int e) { return cpre[c0 + e + 1] - cpre[c0 + e]; }) &&
+                               -1, where, c1 - c0 + 1, bd, [&](int e) { return cpre[c0 + e + 1] - cpre[c0 + e]; }) &&
                     static_cast<int>(threadIdx.x) <= c1 - c0 && u.pmin[threadIdx.x] != ~0ull)
                     lexmin(bd, bp, from_ordered_bits(u.dmin[threadIdx.x]), static_cast<long long>(u.pmin[threadIdx.x]));
             }
@@ -947,7 +1038,7 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
                 for (long long w0 = 0; w0 < nk; w0 += kBlock) {
                     const long long j = w0 + threadIdx.x;
                     if (solve_tile(b, a, sw, u, centre, reach, static_cast<long long>(q) * kMoverTile, nt,
-                                   j < nk ? 0 : -1, j, sk + j, 1, bd, [&](int) { return nk; }) &&
+                                   j < nk ? 0 : -1, j, sk + j, -1, where, 1, bd, [&](int) { return nk; }) &&
                         threadIdx.x == 0 && u.pmin[0] != ~0ull)
                         lexmin(bd, bp, from_ordered_bits(u.dmin[0]), static_cast<long long>(u.pmin[0]));
                 }
@@ -994,13 +1085,17 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
         }
     }
     __syncthreads();  // every candidate's minimum before the ordered scan reads them
-    StepTotals t;
-    t.nquery = b.ss->nquery;
-    t.nfilt = b.ss->nfilt;
-    t.overflow = b.ss->overflow != 0u;
-    t.src_slot = b.cslot[a.src];
-    t.tpairs = nsrc * T;
-    finish_step(b, a, F, nsrc, ssrc, t, MoverSphere{0, -1, 0., 0., 0.}, nullptr, true, lds.merge);
+    __shared__ StepPick pick;
+    scan_candidates(b, F, ssrc, nullptr, b.order, pick);
+    if (threadIdx.x == 0) {
+        pick.nquery = b.ss->nquery;
+        pick.nfilt = b.ss->nfilt;
+        pick.overflow = b.ss->overflow != 0u;
+        pick.src_slot = b.cslot[a.src];
+        pick.tpairs = nsrc * T;
+        pick.handover = 0;
+    }
+    apply_step(b, a, pick, MoverSphere{0, -1, 0., 0., 0.}, true, lds.merge);
 }
 
 __global__ __launch_bounds__(kBlock) void k_solve(DevBox b, SearchArgs a) {
@@ -1021,7 +1116,8 @@ __global__ __launch_bounds__(kBlock) void k_step_grid(DevBox b, SearchArgs a) {
     if (behind_gate(b, a)) return;  // every block reads the same gate: the host knows it is skipped
     __shared__ StepLds lds;
     const unsigned long long tot =
-        block_sum(filter_phase(b, a, blockIdx.x, gridDim.x, CellBounds{0, 0, 0}, false, lds.filter)) & 0xffffffffull;
+        block_sum(filter_phase<false>(b, a, blockIdx.x, gridDim.x, CellBounds{0, 0, 0}, false, lds.filter, a.dirty_n,
+                                      nullptr, BoxSink{b, a.cap})) & 0xffffffffull;
     __shared__ int s_ok;
     if (threadIdx.x == 0) {
         if (tot) atomicAdd(&b.ss->nquery, tot);
@@ -1045,25 +1141,45 @@ __global__ __launch_bounds__(kBlock) void k_step_grid(DevBox b, SearchArgs a) {
     solve_phase(b, a, lds);
 }
 
-// One MC step for a small mover, worked on by vg blocks (vb is this one):
+// Survivors of a step: into LDS when one block takes the step, else into the
+// step's share of the box's candidate buffer.
+struct StepSink {
+    const DevBox &b;
+    StepCands &sc;
+    int q, slots;  // the step's number and its share of the buffer (-1: LDS)
+    __device__ __forceinline__ void operator()(int id, int rank, double d) const {
+        if (slots < 0) {
+            const unsigned int c = atomicAdd(&sc.n, 1u);
+            if (c >= static_cast<unsigned int>(kStepCands)) return;  // counted: left to the grid form
+            sc.id[c] = id;
+            sc.rank[c] = rank;
+            sc.db[c] = d;
+        } else {
+            const unsigned int c = atomicAdd(&b.ss->step_nfilt[q], 1u);
+            if (c >= static_cast<unsigned int>(slots)) return;
+            b.cand_id[q * slots + c] = id;
+            b.cand_rank[q * slots + c] = rank;
+            b.cand_db[q * slots + c] = d;
+        }
+    }
+};
+
+// Search of one step, number q of its launch, by vg blocks (vb is this one):
 // every block filters its share of the Verlet window; the last block to finish
-// (ticket) solves the sphere pairs of the survivors itself, one candidate at a
-// time, and finishes the step.  When the survivors hold more pairs than one
-// block should take, it leaves them in place, closes the gate for the steps
-// queued behind and publishes a pending record: the host then launches k_solve
-// for the same step.  With vg == 1 the block is the last one by construction.
-// ct: bounds of the visited cells from the host (in LDS), or null.
-// publish: publish the record (else wave 0 writes its body and the caller
-// publishes the sequence number later, after a system-scope fence).
-// gate_open: the caller knows the gate is open for this step; otherwise the
-// gate is read with the first loads and a step behind it does no more than
-// read-only filter work (the host knows it is skipped: no record).  Returns (in
-// thread 0) whether the step closed the gate for the steps behind it.
-// role (optional, LDS, set by thread 0): 0 the step was skipped behind the
-// gate, 1 this block took part, 2 this block finished the step.
-__device__ __forceinline__ bool step_body(const DevBox &b, const SearchArgs &a, unsigned vb, unsigned vg,
-                                          bool gate_open, const CellTable *ct, bool publish, int *role = nullptr,
-                                          const StepPrefetch *pre = nullptr) {
+// (ticket) solves the sphere pairs of the survivors, orders them and has the
+// contact in pick (thread 0).  More survivors or pairs than one block should
+// take are left to the grid form (pick.handover).  Nothing of the box changes.
+// nd: dirty-list entries; mv: its predecessors' moves (kMoved); ct: bounds of
+// the visited cells from the host (in LDS), or null.  gate_open: the caller
+// knows the gate is open for this step; otherwise the gate is read with the
+// first loads and a step behind it does no more than read-only filter work.
+// Returns 0 for a step behind the gate, 1 where this block took part, 2 where it
+// finished the search, 3 where it leaves it to the grid form (uniform over the
+// block).
+template <bool kMoved>
+__device__ __forceinline__ int search_step(const DevBox &b, const SearchArgs &a, unsigned vb, unsigned vg, int q,
+                                           int nd, const Moved *mv, bool gate_open, const CellTable *ct, StepLds &lds,
+                                           StepCands &sc, StepPick &pick, MoverSphere &mover, const StepPrefetch *pre) {
     // independent loads first, so that their latencies overlap: the gate, the
     // mover's cell entry and sphere indices, the bounds of the visited cells
     const unsigned long long gate = (!gate_open && a.gated) ? b.ss->gate : 0ull;
@@ -1078,7 +1194,7 @@ __device__ __forceinline__ bool step_body(const DevBox &b, const SearchArgs &a, 
     }
     const CellBounds cb = load_cell_bounds(b, a, ct);
     const bool skip = gate != 0ull && gate < a.seq && gate > a.released;
-    MoverSphere mover{mload, msp, 0., 0., 0.};
+    mover = MoverSphere{mload, msp, 0., 0., 0.};
     if (pre) {
         mover = pre->mover;
     } else if (msp >= 0) {
@@ -1086,10 +1202,12 @@ __device__ __forceinline__ bool step_body(const DevBox &b, const SearchArgs &a, 
         mover.ry = b.sry[msp];
         mover.rz = b.srz[msp];
     }
-    __shared__ StepLds lds;
-    const unsigned long long cnt = block_sum(filter_phase(b, a, vb, vg, cb, skip, lds.filter));
-    if (role && threadIdx.x == 0) *role = skip ? 0 : 1;
-    if (skip) return false;
+    if (threadIdx.x == 0) sc.n = 0u;  // filter_phase appends behind a barrier
+    const int share = a.cap / kMaxSteps < kStepCands ? a.cap / kMaxSteps : kStepCands;
+    const StepSink sink{b, sc, q, vg > 1 ? share : -1};
+    const unsigned long long cnt =
+        block_sum(filter_phase<kMoved>(b, a, vb, vg, cb, skip, lds.filter, nd, mv, sink));
+    if (skip) return 0;
     // one atomic per block: finished blocks, appended candidates, visited aggregates
     __shared__ bool last;
     __shared__ unsigned long long s_total;
@@ -1097,84 +1215,79 @@ __device__ __forceinline__ bool step_body(const DevBox &b, const SearchArgs &a, 
         if (threadIdx.x == 0) {
             const unsigned long long mine = kTicketOne + cnt;
             __threadfence();
-            const unsigned long long old = atomicAdd(&b.ss->tick, mine);
+            const unsigned long long old = atomicAdd(&b.ss->step_tick[q], mine);
             last = (old >> 56) == vg - 1u;
             s_total = old + mine;
         }
         __syncthreads();
-        if (!last) return false;
+        if (!last) return 1;
         __threadfence();
-        if (role && threadIdx.x == 0) *role = 2;
+        if (threadIdx.x == 0) {  // for the next launch
+            b.ss->step_tick[q] = 0ull;
+            b.ss->step_nfilt[q] = 0u;
+        }
     } else {
-        if (role && threadIdx.x == 0) *role = 2;
         if (threadIdx.x == 0) s_total = cnt;
-        __syncthreads();  // the block's appended candidates are visible to all its threads
+        lds_barrier();
     }
-    SearchState *s = b.ss;
     const unsigned long long total = s_total;
-    StepTotals t;
-    t.nquery = total & 0xffffffffull;
-    t.nfilt = static_cast<unsigned int>((total >> 32) & 0xffffffull);
-    t.overflow = t.nfilt > static_cast<unsigned int>(a.cap);
-    t.src_slot = src_slot;
-    const unsigned int F = t.overflow ? static_cast<unsigned int>(a.cap) : t.nfilt;
+    const unsigned int nfilt = static_cast<unsigned int>((total >> 32) & 0xffffffull);
+    const unsigned int most = vg > 1 ? static_cast<unsigned int>(share) : static_cast<unsigned int>(kStepCands);
+    const unsigned int F = nfilt < most ? nfilt : most;
     const long long nsrc = a.n_mov;
     const int ssrc = a.start;
-    __shared__ StepCands sc;
-    t.tpairs = 0;
-    if (F > 0) {
+    const Places<kMoved> where{b, mv};
+    const int self = kMoved ? mv->self : -1;
+    if (threadIdx.x == 0) {
+        pick.nquery = total & 0xffffffffull;
+        pick.nfilt = nfilt;
+        pick.overflow = 0;
+        pick.src_slot = src_slot;
+        pick.tpairs = 0;
+        pick.handover = 0;
+    }
+    if (F > 0 || nfilt > F) {
         // survivors into LDS: label, size, member segment, bounding key, and
         // the prefix of the sizes
         long long tp = 0;
         for (unsigned int c = threadIdx.x; c < F; c += blockDim.x) {
-            const int k = b.cand_id[c];
+            if (vg > 1) {
+                sc.id[c] = b.cand_id[q * share + c];
+                sc.db[c] = b.cand_db[q * share + c];
+                sc.rank[c] = b.cand_rank[q * share + c];
+            }
+            const int k = sc.id[c];
             const int nk = b.acount[k];
             tp += nsrc * nk;
-            if (c < static_cast<unsigned int>(kStepCands)) {
-                sc.id[c] = k;
-                sc.nk[c] = nk;
-                sc.sk[c] = b.astart[k];
-                sc.db[c] = b.cand_db[c];
-                sc.rank[c] = b.cand_rank[c];
-            }
+            sc.nk[c] = nk;
+            sc.sk[c] = b.astart[k];
+            sc.mv[c] = where.entry(k);
         }
         const long long tpairs = block_sum(tp);
-        t.tpairs = tpairs;
-        __shared__ bool handover;
+        __shared__ int s_over;
         __shared__ long long s_most;  // most pairs a survivor brings
-        if (threadIdx.x == 0) handover = F > static_cast<unsigned int>(kStepCands) || t.overflow ||
-                                          tpairs > (a.lpm < 0.25 * a.L ? kStepPairs : kStepExactPairs);
-        if (threadIdx.x < 64 && F <= static_cast<unsigned int>(kStepCands)) {  // block_sum's barrier published the sizes
+        if (threadIdx.x == 0) {
+            s_over = nfilt > most || tpairs > (a.lpm < 0.25 * a.L ? kStepPairs : kStepExactPairs);
+            pick.tpairs = tpairs;
+            pick.handover = s_over;
+        }
+        if (threadIdx.x < 64) {  // block_sum's barrier published the sizes
             const int nk = threadIdx.x < F ? sc.nk[threadIdx.x] : 0;
             const int incl = wave_inclusive_scan(nk);
             if (threadIdx.x < F) sc.pre[threadIdx.x + 1] = incl;
-            int most = nk;
+            int big = nk;
             for (int off = 32; off > 0; off >>= 1) {
-                const int o = __shfl_xor(most, off, 64);
-                most = o > most ? o : most;
+                const int o = __shfl_xor(big, off, 64);
+                big = o > big ? o : big;
             }
             if (threadIdx.x == 0) {
                 sc.pre[0] = 0;
-                s_most = nsrc * most;
+                s_most = nsrc * big;
             }
         }
+        static_assert(kStepCands <= 64, "the prefix of the survivors' sizes is one wave's");
         lds_barrier();
-        if (handover) {
-            if (threadIdx.x == 0) {
-                s->tick = 0ull;
-                s->nquery = t.nquery;  // k_solve reports it
-                if (a.gated) s->gate = a.seq;
-                StepRecord *o = a.out;
-                o->status = kPendingSolve;
-                o->contact = 0;
-                o->skipped = 0;
-                if (publish) {
-                    __threadfence_system();
-                    __hip_atomic_store(&o->seq, a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-                }
-            }
-            return a.gated != 0;
-        }
+        if (s_over) return 3;
         // exact sphere-pair distances, lexicographic (d, i, j) minimum per
         // candidate: when every candidate has at most kThreadPairs pairs
         // (monomers), one thread walks a candidate's in (i, j) order (strict <
@@ -1189,8 +1302,11 @@ __device__ __forceinline__ bool step_body(const DevBox &b, const SearchArgs &a, 
                 for (long long p = 0; p < nsrc * nk; ++p) {
                     const long long i = p / nk, j = p - i * nk;
                     const int si = b.members[ssrc + i], sj = b.members[sk + j];
-                    const double d = swept_sphere(b.sx[si], b.sy[si], b.sz[si], b.sr[si], b.sx[sj], b.sy[sj],
-                                                  b.sz[sj], b.sr[sj], a.dir[0], a.dir[1], a.dir[2], a.lpm, a.L);
+                    double x1, y1, z1, x2, y2, z2;
+                    where(self, si, x1, y1, z1);
+                    where(sc.mv[c], sj, x2, y2, z2);
+                    const double d = swept_sphere(x1, y1, z1, b.sr[si], x2, y2, z2, b.sr[sj], a.dir[0], a.dir[1],
+                                                  a.dir[2], a.lpm, a.L);
                     lexmin(bd, bp, d, p);
                 }
                 sc.ex[c] = bd;
@@ -1208,17 +1324,18 @@ __device__ __forceinline__ bool step_body(const DevBox &b, const SearchArgs &a, 
             for (long long i0 = 0; i0 < nsrc; i0 += kMoverTile) {
                 const int nt = static_cast<int>(nsrc - i0 < kMoverTile ? nsrc - i0 : kMoverTile);
                 if (i0 > 0) lds_barrier();
-                const double reach = load_mover_tile(b, u, ssrc, i0, nt, centre);
+                const double reach = load_mover_tile(b, u, ssrc, i0, nt, centre, self, where);
                 for (int w0 = 0; w0 < T; w0 += kBlock) {
                     const int w = w0 + static_cast<int>(threadIdx.x);
-                    int c = -1, j = 0, m = 0;
+                    int c = -1, j = 0, m = 0, e = -1;
                     if (w < T) {
                         c = last_not_above(sc.pre, static_cast<int>(F), w);
                         j = w - sc.pre[c];
                         m = sc.sk[c] + j;
+                        e = sc.mv[c];
                     }
-                    if (solve_tile(b, a, sw, u, centre, reach, i0, nt, c, j, m, static_cast<int>(F), bd,
-                                   [&](int e) { return static_cast<long long>(sc.nk[e]); }) &&
+                    if (solve_tile(b, a, sw, u, centre, reach, i0, nt, c, j, m, e, where, static_cast<int>(F), bd,
+                                   [&](int k) { return static_cast<long long>(sc.nk[k]); }) &&
                         threadIdx.x < F && u.pmin[threadIdx.x] != ~0ull)
                         lexmin(bd, bp, from_ordered_bits(u.dmin[threadIdx.x]),
                                static_cast<long long>(u.pmin[threadIdx.x]));
@@ -1231,84 +1348,306 @@ __device__ __forceinline__ bool step_body(const DevBox &b, const SearchArgs &a, 
             lds_barrier();
         }
     }
-    return finish_step(b, a, F, nsrc, ssrc, t, mover, &sc, publish, lds.merge);
+    scan_candidates(b, F, ssrc, &sc, sc.order, pick);
+    return 2;
 }
 
-__global__ __launch_bounds__(kBlock) void k_step(DevBox b, SearchArgs a) {
-    step_body(b, a, blockIdx.x, gridDim.x, false, nullptr, true);
+// A step left to the grid form: its record says so, and the gate closes for the
+// steps queued behind it (thread 0).
+__device__ __forceinline__ void hand_over(const DevBox &b, const SearchArgs &a, bool publish) {
+    if (a.gated) b.ss->gate = a.seq;
+    StepRecord *o = a.out;
+    o->status = kPendingSolve;
+    o->contact = 0;
+    o->skipped = 0;
+    if (publish) {
+        __threadfence_system();
+        __hip_atomic_store(&o->seq, a.seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
 }
 
-// Steps of many boxes in one launch: block i runs jobs seg[i] .. seg[i+1]-1,
-// consecutive queued steps of one box (at most kMaxBlockJobs), in order; jobs
-// are in pinned host memory.  Small boxes are bound by launch and memory
-// latency, so their steps share launches instead of each taking one.  A step
-// behind a contact (or a hand-over to k_solve) of an earlier job of the block
-// does nothing, as it would in separate launches behind the gate.
-struct StepJob {
+// One MC step for a small mover, searched by vg blocks and carried out by the
+// one that finishes the search.  publish: publish the record (else wave 0
+// writes its body and the caller publishes the sequence number later, after a
+// system-scope fence).  Returns (in thread 0) whether the step closed the gate.
+// role (optional, LDS, set by thread 0): as search_step's result.
+__device__ __forceinline__ bool step_body(const DevBox &b, const SearchArgs &a, unsigned vb, unsigned vg,
+                                          bool gate_open, const CellTable *ct, bool publish, int *role = nullptr,
+                                          const StepPrefetch *pre = nullptr) {
+    __shared__ StepLds lds;
+    __shared__ StepCands sc;
+    __shared__ StepPick pick;
+    MoverSphere mover;
+    const int r = search_step<false>(b, a, vb, vg, 0, a.dirty_n, nullptr, gate_open, ct, lds, sc, pick, mover, pre);
+    if (role && threadIdx.x == 0) *role = r < 2 ? r : 2;
+    if (r < 2) return false;
+    if (r == 3) {
+        if (threadIdx.x == 0) hand_over(b, a, publish);
+        return a.gated != 0;
+    }
+    return apply_step(b, a, pick, mover, publish, lds.merge);
+}
+
+// Kernel arguments read where the launch put them, in constant memory, when
+// they are needed: taken by value, the box's 70 pointers are all loaded first
+// and most of them spilled (219 spilled scalars against 35; a run of 2347
+// monomers 189 ms against 175).
+template <class T> __device__ __forceinline__ const T &kernel_arguments() {
+    using Const = const T __attribute__((address_space(4)));
+    return *(const T *)(Const *)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
+struct StepOne {
     DevBox b;
     SearchArgs a;
-    CellTable cells;
 };
-constexpr int kMaxBlockJobs = 8;
-static_assert(sizeof(DevBox) % sizeof(unsigned long long) == 0 && sizeof(SearchArgs) % sizeof(unsigned long long) == 0 &&
-                  sizeof(CellTable) % sizeof(unsigned long long) == 0,
-              "job copied in 8-byte words");
+__global__ __launch_bounds__(kBlock) void k_step(StepOne) {
+    const StepOne &k = kernel_arguments<StepOne>();
+    step_body(k.b, k.a, blockIdx.x, gridDim.x, false, nullptr, true);
+}
 
-__global__ __launch_bounds__(kBlock) void k_step_batch(const StepJob *jobs, const int *seg) {
-    __shared__ DevBox box;
-    __shared__ SearchArgs args[kMaxBlockJobs];
-    __shared__ CellTable cells[kMaxBlockJobs];
-    __shared__ int s_closed;
-    constexpr int kBoxWords = static_cast<int>(sizeof(DevBox) / sizeof(unsigned long long));
-    constexpr int kArgWords = static_cast<int>(sizeof(SearchArgs) / sizeof(unsigned long long));
-    constexpr int kCellWords = static_cast<int>(sizeof(CellTable) / sizeof(unsigned long long));
-    const int j0 = seg[blockIdx.x];
-    int nj = seg[blockIdx.x + 1] - j0;
-    nj = nj < 0 ? 0 : (nj > kMaxBlockJobs ? kMaxBlockJobs : nj);  // the host never lists more
-    // one round trip: the box (the same for every job of the block), every
-    // job's arguments and cell table
-    unsigned long long *bw = reinterpret_cast<unsigned long long *>(&box);
-    unsigned long long *aw = reinterpret_cast<unsigned long long *>(args);
-    unsigned long long *cw = reinterpret_cast<unsigned long long *>(cells);
-    const int na = nj * kArgWords;
-    for (int i = threadIdx.x; i < kBoxWords + na + nj * kCellWords; i += blockDim.x) {
-        if (i < kBoxWords) {
-            bw[i] = reinterpret_cast<const unsigned long long *>(&jobs[j0].b)[i];
-        } else if (i < kBoxWords + na) {
-            const int q = (i - kBoxWords) / kArgWords, w = (i - kBoxWords) - q * kArgWords;
-            aw[q * kArgWords + w] = reinterpret_cast<const unsigned long long *>(&jobs[j0 + q].a)[w];
-        } else {
-            const int q = (i - kBoxWords - na) / kCellWords, w = (i - kBoxWords - na) - q * kCellWords;
-            cw[q * kCellWords + w] = reinterpret_cast<const unsigned long long *>(&jobs[j0 + q].cells)[w];
+// Several consecutive queued steps of a box in one launch (at most kMaxSteps).
+// A step is a chain of dependent loads of about 8 us in which one workgroup
+// hardly uses its CU, and a step without a contact only moves its mover by a
+// vector that the host knows beforehand.  So all steps of the launch search at
+// the same time, each by its own blocks, against the box as it is before the
+// launch with the moves of its predecessors put in (Moved); the last block to
+// finish carries the steps out in order up to the first contact (or hand-over),
+// behind which the others do nothing, as they would behind the gate.  Every
+// step sees the very values it would see in launches of its own.
+// Eight steps take about as long as one, plus one ticket between blocks.
+struct StepsLds {
+    StepLds lds;
+    StepCands sc;
+    StepPick pick;
+    Moved mv;
+    SearchArgs args[kMaxSteps];
+    StepPick picks[kMaxSteps];
+    StepRecord head[kMaxSteps];
+    int over, last;
+};
+
+// Fills the moved set of step q from its predecessors' arguments.
+template <class Args>
+__device__ __forceinline__ void set_moved(Moved &mv, int q, int src, const Args &args) {
+    if (static_cast<int>(threadIdx.x) < q) {
+        const int p = threadIdx.x;
+        const SearchArgs &e = args(p);
+        int id = e.src;
+        for (int r = p + 1; r < q; ++r)
+            if (args(r).src == e.src) id = -1;  // moved again later
+        mv.id[p] = id;
+        mv.cell[p] = e.nc_cell;
+        mv.x[p] = e.nc_com[0];
+        mv.y[p] = e.nc_com[1];
+        mv.z[p] = e.nc_com[2];
+        mv.r[p] = e.srmax;
+        mv.rx[p] = e.nc_ref[0];
+        mv.ry[p] = e.nc_ref[1];
+        mv.rz[p] = e.nc_ref[2];
+    }
+    if (threadIdx.x == 0) {
+        int self = -1;
+        for (int p = 0; p < q; ++p)
+            if (args(p).src == src) self = p;
+        mv.n = q;
+        mv.self = self;
+    }
+}
+
+// Carries out the nj searched steps in u.args / u.picks in order up to the first
+// contact or hand-over and publishes their records (whole block).
+__device__ __forceinline__ void commit_steps(const DevBox &b, StepsLds &u, int nj) {
+    SearchState *s = b.ss;
+    int f = 0;
+    while (f < nj && !u.picks[f].handover && !(u.picks[f].dist <= u.args[f].lpm)) ++f;
+    constexpr int kHead = static_cast<int>(offsetof(StepRecord, merge) / sizeof(unsigned long long));
+    static_assert(offsetof(StepRecord, merge) % sizeof(unsigned long long) == 0, "record head in 8-byte words");
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    // moves without contact: a wave per step; a mover that moves again later in
+    // the launch is placed by its last move
+    for (int q = wave; q < f; q += kBlock / 64) {
+        const SearchArgs &a = u.args[q];
+        bool later = false;
+        for (int p = q + 1; p < f; ++p) later = later || u.args[p].src == a.src;
+        if (!later)
+            for (int t = lane; t < a.n_mov; t += 64) {
+                const int sp = b.members[a.start + t];
+                b.sx[sp] = a.nc_ref[0] + b.srx[sp];
+                b.sy[sp] = a.nc_ref[1] + b.sry[sp];
+                b.sz[sp] = a.nc_ref[2] + b.srz[sp];
+            }
+        if (lane == 0) {
+            const StepPick &pk = u.picks[q];
+            StepRecord &o = u.head[q];
+            o.dist = pk.dist;
+            o.move = a.lpm;
+            o.ms = pk.ms;
+            o.os = pk.os;
+            o.oagg = pk.oagg;
+            o.contact = 0;
+            o.status = 0;
+            o.nquery = pk.nquery;
+            o.nfilt = pk.nfilt;
+            o.npairs = static_cast<unsigned long long>(pk.tpairs);
+            o.skipped = 0;
+            o.dirty_count = a.dirty_n + (a.dirty_slot >= 0 ? 1 : 0);
+            o.merged_inline = o.m_new_start = o.m_new_cap = o.pad = 0;
+            if (a.dirty_slot >= 0) {  // first move since the cell-list build
+                b.dirty[a.src] = 1;
+                b.dirty_list[a.dirty_slot] = a.src;
+                b.dslot[a.src] = a.dirty_slot;
+                if (pk.src_slot >= 0) {
+                    b.cpr[pk.src_slot] = -1.0;
+                    b.cf[pk.src_slot].w = -1.f;
+                }
+            }
+            if (!later) {
+                b.ax[a.src] = a.nc_com[0];
+                b.ay[a.src] = a.nc_com[1];
+                b.az[a.src] = a.nc_com[2];
+                b.acell[a.src] = a.nc_cell;
+                set_dirty_entry(b, a.dirty_pos, a.nc_com[0], a.nc_com[1], a.nc_com[2], a.srmax, a.nc_cell);
+            }
         }
     }
-    if (threadIdx.x == 0) s_closed = 0;
-    __syncthreads();
-    if (nj == 0 || behind_gate(box, args[0])) return;  // every job of the block is behind the same gate
-    int ran = 0;
-    // the mover's entry slot and spheres of the next job load while a step
-    // runs: no queued step changes them unless it closes the gate (the slot
-    // holds until the next cell-list build, a move keeps the relative
-    // positions, a merge is a contact)
-    StepPrefetch next = prefetch_step(box, args[0]);
-    for (int q = 0; q < nj; ++q) {
-        // the previous step's writes (positions, lists) and its use of the
-        // shared state are complete before the next step starts
-        if (q > 0) __syncthreads();
-        if (s_closed) break;
-        const StepPrefetch cur = next;
-        if (q + 1 < nj) next = prefetch_step(box, args[q + 1]);
-        const bool closed = step_body(box, args[q], 0u, 1u, true, &cells[q], false, nullptr, &cur);
-        ran = q + 1;
-        if (threadIdx.x == 0 && closed) s_closed = 1;
+    if (threadIdx.x == 0) {
+        for (int q = f - 1; q >= 0; --q)
+            if (u.args[q].dirty_slot >= 0) {  // slots are handed out in order
+                s->dirty_count = static_cast<unsigned int>(u.args[q].dirty_slot + 1);
+                break;
+            }
+        s->steps_done = 0u;
     }
-    // the records of the steps that ran, written by wave 0: one system-scope
-    // fence, then their sequence numbers (the host reads them after the launch)
-    if (threadIdx.x == 0 && ran > 0) {
+    __syncthreads();  // the moves are in the box for the step that follows; the heads are in LDS
+    if (wave == kBlock / 64 - 1 && f > 0) {
+        // records of the moves, published while the contact below is carried out
+        for (int i = lane; i < f * kHead; i += 64)
+            reinterpret_cast<unsigned long long *>(u.args[i / kHead].out)[i % kHead] =
+                reinterpret_cast<const unsigned long long *>(&u.head[i / kHead])[i % kHead];
         __threadfence_system();
-        for (int q = 0; q < ran; ++q)
-            __hip_atomic_store(&args[q].out->seq, args[q].seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        if (lane < f)
+            __hip_atomic_store(&u.args[lane].out->seq, u.args[lane].seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+    if (f >= nj) return;
+    if (u.picks[f].handover) {
+        if (threadIdx.x == 0) hand_over(b, u.args[f], true);
+        return;
+    }
+    const MoverSphere mover = load_mover_sphere(b, u.args[f]);
+    apply_step(b, u.args[f], u.picks[f], mover, true, u.lds.merge);
+}
+
+// The rest of a step's launch once its arguments are known: args(p) gives those
+// of step p <= q, fetch(p) loads all of step p's into LDS (for p < nj, when
+// every step has finished its search).
+template <class Args, class Fetch>
+__device__ __forceinline__ void run_steps(const DevBox &b, StepsLds &u, const SearchArgs &a, int q, int nj,
+                                          int nd, unsigned vb, unsigned vg, const Args &args, const Fetch &fetch) {
+    set_moved(u.mv, q, a.src, args);
+    lds_barrier();
+    MoverSphere mover;
+    const int r = search_step<true>(b, a, vb, vg, q, nd, &u.mv, false, nullptr, u.lds, u.sc, u.pick, mover, nullptr);
+    if (r < 2) return;
+    if (threadIdx.x == 0) {
+        if (nj > 1) {
+            b.picks[q] = u.pick;
+            __threadfence();
+            u.last = atomicAdd(&b.ss->steps_done, 1u) == static_cast<unsigned int>(nj) - 1u;
+        } else {
+            u.picks[0] = u.pick;
+            u.last = 1;
+        }
+    }
+    __syncthreads();
+    if (!u.last) return;
+    if (nj > 1) {
+        __threadfence();
+        constexpr int kPickWords = static_cast<int>(sizeof(StepPick) / sizeof(unsigned long long));
+        for (int i = threadIdx.x; i < nj * kPickWords; i += blockDim.x)
+            reinterpret_cast<unsigned long long *>(u.picks)[i] = reinterpret_cast<const unsigned long long *>(b.picks)[i];
+    }
+    fetch();
+    __syncthreads();
+    commit_steps(b, u, nj);
+}
+
+constexpr int kArgWords = static_cast<int>(sizeof(SearchArgs) / sizeof(unsigned long long));
+static_assert(sizeof(SearchArgs) % sizeof(unsigned long long) == 0 && sizeof(StepPick) % sizeof(unsigned long long) == 0,
+              "copied in 8-byte words");
+
+struct StepSet {
+    DevBox b;
+    int nj, pad;
+    SearchArgs a[kMaxSteps];
+};
+
+// Steps of one box, blockIdx.y the step and blockIdx.x its block.
+__global__ __launch_bounds__(kBlock) void k_steps(StepSet) {
+    __shared__ StepsLds u;
+    const StepSet &set = kernel_arguments<StepSet>();
+    const int q = static_cast<int>(blockIdx.y);
+    const SearchArgs &a = set.a[q];
+    const unsigned vg = static_cast<unsigned>(a.vg);
+    if (blockIdx.x >= vg) return;
+    run_steps(set.b, u, a, q, set.nj, a.run_dirty, blockIdx.x, vg,
+              [&](int p) -> const SearchArgs & { return set.a[p]; },
+              [&] {
+                  for (int i = threadIdx.x; i < set.nj * kArgWords; i += blockDim.x)
+                      reinterpret_cast<unsigned long long *>(u.args)[i] =
+                          reinterpret_cast<const unsigned long long *>(set.a)[i];
+              });
+}
+
+// Steps of many boxes: blockIdx.y a box and blockIdx.x its step, one block each
+// (windows of few aggregates).  The runs are in pinned host memory; a block
+// reads its own step's arguments and of its predecessors what the moved set
+// takes (the first kMoveWords words), and leaves its own in device memory for
+// the block that carries the steps out.
+struct BoxRun {
+    const DevBox *box;  // device copy of the box's descriptor
+    int nj, pad;
+    SearchArgs a[kMaxSteps];
+};
+constexpr int kMoveWords = static_cast<int>(offsetof(SearchArgs, n_mov) / sizeof(unsigned long long));
+
+__global__ __launch_bounds__(kBlock) void k_steps_group(const BoxRun *runs) {
+    __shared__ StepsLds u;
+    __shared__ unsigned long long head[2];
+    const BoxRun *run = runs + blockIdx.y;
+    const int q = static_cast<int>(blockIdx.x);
+    for (int i = threadIdx.x; i < 2 + kArgWords + q * kMoveWords; i += blockDim.x) {
+        if (i < 2) {
+            head[i] = reinterpret_cast<const unsigned long long *>(run)[i];
+        } else if (i < 2 + kArgWords) {
+            const int w = i - 2;
+            reinterpret_cast<unsigned long long *>(&u.args[q])[w] =
+                reinterpret_cast<const unsigned long long *>(&run->a[q])[w];
+        } else {
+            const int p = (i - 2 - kArgWords) / kMoveWords, w = (i - 2 - kArgWords) - p * kMoveWords;
+            reinterpret_cast<unsigned long long *>(&u.args[p])[w] =
+                reinterpret_cast<const unsigned long long *>(&run->a[p])[w];
+        }
+    }
+    __syncthreads();
+    const int nj = __builtin_amdgcn_readfirstlane(static_cast<int>(head[1] & 0xffffffffull));
+    if (q >= nj) return;
+    const unsigned lo = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(head[0] & 0xffffffffull));
+    const unsigned hi = __builtin_amdgcn_readfirstlane(static_cast<unsigned>(head[0] >> 32));
+    using Const = const DevBox __attribute__((address_space(4)));
+    const DevBox &b = *(const DevBox *)(Const *)((static_cast<unsigned long long>(hi) << 32) | lo);
+    if (nj > 1)
+        for (int i = threadIdx.x; i < kArgWords; i += blockDim.x)
+            reinterpret_cast<unsigned long long *>(&b.sargs[q])[i] =
+                reinterpret_cast<const unsigned long long *>(&u.args[q])[i];
+    const SearchArgs &a = u.args[q];
+    run_steps(b, u, a, q, nj, a.run_dirty, 0u, 1u, [&](int p) -> const SearchArgs & { return u.args[p]; },
+              [&] {
+                  if (nj > 1)
+                      for (int i = threadIdx.x; i < nj * kArgWords; i += blockDim.x)
+                          reinterpret_cast<unsigned long long *>(u.args)[i] =
+                              reinterpret_cast<const unsigned long long *>(b.sargs)[i];
+              });
 }
 
 // Persistent form of k_step for one box: a resident grid takes the queued

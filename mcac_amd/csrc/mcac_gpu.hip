@@ -39,6 +39,7 @@ struct mcac_box {
     mcac_group *group = nullptr;
     int64_t group_call = -1;         // last group enqueue that took a move of this box
     DevBox d{};
+    DevBox *d_self = nullptr;        // device copy of d (group launches)
     int64_t n_spheres = 0, n_aggs = 0;
     int64_t cand_cap = 0, part_cap = 0, pool_cap = 0;
     int n_cells = 0, n_built = 0;
@@ -88,7 +89,7 @@ struct mcac_box {
     int64_t slot_epoch[kRing] = {0};
     int slot_void[kRing] = {0};      // known to be skipped: its predictions were taken out
     int slot_fused[kRing] = {0};
-    int slot_solving[kRing] = {0};   // its k_solve was launched before a cell-list rebuild
+    int slot_solving[kRing] = {0};   // its grid form was launched before a cell-list rebuild
     int max_count = 0;               // upper bound of the aggregate sizes
     int64_t n_handover = 0;          // k_step searches finished by k_solve
     int64_t n_fused = 0, n_split = 0;  // searches launched as k_step / k_filter + k_solve
@@ -128,20 +129,29 @@ struct mcac_box {
     bool mirrors_exact = true;   // the host mirrors of positions and rmax hold every aggregate exactly
 };
 
-// Boxes that share one stream; their queued steps go into k_step_batch
-// launches, one block per box.  Jobs and block segments are written to pinned
-// memory, in turn into kBuffers job lists, so that a list is written while the
-// launches that read the others are still queued.
+// Queued steps of one box written for a launch of several.
+struct StepRun {
+    mcac_box *box = nullptr;
+    int n = 0;
+    double items = 0;  // most window entries of a step
+    StepSet set;
+};
+
+// Boxes that share one stream; their queued steps go into launches of several
+// steps of several boxes (k_steps_group), or of one box where a step's window
+// takes several blocks (k_steps).  The boxes' runs are written to pinned memory,
+// in turn into kBuffers lists, so that a list is written while the launches that
+// read the others are still queued.
 struct mcac_group {
-    static constexpr int kMovesPerBox = 8;  // = kMaxBlockJobs, steps of a box in one launch
-    static constexpr int kBuffers = 3;      // job lists
+    static constexpr int kMovesPerBox = kMaxSteps;  // steps of a box in one launch
+    static constexpr int kBuffers = 3;      // run lists
     int device = 0;
     hipStream_t stream = nullptr;
     int cap = 0;                           // boxes
-    int job_cap = 0;                       // jobs per list
+    int job_cap = 0;                       // moves of one enqueue
     int parity = 0;                        // the list written next
-    StepJob *h_jobs = nullptr, *d_jobs = nullptr;  // kBuffers * job_cap jobs
-    int *h_seg = nullptr, *d_seg = nullptr;        // kBuffers * (job_cap + 1) segment starts
+    BoxRun *h_runs = nullptr, *d_runs = nullptr;   // kBuffers * cap runs
+    StepRun *run = nullptr;                // steps of the box being enqueued
     hipEvent_t read[kBuffers]{};                    // recorded after the launch reading each list
     bool pending[kBuffers] = {};
     int64_t calls = 0;
@@ -169,6 +179,13 @@ template <class T> int dalloc(mcac_box *b, T **ptr, int64_t n) {
     HIP_TRY(hipMemset(p, 0, bytes));
     b->allocs.push_back(p);
     *ptr = static_cast<T *>(p);
+    return 0;
+}
+
+// Brings the device copy of the box's descriptor up to date (at creation and
+// when a buffer has moved; nothing of the box may be running).
+int copy_descriptor(mcac_box *b) {
+    HIP_TRY(hipMemcpy(b->d_self, &b->d, sizeof(DevBox), hipMemcpyHostToDevice));
     return 0;
 }
 
@@ -426,6 +443,7 @@ int compact_pool(mcac_box *b, int64_t need) {
     b->d.members = nm;
     b->pool_cap = cap;
     b->pool_used = used;
+    if (int rc = copy_descriptor(b)) return rc;
     HIP_TRY(hipFree(d_ids));
     HIP_TRY(hipFree(d_ns));
     HIP_TRY(hipFree(d_os));
@@ -434,12 +452,37 @@ int compact_pool(mcac_box *b, int64_t need) {
 
 int harvest_timing(mcac_box *b, int slot);
 
-// A step handed over to k_solve finishes (moves its aggregate, drops its cell
-// entry and writes its dirty-list entry at the slot predicted for the current
-// cell list) only when its k_solve runs, which the host launches when it reads
+// Blocks of the grid form for a mover of n_mov spheres: the filter grid,
+// widened to the sphere tiles that four survivors as large as the largest
+// aggregate would bring, at most grid_blocks (a block of it holds 75 KB of LDS;
+// all of them are resident together for its barrier, whose arrivals are
+// atomics on one counter).
+int grid_form_blocks(const mcac_box *b, int filter_grid) {
+    const double tiles = std::ceil(4.0 * static_cast<double>(b->max_count) / 64);
+    return std::min(b->grid_blocks, std::max(filter_grid, static_cast<int>(std::min<double>(kFilterBlocks, tiles))));
+}
+
+// The grid form of a step that a block left to it: filter and solve again, the
+// box being as it was when the step ran.
+int launch_handed_over(mcac_box *b, const SearchArgs &a) {
+    if (b->grid_solve) {
+        hipLaunchKernelGGL(k_step_grid, dim3(static_cast<unsigned>(grid_form_blocks(b, b->grid_blocks))), dim3(kBlock),
+                           0, bstream(b), b->d, a);
+    } else {
+        hipLaunchKernelGGL(k_filter, dim3(kFilterBlocks), dim3(kBlock), 0, bstream(b), b->d, a);
+        hipLaunchKernelGGL(k_solve, dim3(kSolveBlocks), dim3(kBlock), 0, bstream(b), b->d, a);
+    }
+    HIP_TRY(hipGetLastError());
+    b->n_handover += 1;
+    return 0;
+}
+
+// A step handed over to the grid form finishes (moves its aggregate, drops its
+// cell entry and writes its dirty-list entry at the slot predicted for the
+// current cell list) only when that runs, which the host launches when it reads
 // the pending record.  A cell-list rebuild must not run in between: before a
-// rebuild with steps in flight, every queued kernel is drained and the
-// k_solve of a pending step (at most one: it closes the gate) is launched now.
+// rebuild with steps in flight, every queued kernel is drained and the grid
+// form of a pending step (at most one: it closes the gate) is launched now.
 int settle_handovers(mcac_box *b) {
     if (b->inflight == 0) return 0;
     HIP_TRY(hipStreamSynchronize(bstream(b)));
@@ -448,11 +491,9 @@ int settle_handovers(mcac_box *b) {
         if (b->slot_void[slot] || b->slot_solving[slot]) continue;
         StepRecord &r = b->h_step[slot];
         if (__atomic_load_n(&r.seq, __ATOMIC_ACQUIRE) != t || r.skipped || r.status != kPendingSolve) continue;
-        __atomic_store_n(&r.seq, 0ull, __ATOMIC_RELEASE);  // the k_solve publishes the final record
-        hipLaunchKernelGGL(k_solve, dim3(kSolveBlocks), dim3(kBlock), 0, bstream(b), b->d, b->slot_args[slot]);
-        HIP_TRY(hipGetLastError());
+        __atomic_store_n(&r.seq, 0ull, __ATOMIC_RELEASE);  // the grid form publishes the final record
+        if (int rc = launch_handed_over(b, b->slot_args[slot])) return rc;
         b->slot_solving[slot] = 1;
-        b->n_handover += 1;
     }
     return 0;
 }
@@ -494,13 +535,33 @@ bool next_step_timed(const mcac_box *b) {
     return b->timing > 0 && (b->seq + 1 - b->timing_base) % static_cast<unsigned long long>(b->timing) == 0;
 }
 
-// Picks the launch of one step and enqueues it.  With job_out (given only for
-// a step that one block can take whole: one-launch form, mover moved by the
-// finishing block, not timed, few window entries) the step is written there
-// instead, for a k_step_batch launch by the caller (*batched = true).
+// Position of the mover when its next queued step runs: the mirror's, or with
+// steps of it in flight the newest one's move without contact (a contact before
+// the step would have it skipped).  False when the host does not know it.
+bool mover_position(const mcac_box *b, size_t A, double com[3]) {
+    if (!b->mirrors_exact) return false;
+    if (b->pend[A] == 0) {
+        com[0] = b->h_x[A];
+        com[1] = b->h_y[A];
+        com[2] = b->h_z[A];
+        return true;
+    }
+    for (unsigned long long t = b->seq; t >= b->oldest; --t) {
+        const int slot = static_cast<int>(t % mcac_box::kRing);
+        const SearchArgs &e = b->slot_args[slot];
+        if (b->slot_void[slot] || !b->slot_apply[slot] || b->slot_agg[slot] != static_cast<int64_t>(A)) continue;
+        if (!e.nc_ok || !e.gated) return false;
+        for (int l = 0; l < 3; ++l) com[l] = e.nc_com[l];
+        return true;
+    }
+    return false;
+}
+
+// Picks the launch of one step and enqueues it.  With run (given only for a
+// step that takes the one-launch form, known to the host and not timed) the
+// step is added there instead, for a launch by the caller.
 int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, double maxradius, int apply, int gated,
-                   unsigned long long *ticket, StepJob *job_out = nullptr, bool *batched = nullptr) {
-    if (batched) *batched = false;
+                   unsigned long long *ticket, StepRun *run = nullptr) {
     if (agg < 0 || agg >= b->n_aggs || b->count[static_cast<size_t>(agg)] <= 0) return MCAC_E_ARGUMENT;
     if (b->inflight >= mcac_box::kRing) return MCAC_E_CAPACITY;
     if (b->inline_pending) return MCAC_E_ARGUMENT;  // the caller merges the contact first
@@ -511,7 +572,7 @@ int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, do
     }
     const size_t A = static_cast<size_t>(agg);
     const int n_mov = b->count[A];
-    const unsigned long long seq = ++b->seq;
+    const unsigned long long seq = b->seq + 1;
     const int slot = static_cast<int>(seq % mcac_box::kRing);
     SearchArgs a{};
     a.src = static_cast<int>(agg);
@@ -519,19 +580,21 @@ int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, do
     a.start = b->start[A];
     // a queued step behind a known closed gate does nothing: no predictions
     const bool doomed = gated && b->gate_closed;
-    if (b->pend[A] == 0 && b->mirrors_exact) {
+    double src[3];
+    const bool known = mover_position(b, A, src);
+    b->seq = seq;
+    if (known) {
         a.known = 1;
-        a.sx = b->h_x[A];
-        a.sy = b->h_y[A];
-        a.sz = b->h_z[A];
+        a.sx = src[0];
+        a.sy = src[1];
+        a.sz = src[2];
         a.srmax = b->h_rmax[A];
         a.srx = b->h_rx[A];
         a.sry = b->h_ry[A];
         a.srz = b->h_rz[A];
-        const double src[3] = {a.sx, a.sy, a.sz};
         const double vec[3] = {lpm * dir[0], lpm * dir[1], lpm * dir[2]};
         verlet_window(src, vec, a.srmax + maxradius, static_cast<int>(b->p.n_div), b->p.box_length, a.b1, a.len);
-        // the move without contact (finish_step: calcul.cpp:128-130, aggregat.cpp:148-153)
+        // the move without contact (apply_step: calcul.cpp:128-130, aggregat.cpp:148-153)
         for (int l = 0; l < 3; ++l) {
             a.nc_com[l] = periodic_position(src[l] + dir[l] * lpm, b->p.box_length);
             a.nc_ref[l] = a.nc_com[l] - (l == 0 ? a.srx : (l == 1 ? a.sry : a.srz));
@@ -590,27 +653,34 @@ int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, do
     // filter grid sized to the expected work: entries of the visited cells
     // (1.5x the mean cell occupancy) plus the dirty list, one per thread
     int grid = kFilterBlocks;
+    double items = 0;
     if (a.known && b->n_cells > 0) {
         const double per_cell = static_cast<double>(b->n_built) / b->n_cells;
-        const double items = 1.5 * per_cell * a.len[0] * a.len[1] * a.len[2] + a.dirty_n + 1;
+        items = 1.5 * per_cell * a.len[0] * a.len[1] * a.len[2] + a.dirty_n + 1;
         grid = static_cast<int>(std::min<double>(kFilterBlocks, std::ceil(items / kBlock)));
         grid = std::max(grid, 1);
     }
+    a.vg = grid;
+    a.run_dirty = a.dirty_n;
     // timed launches carry start/stop events that the runtime stamps with the
     // kernel's own execution interval; the queue is drained first so that the
     // interval does not include waiting behind the steps queued before it
     if (timed && b->inflight > 0) HIP_TRY(hipStreamSynchronize(bstream(b)));
     // the persistent engine takes one-launch steps whose mover the finishing
     // block moves (not timed: a timed step is its own launch between events)
-    const bool engine = !job_out && b->eng_blocks > 0 && !b->group && fused && !timed && gated &&
+    const bool engine = !run && b->eng_blocks > 0 && !b->group && fused && !timed && gated &&
                         (!apply || a.translate_in_finish);
-    if (job_out || engine) {
-        // queued step arguments sit in LDS: the host adds the bounds of the
-        // visited cells, saving the kernel a dependent load (a launch of its
-        // own reads them faster from cstart than from its arguments)
+    if (run) {
+        run->box = b;
+        if (run->n > 0) a.run_dirty = run->set.a[0].dirty_n;
+        run->items = run->n > 0 ? std::max(run->items, items) : items;
+        run->set.a[run->n++] = a;
+    } else if (engine) {
+        // the host adds the bounds of the visited cells, saving the resident
+        // grid a dependent load (a launch of its own reads them faster from
+        // cstart than from its arguments)
         const int V = a.len[0] * a.len[1] * a.len[2];
-        CellTable ct_local;
-        CellTable &ct = job_out ? job_out->cells : ct_local;
+        CellTable ct;
         ct.n = 0;
         if (a.known && b->cstart_ok && V <= 64) {
             const int n = static_cast<int>(b->p.n_div), lj = a.len[1], lk = a.len[2];
@@ -623,28 +693,16 @@ int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, do
             }
             ct.n = V;
         }
-        if (job_out) {
-            job_out->b = b->d;
-            job_out->a = a;
-            *batched = true;
-        } else {
-            // the resident grid has eng_blocks workgroups; the step takes the
-            // share its window needs, as a launch of its own would
-            int rc = engine_start(b, b->eng_blocks);
-            if (rc) return rc;
-            engine_post(b, &a, &ct, std::min(grid, b->eng_blocks));
-        }
+        // the resident grid has eng_blocks workgroups; the step takes the
+        // share its window needs, as a launch of its own would
+        int rc = engine_start(b, b->eng_blocks);
+        if (rc) return rc;
+        engine_post(b, &a, &ct, std::min(grid, b->eng_blocks));
     } else if (fused) {
-        if (timed) hipExtLaunchKernelGGL(k_step, dim3(grid), dim3(kBlock), 0, bstream(b), ev[0], ev[1], 0, b->d, a);
-        else hipLaunchKernelGGL(k_step, dim3(grid), dim3(kBlock), 0, bstream(b), b->d, a);
+        if (timed) hipExtLaunchKernelGGL(k_step, dim3(grid), dim3(kBlock), 0, bstream(b), ev[0], ev[1], 0, StepOne{b->d, a});
+        else hipLaunchKernelGGL(k_step, dim3(grid), dim3(kBlock), 0, bstream(b), StepOne{b->d, a});
     } else if (b->grid_solve) {
-        // one launch: the filter grid, widened to the sphere tiles that four
-        // survivors as large as the largest aggregate would bring, at most
-        // grid_blocks (a block of it holds 81 KB of LDS, one per CU, all of
-        // them resident together for its barrier, whose arrivals are atomics
-        // on one counter)
-        const double tiles = std::ceil(4.0 * static_cast<double>(b->max_count) / 64);
-        const int g2 = std::min(b->grid_blocks, std::max(grid, static_cast<int>(std::min<double>(kFilterBlocks, tiles))));
+        const int g2 = grid_form_blocks(b, grid);
         if (timed) hipExtLaunchKernelGGL(k_step_grid, dim3(g2), dim3(kBlock), 0, bstream(b), ev[0], ev[1], 0, b->d, a);
         else hipLaunchKernelGGL(k_step_grid, dim3(g2), dim3(kBlock), 0, bstream(b), b->d, a);
     } else if (timed) {
@@ -722,17 +780,15 @@ int wait_search(mcac_box *b, unsigned long long ticket, int64_t agg, mcac_contac
     }
     int rc = wait_seq(b, &b->h_step[slot].seq, ticket);
     if (rc) return rc;
-    bool handed_over = b->slot_solving[slot] != 0;  // its k_solve already ran (settle_handovers)
+    bool handed_over = b->slot_solving[slot] != 0;  // its grid form already ran (settle_handovers)
     b->slot_solving[slot] = 0;
     if (!handed_over && !b->h_step[slot].skipped && b->h_step[slot].status == kPendingSolve) {
         handed_over = true;
-        // k_step left its survivors to the multi-block solve; the gate it
+        // the step left its survivors to the grid form; the gate it
         // closed keeps the queued steps behind it from running meanwhile
         __atomic_store_n(&b->h_step[slot].seq, 0ull, __ATOMIC_RELEASE);
-        SearchArgs sa = b->slot_args[slot];
-        hipLaunchKernelGGL(k_solve, dim3(kSolveBlocks), dim3(kBlock), 0, bstream(b), b->d, sa);
-        HIP_TRY(hipGetLastError());
-        b->n_handover += 1;
+        rc = launch_handed_over(b, b->slot_args[slot]);
+        if (rc) return rc;
         rc = wait_seq(b, &b->h_step[slot].seq, ticket);
         if (rc) return rc;
     }
@@ -846,6 +902,7 @@ template <class F> int box_buffers(DevBox &d, const BoxSizes &z, int volsurf, F 
     }
     ALLOC(d.ss, 1); ALLOC(d.ms, 1);
     ALLOC(d.eng_jobs, kEngineRing); ALLOC(d.eng_closed, kEngineRing);
+    ALLOC(d.picks, kMaxSteps); ALLOC(d.sargs, kMaxSteps);
 #undef ALLOC
     return 0;
 }
@@ -999,6 +1056,8 @@ int mcac_box_create(const mcac_box_params *params, mcac_box **out) {
     b->part_cap = z.part_cap;
     b->pool_cap = z.pool_cap;
     rc = box_buffers(b->d, z, params->volsurf, [&](auto *&ptr, int64_t n) { return dalloc(b, &ptr, n); });
+    if (rc == 0) rc = dalloc(b, &b->d_self, 1);
+    if (rc == 0) rc = copy_descriptor(b);
     if (rc) return fail(rc);
     if (b->n_cells + 1 <= (1 << 20) &&
         hipHostMalloc(reinterpret_cast<void **>(&b->h_cstart), (static_cast<size_t>(b->n_cells) + 1) * sizeof(int),
@@ -1482,21 +1541,18 @@ int mcac_group_create(int device, int max_boxes, mcac_group **out) {
     g->device = device;
     g->cap = max_boxes;
     g->job_cap = max_boxes * mcac_group::kMovesPerBox;
-    const size_t bytes = mcac_group::kBuffers * static_cast<size_t>(g->job_cap) * sizeof(StepJob);
-    const size_t seg_bytes = mcac_group::kBuffers * (static_cast<size_t>(g->job_cap) + 1) * sizeof(int);
-    if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void **>(&g->h_jobs), bytes, hipHostMallocCoherent) != hipSuccess ||
-        hipHostGetDevicePointer(reinterpret_cast<void **>(&g->d_jobs), g->h_jobs, 0) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void **>(&g->h_seg), seg_bytes, hipHostMallocCoherent) != hipSuccess ||
-        hipHostGetDevicePointer(reinterpret_cast<void **>(&g->d_seg), g->h_seg, 0) != hipSuccess ||
+    const size_t bytes = mcac_group::kBuffers * static_cast<size_t>(g->cap) * sizeof(BoxRun);
+    g->run = new (std::nothrow) StepRun();
+    if (!g->run || hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess ||
+        hipHostMalloc(reinterpret_cast<void **>(&g->h_runs), bytes, hipHostMallocCoherent) != hipSuccess ||
+        hipHostGetDevicePointer(reinterpret_cast<void **>(&g->d_runs), g->h_runs, 0) != hipSuccess ||
         hipEventCreateWithFlags(&g->read[0], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&g->read[1], hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&g->read[2], hipEventDisableTiming) != hipSuccess) {
         mcac_group_destroy(g);
         return MCAC_E_DEVICE;
     }
-    std::memset(g->h_jobs, 0, bytes);
-    std::memset(g->h_seg, 0, seg_bytes);
+    std::memset(g->h_runs, 0, bytes);
     *out = g;
     return 0;
 }
@@ -1504,8 +1560,8 @@ int mcac_group_create(int device, int max_boxes, mcac_group **out) {
 int mcac_group_destroy(mcac_group *g) {
     if (!g) return 0;
     if (g->stream) (void)hipStreamSynchronize(g->stream);
-    if (g->h_jobs) (void)hipHostFree(g->h_jobs);
-    if (g->h_seg) (void)hipHostFree(g->h_seg);
+    if (g->h_runs) (void)hipHostFree(g->h_runs);
+    delete g->run;
     for (auto &e : g->read)
         if (e) (void)hipEventDestroy(e);
     if (g->stream) (void)hipStreamDestroy(g->stream);
@@ -1526,49 +1582,80 @@ int mcac_group_add(mcac_group *g, mcac_box *b) {
 
 namespace {
 
-// Job list being written: jobs[0..n), block segments seg[0..blocks]; opened
-// when its first job is written (open = false: none yet).
-struct JobList {
-    StepJob *jobs = nullptr;
-    int *seg = nullptr;
-    int n = 0, blocks = 0;
+// List of runs being written; opened when its first run is written.
+struct RunList {
+    BoxRun *runs = nullptr;
+    int n = 0, widest = 0;          // runs, and the steps of the longest
     bool open = false;
-    const mcac_box *last = nullptr;
+    const mcac_box *last = nullptr;  // box of the newest run
 };
 
-int group_open(mcac_group *g, JobList &l) {
-    const int q = g->parity;
-    if (g->pending[q]) {  // the launch that read this list has copied its jobs
-        const auto t0 = std::chrono::steady_clock::now();
-        HIP_TRY(hipEventSynchronize(g->read[q]));
-        g->t_list += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-        g->pending[q] = false;
-    }
-    l.jobs = g->h_jobs + static_cast<size_t>(q) * static_cast<size_t>(g->job_cap);
-    l.seg = g->h_seg + static_cast<size_t>(q) * (static_cast<size_t>(g->job_cap) + 1);
-    l.n = l.blocks = 0;
-    l.open = true;
-    l.last = nullptr;
-    return 0;
-}
-
-int group_flush(mcac_group *g, JobList &l) {
+int group_flush(mcac_group *g, RunList &l) {
     if (!l.open || l.n == 0) return 0;
     const int q = g->parity;
-    l.seg[l.blocks] = l.n;
     const auto t0 = std::chrono::steady_clock::now();
-    hipLaunchKernelGGL(k_step_batch, dim3(static_cast<unsigned>(l.blocks)), dim3(kBlock), 0, g->stream,
-                       g->d_jobs + static_cast<size_t>(q) * static_cast<size_t>(g->job_cap),
-                       g->d_seg + static_cast<size_t>(q) * (static_cast<size_t>(g->job_cap) + 1));
+    hipLaunchKernelGGL(k_steps_group, dim3(static_cast<unsigned>(l.widest), static_cast<unsigned>(l.n)), dim3(kBlock), 0,
+                       g->stream, g->d_runs + static_cast<size_t>(q) * static_cast<size_t>(g->cap));
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipEventRecord(g->read[q], g->stream));
     g->t_launch += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     g->pending[q] = true;
     g->parity = (q + 1) % mcac_group::kBuffers;
     g->launches += 1;
-    g->batched_steps += l.n;
     l.open = false;
     l.last = nullptr;
+    return 0;
+}
+
+// Launches the steps gathered in the group's run, or puts them on the list:
+// with several boxes in the call, runs whose windows one block per step can
+// sweep share a launch.
+int run_flush(mcac_group *g, RunList &l, bool several) {
+    StepRun &r = *g->run;
+    if (r.n == 0) return 0;
+    mcac_box *b = r.box;
+    const int n = r.n;
+    r.n = 0;
+    g->batched_steps += n;
+    if (!several || r.items > kBlockItems) {
+        if (l.last == b) {  // after the box's earlier steps
+            int rc = group_flush(g, l);
+            if (rc) return rc;
+        }
+        const auto t0 = std::chrono::steady_clock::now();
+        r.set.b = b->d;
+        r.set.nj = n;
+        int vg = 1;
+        for (int q = 0; q < n; ++q) vg = std::max(vg, r.set.a[q].vg);
+        hipLaunchKernelGGL(k_steps, dim3(static_cast<unsigned>(vg), static_cast<unsigned>(n)), dim3(kBlock), 0,
+                           g->stream, r.set);
+        HIP_TRY(hipGetLastError());
+        g->t_launch += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+        g->launches += 1;
+        return 0;
+    }
+    if (l.open && (l.last == b || l.n >= g->cap)) {
+        int rc = group_flush(g, l);
+        if (rc) return rc;
+    }
+    if (!l.open) {
+        const int q = g->parity;
+        if (g->pending[q]) {  // the launch that read this list has ended
+            const auto t0 = std::chrono::steady_clock::now();
+            HIP_TRY(hipEventSynchronize(g->read[q]));
+            g->t_list += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+            g->pending[q] = false;
+        }
+        l.runs = g->h_runs + static_cast<size_t>(q) * static_cast<size_t>(g->cap);
+        l.n = l.widest = 0;
+        l.open = true;
+    }
+    BoxRun &o = l.runs[l.n++];
+    o.box = b->d_self;
+    o.nj = n;
+    std::memcpy(o.a, r.set.a, static_cast<size_t>(n) * sizeof(SearchArgs));
+    l.widest = std::max(l.widest, n);
+    l.last = b;
     return 0;
 }
 
@@ -1588,54 +1675,47 @@ int mcac_move_enqueue_group(mcac_group *g, mcac_box *const *boxes, const int64_t
         if (b->group_call == call) return MCAC_E_ARGUMENT;
         b->group_call = call;
     }
-    JobList l;
+    RunList l;
+    StepRun &run = *g->run;
+    run.n = 0;
+    bool several = false;
+    for (int i = 1; i < n; ++i) several = several || boxes[i] != boxes[0];
     int rc = 0;
     for (int i = 0; i < n; ++i) {
         mcac_box *b = boxes[i];
         const int64_t agg = aggs[i];
         const bool valid = agg >= 0 && agg < b->n_aggs;
-        const double reach = valid ? b->h_rmax[static_cast<size_t>(agg)] + maxradius[i] + lpm[i] : 0.0;
-        const bool batch = valid && one_block_step(b, b->count[static_cast<size_t>(agg)], next_step_timed(b)) &&
-                           window_items(b, reach) <= kBlockItems;
-        // a step launched on its own, or the cell-list rebuild that the
-        // enqueue launches, runs after every job already listed; a block
-        // runs at most kMaxBlockJobs jobs (the batch runner gives a box at
-        // most that many moves per call, so this never splits them there)
+        if (run.n > 0 && (run.box != b || run.n == kMaxSteps) && (rc = run_flush(g, l, several)) != 0) break;
         if ((i == 0 || boxes[i - 1] != b) && b->inflight == 0 && !b->inline_pending &&
             (b->cells_stale || b->dirty_count + mcac_group::kMovesPerBox + 3 >= rebuild_threshold(b))) {
             // a rebuild that this call's moves would make due, run before the
             // box's first move: nothing of the box is in flight, so it needs no
-            // drain, and its kernels run ahead of the box's jobs on the stream
+            // drain, and its kernels run ahead of the box's steps on the stream
             const auto t_r = std::chrono::steady_clock::now();
             rc = rebuild_cells(b);
             g->t_rebuild += std::chrono::duration<double>(std::chrono::steady_clock::now() - t_r).count();
             if (rc) break;
         }
-        const bool full = batch && l.last == b && l.n - l.seg[l.blocks - 1] >= kMaxBlockJobs;
+        // a step launched on its own, or the cell-list rebuild that the
+        // enqueue launches, runs after the box's steps gathered or listed so far
+        double com[3];
+        const bool batch = valid && one_block_step(b, b->count[static_cast<size_t>(agg)], next_step_timed(b)) &&
+                           mover_position(b, static_cast<size_t>(agg), com);
         const bool rebuild = rebuild_due(b) || b->cells_stale;
-        if ((!batch || full || (rebuild && l.last == b)) && (rc = group_flush(g, l)) != 0) break;
-        if (batch && !l.open && (rc = group_open(g, l)) != 0) break;
+        if (!batch || rebuild) {
+            if ((rc = run_flush(g, l, several)) != 0) break;
+            if (l.last == b && (rc = group_flush(g, l)) != 0) break;
+        }
         unsigned long long t = 0;
-        bool batched = false;
         const auto t_s = std::chrono::steady_clock::now();
-        rc = enqueue_search(b, agg, dirs + 3 * i, lpm[i], maxradius[i], 1, 1, &t, batch ? l.jobs + l.n : nullptr,
-                            batch ? &batched : nullptr);
+        rc = enqueue_search(b, agg, dirs + 3 * i, lpm[i], maxradius[i], 1, 1, &t, batch ? &run : nullptr);
         if (rebuild) g->t_rebuild += std::chrono::duration<double>(std::chrono::steady_clock::now() - t_s).count();
         if (rc) break;
-        if (batched != batch) {
-            rc = MCAC_UNKNOWN_ERROR;  // the two decisions must agree
-            break;
-        }
         tickets[i] = t;
-        if (batched) {
-            if (l.last != b) l.seg[l.blocks++] = l.n;  // a new block: the box's first job of this launch
-            l.last = b;
-            l.n += 1;
-        } else {
-            g->single_steps += 1;
-            l.last = nullptr;
-        }
+        if (!batch) g->single_steps += 1;
     }
+    const int rrc = run_flush(g, l, several);
+    if (rc == 0) rc = rrc;
     // the steps enqueued before a failing one still run: their results are read as usual
     const int frc = group_flush(g, l);
     g->t_enqueue += std::chrono::duration<double>(std::chrono::steady_clock::now() - t_in).count();
