@@ -1051,13 +1051,13 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
     }
     __syncthreads();  // the block's partials are written
     if (threadIdx.x == 0) {
-        __threadfence();
+        release_to_device();
         unsigned int ticket = atomicAdd(&b.ss->done_solve, 1u);
         last = (ticket == static_cast<unsigned int>(P) - 1u);
     }
     __syncthreads();
     if (!last) return;
-    __threadfence();
+    acquire_from_device();
     if (planned) {
         // per-candidate reduction of the tiles' minima: a candidate in a few
         // tiles by one thread, one in many by the whole block
@@ -1121,12 +1121,12 @@ __global__ __launch_bounds__(kBlock) void k_step_grid(DevBox b, SearchArgs a) {
     __shared__ int s_ok;
     if (threadIdx.x == 0) {
         if (tot) atomicAdd(&b.ss->nquery, tot);
-        __threadfence();  // this block's candidates and counts before its arrival
+        release_to_device();  // this block's candidates and counts before its arrival
         atomicAdd(&b.ss->grid_bar, 1u);
         const unsigned long long t0 = wall_clock64();
         int ok = 0;
         while (wall_clock64() - t0 <= kGridWaitTicks) {
-            if (__hip_atomic_load(&b.ss->grid_bar, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) >= gridDim.x) {
+            if (__hip_atomic_load(&b.ss->grid_bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= gridDim.x) {
                 ok = 1;
                 break;
             }
@@ -1137,7 +1137,7 @@ __global__ __launch_bounds__(kBlock) void k_step_grid(DevBox b, SearchArgs a) {
     }
     __syncthreads();
     if (!s_ok) return;
-    __threadfence();  // every block's candidates are visible to this one
+    acquire_from_device();  // every block's candidates are visible to this one
     solve_phase(b, a, lds);
 }
 
@@ -1214,14 +1214,14 @@ __device__ __forceinline__ int search_step(const DevBox &b, const SearchArgs &a,
     if (vg > 1) {
         if (threadIdx.x == 0) {
             const unsigned long long mine = kTicketOne + cnt;
-            __threadfence();
+            if (cnt >= kAppendOne) release_to_device();  // most blocks have written nothing
             const unsigned long long old = atomicAdd(&b.ss->step_tick[q], mine);
             last = (old >> 56) == vg - 1u;
             s_total = old + mine;
         }
         __syncthreads();
         if (!last) return 1;
-        __threadfence();
+        if (static_cast<unsigned int>((s_total >> 32) & 0xffffffull) > 0u) acquire_from_device();
         if (threadIdx.x == 0) {  // for the next launch
             b.ss->step_tick[q] = 0ull;
             b.ss->step_nfilt[q] = 0u;
@@ -1552,7 +1552,7 @@ __device__ __forceinline__ void run_steps(const DevBox &b, StepsLds &u, const Se
     if (threadIdx.x == 0) {
         if (nj > 1) {
             b.picks[q] = u.pick;
-            __threadfence();
+            release_to_device();
             u.last = atomicAdd(&b.ss->steps_done, 1u) == static_cast<unsigned int>(nj) - 1u;
         } else {
             u.picks[0] = u.pick;
@@ -1562,7 +1562,7 @@ __device__ __forceinline__ void run_steps(const DevBox &b, StepsLds &u, const Se
     __syncthreads();
     if (!u.last) return;
     if (nj > 1) {
-        __threadfence();
+        acquire_from_device();
         constexpr int kPickWords = static_cast<int>(sizeof(StepPick) / sizeof(unsigned long long));
         for (int i = threadIdx.x; i < nj * kPickWords; i += blockDim.x)
             reinterpret_cast<unsigned long long *>(u.picks)[i] = reinterpret_cast<const unsigned long long *>(b.picks)[i];
