@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "../../../include/mcac_sim.h"
+#include "../box_runs.hpp"
 #include "physics.hpp"
 #include "pick_table.hpp"
 #include "sim_group.hpp"
@@ -116,13 +117,11 @@ struct Simulation {
     int precision = 0;  // box contact-search precision (mcac_box_params)
     mcac_box *box = nullptr;
     mcac_group *group = nullptr;  // lock-step form: the box works on the group's stream
-    mcac_group *own_group = nullptr;  // one-box group for rounds of steps in one launch
-    bool rounds = false;              // issue rounds through own_group when the steps fit one workgroup
+    bool rounds = true;               // several steps per launch (mcac_move_enqueue_run), else one launch each
     int engine_blocks = 0;            // persistent step engine grid (mcac_box_set_engine), 0: off
-    std::vector<int64_t> r_aggs;      // scratch of issue_round
+    std::vector<int64_t> r_aggs;      // scratch of issue_run
     std::vector<double> r_dirs, r_lpm, r_maxr;
     std::vector<uint64_t> r_tickets;
-    std::vector<mcac_box *> r_boxes;
     // spheres (index order) — host copy of the initial state only
     size_t N = 0;              // spheres in the box
     size_t n_ids = 0;          // stable ids handed out (per-id host arrays hold this many)
@@ -155,7 +154,6 @@ struct Simulation {
 
     ~Simulation() {
         if (box) mcac_box_destroy(box);
-        if (own_group) mcac_group_destroy(own_group);  // after the box that works on its stream
     }
 
     // Volume and surface a one-sphere aggregate carries (compute_volume_surface,
@@ -315,7 +313,7 @@ struct Simulation {
         if (rc) return rc;
         if (pm.with_surface_reactions)
             for (auto *v : {&g_vol, &g_surf, &g_rsum, &g_rg, &g_rmax}) v->assign(n_ids, 0.0);
-        if (!group && !own_group && engine_blocks > 0) rc = mcac_box_set_engine(box, engine_blocks);
+        if (!group && engine_blocks > 0) rc = mcac_box_set_engine(box, engine_blocks);
         return rc;
     }
 
@@ -481,10 +479,10 @@ struct Simulation {
         if (rc) return rc;
         if (group) {
             depth = group_depth;  // steps picked ahead per box over its group launches
-        } else if (rounds && out_dir.empty() && depth > 1) {
-            rc = mcac_group_create(device, 1, &own_group);
-            if (rc == 0) rc = mcac_group_add(own_group, box);
-            if (rc) return rc;
+        } else if (rounds && out_dir.empty() && depth > 1 && engine_blocks == 0 && !pm.with_surface_reactions) {
+            depth = 2 * kRunSteps;  // two launches
+        } else {
+            rounds = false;
         }
         std::vector<double> pos3(3 * N), rcm3(3 * N, 0.0);
         std::vector<int64_t> cnt(N, 1), mem(N);
@@ -731,68 +729,63 @@ struct Simulation {
         return 0;
     }
 
-    // Steps picked ahead in rounds: when the next move's cell window is small
-    // enough for one workgroup, up to kRoundDepth moves go into one group
-    // launch (a workgroup runs them in order; those behind a contact do
-    // nothing, as behind the gate); otherwise the 3-deep one-launch pipeline.
-    // A new round is picked once at most kRoundRefill steps remain in flight.
-    static constexpr size_t kRoundDepth = 8, kRoundRefill = 3;
+    // Several steps per launch (mcac_move_enqueue_run): those behind a contact
+    // do nothing, as behind the gate, so a launch takes as many as are likely
+    // to run: all whose predecessors in it are without a contact with a
+    // probability of at least kWorth, by the rate p_contact of the last steps
+    // (one at the rates of a dense box, eight below a fifth).  While the steps in
+    // flight are more likely than not to run without a contact a second launch
+    // queues behind them, so that the picks overlap the device's work.
+    static constexpr size_t kRunSteps = 8;
+    static constexpr double kWorth = 0.2, kRate = 1.0 / 32.0;
+    double p_contact = 0.0;
+
+    int issue_run(size_t most, int64_t consumed, int64_t max_steps) {
+        r_aggs.clear();
+        r_dirs.clear();
+        r_lpm.clear();
+        while (r_aggs.size() < most && !finished() && can_issue(consumed, max_steps)) {
+            flight.push_back(pick_move());
+            const Pending &P = flight.back();
+            r_aggs.push_back(P.num);
+            r_dirs.insert(r_dirs.end(), P.draw.dir.begin(), P.draw.dir.end());
+            r_lpm.push_back(P.full);
+        }
+        const size_t k = r_aggs.size();
+        if (k == 0) return 0;
+        r_tickets.assign(k, 0);
+        auto te0 = Clock::now();
+        int rc = mcac_move_enqueue_run(box, r_aggs.data(), r_dirs.data(), r_lpm.data(), maxradius, static_cast<int>(k),
+                                       r_tickets.data());
+        t_enqueue += ms_since(te0);
+        if (rc) return rc;
+        for (size_t q = 0; q < k; ++q) flight[flight.size() - k + q].ticket = r_tickets[q];
+        return 0;
+    }
 
     int issue_more(int64_t consumed, int64_t max_steps) {
         if (duplication_due() && !finished()) {
             int rc = duplicate();
             if (rc) return rc;
         }
-        if (!own_group) {
+        if (!rounds) {
             while (!finished() && can_issue(consumed, max_steps)) {
                 int rc = issue();
                 if (rc) return rc;
             }
             return 0;
         }
-        if (flight.size() > kRoundRefill || finished() || !can_issue(consumed, max_steps)) return 0;
-        Pending first = pick_move();
-        const size_t U = static_cast<size_t>(first.num);
-        if (mcac_box_block_steps(box, rmax[U] + maxradius + first.full) != 1) {
-            // one launch per step for this one and up to the pipeline depth
-            auto te0 = Clock::now();
-            int rc = mcac_move_enqueue(box, first.num, first.draw.dir.data(), first.full, maxradius, &first.ticket);
-            t_enqueue += ms_since(te0);
+        if (flight.empty()) {
+            size_t k = 1;
+            for (double run = 1.0 - p_contact; k < kRunSteps && run >= kWorth; run *= 1.0 - p_contact) ++k;
+            int rc = issue_run(k, consumed, max_steps);
             if (rc) return rc;
-            flight.push_back(first);
-            while (!finished() && can_issue(consumed, max_steps)) {
-                rc = issue();
-                if (rc) return rc;
-            }
-            return 0;
         }
-        const size_t saved = depth;
-        depth = kRoundDepth;
-        flight.push_back(first);
-        size_t k = 1;
-        while (!finished() && can_issue(consumed, max_steps)) {
-            flight.push_back(pick_move());
-            ++k;
+        if (!flight.empty() && flight.size() <= kRunSteps &&
+            std::pow(1.0 - p_contact, static_cast<double>(flight.size())) >= 0.5) {
+            const size_t spare = static_cast<size_t>(mcac_box_spare_moves(box));
+            if (spare > 0) return issue_run(std::min(kRunSteps, spare), consumed, max_steps);
         }
-        depth = saved;
-        r_boxes.assign(k, box);
-        r_aggs.resize(k);
-        r_dirs.resize(3 * k);
-        r_lpm.resize(k);
-        r_maxr.assign(k, maxradius);
-        r_tickets.assign(k, 0);
-        for (size_t q = 0; q < k; ++q) {
-            const Pending &P = flight[flight.size() - k + q];
-            r_aggs[q] = P.num;
-            for (int l = 0; l < 3; ++l) r_dirs[3 * q + static_cast<size_t>(l)] = P.draw.dir[static_cast<size_t>(l)];
-            r_lpm[q] = P.full;
-        }
-        auto te0 = Clock::now();
-        int rc = mcac_move_enqueue_group(own_group, r_boxes.data(), r_aggs.data(), r_dirs.data(), r_lpm.data(),
-                                         r_maxr.data(), static_cast<int>(k), r_tickets.data());
-        t_enqueue += ms_since(te0);
-        if (rc) return rc;
-        for (size_t q = 0; q < k; ++q) flight[flight.size() - k + q].ticket = r_tickets[q];
         return 0;
     }
 
@@ -1236,6 +1229,7 @@ struct Simulation {
         q_filtered += static_cast<double>(c.n_filtered);
         q_pairs += static_cast<double>(c.n_pairs);
         const bool contact_flag = c.contact != 0;
+        p_contact += kRate * ((contact_flag ? 1.0 : 0.0) - p_contact);
         const double move = c.move;
         // calcul.cpp:147-153
         deltatemps = deltatemps * (move / full + static_cast<double>(1 - 1));
@@ -1413,7 +1407,7 @@ struct Simulation {
         *done = n;
         // the resident engine grid ends with the call, so that the device is
         // idle for the caller (it is launched again by the next step)
-        if (!group && !own_group && engine_blocks > 0) return mcac_box_set_engine(box, engine_blocks);
+        if (!group && engine_blocks > 0) return mcac_box_set_engine(box, engine_blocks);
         return 0;
     }
 };
@@ -1494,8 +1488,9 @@ int mcac_sim_create(const char *ini_text, const char *output_dir, int device, mc
     if (const char *e = std::getenv("MCAC_PIPELINE_DEPTH")) {  // steps kept in flight, 1..6
         const long v = std::strtol(e, nullptr, 10);
         h->s.depth = static_cast<size_t>(v < 1 ? 1 : (v > 6 ? 6 : v));
+        h->s.rounds = false;  // that many launches of one step
     }
-    if (const char *e = std::getenv("MCAC_ROUNDS")) {  // 0: always one launch per step
+    if (const char *e = std::getenv("MCAC_ROUNDS")) {  // 0: one launch per step
         h->s.rounds = std::strtol(e, nullptr, 10) != 0;
     }
     if (const char *e = std::getenv("MCAC_ENGINE")) {  // 0: one launch per step; n: resident grid of n blocks

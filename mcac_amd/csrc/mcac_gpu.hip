@@ -20,11 +20,13 @@
 #include <cstdlib>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <vector>
 
 #include "../../include/mcac_gpu.h"
+#include "box_runs.hpp"
 #include "kernels_cells.hpp"
 #include "kernels_growth.hpp"
 #include "kernels_merge.hpp"
@@ -32,11 +34,28 @@
 
 using namespace mcac_dev;
 
+// Host mirror of one aggregate.
+struct alignas(64) Mirror {
+    double x, y, z, rx, ry, rz, rmax;
+    int pend;   // queued steps that move it
+    int dslot;  // dirty-list index, -1: not moved since the cell-list build
+};
+static_assert(sizeof(Mirror) == 64, "one cache line");
+
+// Queued steps of one box written for a launch of several.
+struct StepRun {
+    mcac_box *box = nullptr;
+    int n = 0;
+    double items = 0;  // most window entries of a step
+    StepSet set;
+};
+
 struct mcac_box {
     mcac_box_params p{};
     hipStream_t stream = nullptr;
     bool own_stream = true;          // false once the box works on a group's stream
     mcac_group *group = nullptr;
+    std::unique_ptr<StepRun> run;    // steps of mcac_move_enqueue_run being gathered
     int64_t group_call = -1;         // last group enqueue that took a move of this box
     DevBox d{};
     DevBox *d_self = nullptr;        // device copy of d (group launches)
@@ -59,10 +78,10 @@ struct mcac_box {
     // rmax are exact for every aggregate that no queued step moves (pend == 0);
     // the dirty flags and list length are those after every queued step that
     // will run (steps known to be skipped are taken out)
-    std::vector<double> h_x, h_y, h_z, h_rx, h_ry, h_rz, h_rmax;
-    std::vector<int> pend;
-    std::vector<unsigned char> h_dirty;
-    std::vector<int> h_dslot;        // dirty-list index of each dirty aggregate
+    // (one cache line per aggregate: a step's mover is a random one, and at
+    // 10^6 aggregates each line is a miss; ten arrays took 2.5 us a step)
+    std::vector<Mirror> mir;
+    std::vector<int> dirty_ids;      // aggregates of the dirty list, by index
     int64_t dirty_count = 0;         // device dirty-list length after the queued steps
     int64_t dirty_epoch = 0;         // cell-list builds so far
     bool gate_closed = false;        // a consumed queued step found a contact; not released yet
@@ -127,14 +146,6 @@ struct mcac_box {
     int64_t grow_cap = 0;
     bool cells_stale = false;    // positions changed everywhere: rebuild the cell list before the next step
     bool mirrors_exact = true;   // the host mirrors of positions and rmax hold every aggregate exactly
-};
-
-// Queued steps of one box written for a launch of several.
-struct StepRun {
-    mcac_box *box = nullptr;
-    int n = 0;
-    double items = 0;  // most window entries of a step
-    StepSet set;
 };
 
 // Boxes that share one stream; their queued steps go into launches of several
@@ -306,6 +317,15 @@ int engine_start(mcac_box *b, int grid) {
     return 0;
 }
 
+// Host side of an aggregate joining the dirty list; whether it was not on it.
+bool mark_moved(mcac_box *b, size_t id) {
+    if (b->mir[id].dslot >= 0) return false;
+    b->mir[id].dslot = static_cast<int>(b->dirty_count);
+    b->dirty_ids[static_cast<size_t>(b->dirty_count)] = static_cast<int>(id);
+    b->dirty_count += 1;
+    return true;
+}
+
 int rebuild_alive(mcac_box *b) {
     std::vector<int> ids;
     ids.reserve(b->alive_ids.size());
@@ -339,7 +359,7 @@ void count_cells_on_host(mcac_box *b) {
     for (int id : b->alive_ids) {
         const size_t a = static_cast<size_t>(id);
         if (b->count[a] <= 0) continue;
-        b->cell_fill[static_cast<size_t>(ref_cell(b->h_x[a], b->h_y[a], b->h_z[a], n, b->p.box_length))] += 1;
+        b->cell_fill[static_cast<size_t>(ref_cell(b->mir[a].x, b->mir[a].y, b->mir[a].z, n, b->p.box_length))] += 1;
     }
     int acc = 0;
     for (int c = 0; c < b->n_cells; ++c) {
@@ -351,7 +371,9 @@ void count_cells_on_host(mcac_box *b) {
 
 // CSR cell list from the live ids; clears the dirty list (host and device).
 int rebuild_cells(mcac_box *b) {
-    if (b->dead_in_list > 0) {
+    // dead ids in the list cost a build one skipped entry each; leaving them out
+    // costs the host a pass over all ids and their upload (3 ms at 10^6)
+    if (4 * b->dead_in_list > static_cast<int64_t>(b->alive_ids.size())) {
         int rc = rebuild_alive(b);
         if (rc) return rc;
     }
@@ -368,16 +390,17 @@ int rebuild_cells(mcac_box *b) {
         hipLaunchKernelGGL(k_cell_scatter, dim3(g), dim3(kBlock), 0, bstream(b), b->d, n_alive);
     }
     HIP_TRY(hipGetLastError());
+    for (int64_t k = 0; k < b->dirty_count; ++k)
+        b->mir[static_cast<size_t>(b->dirty_ids[static_cast<size_t>(k)])].dslot = -1;
     b->dirty_count = 0;
-    std::fill(b->h_dirty.begin(), b->h_dirty.end(), 0);
     b->dirty_epoch += 1;
-    b->n_built = n_alive;
+    b->n_built = n_alive - static_cast<int>(b->dead_in_list);
     b->n_rebuilds++;
     b->cells_stale = false;
     b->cstart_ok = false;
-    if (b->h_cstart) {
-        // the host passes the visited cells' bounds with each step: counted
-        // here when the mirrors allow, else read back from the build
+    if (b->h_cstart && (b->eng_blocks > 0 || b->verify_cells)) {
+        // the host passes the visited cells' bounds with each engine step:
+        // counted here when the mirrors allow, else read back from the build
         const bool on_host = b->mirrors_exact && b->inflight == 0;
         if (on_host) count_cells_on_host(b);
         if (!on_host || b->verify_cells) {
@@ -540,10 +563,10 @@ bool next_step_timed(const mcac_box *b) {
 // the step would have it skipped).  False when the host does not know it.
 bool mover_position(const mcac_box *b, size_t A, double com[3]) {
     if (!b->mirrors_exact) return false;
-    if (b->pend[A] == 0) {
-        com[0] = b->h_x[A];
-        com[1] = b->h_y[A];
-        com[2] = b->h_z[A];
+    if (b->mir[A].pend == 0) {
+        com[0] = b->mir[A].x;
+        com[1] = b->mir[A].y;
+        com[2] = b->mir[A].z;
         return true;
     }
     for (unsigned long long t = b->seq; t >= b->oldest; --t) {
@@ -588,10 +611,10 @@ int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, do
         a.sx = src[0];
         a.sy = src[1];
         a.sz = src[2];
-        a.srmax = b->h_rmax[A];
-        a.srx = b->h_rx[A];
-        a.sry = b->h_ry[A];
-        a.srz = b->h_rz[A];
+        a.srmax = b->mir[A].rmax;
+        a.srx = b->mir[A].rx;
+        a.sry = b->mir[A].ry;
+        a.srz = b->mir[A].rz;
         const double vec[3] = {lpm * dir[0], lpm * dir[1], lpm * dir[2]};
         verlet_window(src, vec, a.srmax + maxradius, static_cast<int>(b->p.n_div), b->p.box_length, a.b1, a.len);
         // the move without contact (apply_step: calcul.cpp:128-130, aggregat.cpp:148-153)
@@ -607,15 +630,12 @@ int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, do
     a.dirty_pos = 0;
     int dirty_new = 0;
     if (apply && !doomed) {
-        if (!b->h_dirty[A]) {
-            a.dirty_slot = static_cast<int>(b->dirty_count);
-            b->h_dirty[A] = 1;
-            b->h_dslot[A] = a.dirty_slot;
-            b->dirty_count += 1;
+        if (mark_moved(b, A)) {
+            a.dirty_slot = b->mir[A].dslot;
             dirty_new = 1;
         }
-        a.dirty_pos = b->h_dslot[A];
-        b->pend[A] += 1;
+        a.dirty_pos = b->mir[A].dslot;
+        b->mir[A].pend += 1;
     }
     a.n_div = static_cast<int>(b->p.n_div);
     a.cap = static_cast<int>(b->cand_cap);
@@ -739,9 +759,9 @@ void take_out(mcac_box *b, int slot) {
     b->slot_void[slot] = 1;
     if (!b->slot_apply[slot]) return;
     const size_t A = static_cast<size_t>(b->slot_agg[slot]);
-    b->pend[A] -= 1;
+    b->mir[A].pend -= 1;
     if (b->slot_dirty_new[slot] && b->slot_epoch[slot] == b->dirty_epoch) {
-        b->h_dirty[A] = 0;
+        b->mir[A].dslot = -1;
         b->dirty_count -= 1;
     }
 }
@@ -818,10 +838,10 @@ int wait_search(mcac_box *b, unsigned long long ticket, int64_t agg, mcac_contac
         // the mover's new CoM, as the finishing block computed it (aggregat.cpp:148-161)
         const size_t A = static_cast<size_t>(agg);
         const SearchArgs &sa = b->slot_args[slot];
-        b->h_x[A] = periodic_position(b->h_x[A] + sa.dir[0] * s.move, b->p.box_length);
-        b->h_y[A] = periodic_position(b->h_y[A] + sa.dir[1] * s.move, b->p.box_length);
-        b->h_z[A] = periodic_position(b->h_z[A] + sa.dir[2] * s.move, b->p.box_length);
-        b->pend[A] -= 1;
+        b->mir[A].x = periodic_position(b->mir[A].x + sa.dir[0] * s.move, b->p.box_length);
+        b->mir[A].y = periodic_position(b->mir[A].y + sa.dir[1] * s.move, b->p.box_length);
+        b->mir[A].z = periodic_position(b->mir[A].z + sa.dir[2] * s.move, b->p.box_length);
+        b->mir[A].pend -= 1;
     }
     if (!s.skipped && b->slot_args[slot].gated && (s.contact || handed_over)) {
         // the steps queued behind this one will be skipped
@@ -1221,16 +1241,9 @@ int mcac_box_upload(mcac_box *b, int64_t ns, const double *x, const double *y, c
     b->pool_used = static_cast<int64_t>(pool.size());
     b->inflight = 0;
     b->oldest = b->seq + 1;
-    b->h_x = hx;
-    b->h_y = hy;
-    b->h_z = hz;
-    b->h_rx = hrx;
-    b->h_ry = hry;
-    b->h_rz = hrz;
-    b->h_rmax.assign(rmax, rmax + A);
-    b->pend.assign(A, 0);
-    b->h_dirty.assign(A, 0);
-    b->h_dslot.assign(A, 0);
+    b->mir.resize(A);
+    for (size_t a = 0; a < A; ++a) b->mir[a] = {hx[a], hy[a], hz[a], hrx[a], hry[a], hrz[a], rmax[a], 0, -1};
+    b->dirty_ids.resize(A + 1);
     b->dirty_count = 0;
     b->gate_closed = false;
     b->released = b->seq;
@@ -1264,14 +1277,10 @@ int mcac_translate(mcac_box *b, int64_t agg, const double vec[3]) {
                        static_cast<int>(b->p.n_div), b->p.box_length);
     {
         const size_t A = static_cast<size_t>(agg);
-        b->h_x[A] = periodic_position(b->h_x[A] + vec[0], b->p.box_length);
-        b->h_y[A] = periodic_position(b->h_y[A] + vec[1], b->p.box_length);
-        b->h_z[A] = periodic_position(b->h_z[A] + vec[2], b->p.box_length);
-        if (!b->h_dirty[A]) {
-            b->h_dirty[A] = 1;
-            b->h_dslot[A] = static_cast<int>(b->dirty_count);
-            b->dirty_count += 1;
-        }
+        b->mir[A].x = periodic_position(b->mir[A].x + vec[0], b->p.box_length);
+        b->mir[A].y = periodic_position(b->mir[A].y + vec[1], b->p.box_length);
+        b->mir[A].z = periodic_position(b->mir[A].z + vec[2], b->p.box_length);
+        mark_moved(b, A);
     }
     const int n = b->count[static_cast<size_t>(agg)];
     const int tb = std::min(1024, std::max(1, (n + kBlock - 1) / kBlock));
@@ -1302,19 +1311,14 @@ static int merge_done(mcac_box *b, size_t K, size_t R, int new_start, int new_ca
     // store_merged marks both aggregates as moved since the cell-list build
     // (unless a build ran after the merge on the device)
     if (dirty_now)
-        for (size_t id : {K, R})
-            if (!b->h_dirty[id]) {
-                b->h_dirty[id] = 1;
-                b->h_dslot[id] = static_cast<int>(b->dirty_count);
-                b->dirty_count += 1;
-            }
-    b->h_x[K] = out->com[0];
-    b->h_y[K] = out->com[1];
-    b->h_z[K] = out->com[2];
-    b->h_rx[K] = out->rcm[0];
-    b->h_ry[K] = out->rcm[1];
-    b->h_rz[K] = out->rcm[2];
-    b->h_rmax[K] = out->rmax;
+        for (size_t id : {K, R}) mark_moved(b, id);
+    b->mir[K].x = out->com[0];
+    b->mir[K].y = out->com[1];
+    b->mir[K].z = out->com[2];
+    b->mir[K].rx = out->rcm[0];
+    b->mir[K].ry = out->rcm[1];
+    b->mir[K].rz = out->rcm[2];
+    b->mir[K].rmax = out->rmax;
     return out->status;
 }
 
@@ -1590,7 +1594,18 @@ struct RunList {
     const mcac_box *last = nullptr;  // box of the newest run
 };
 
-int group_flush(mcac_group *g, RunList &l) {
+// An enqueue call: the steps of the box being enqueued, and with a group the
+// list that runs of several boxes go to.
+struct Enqueue {
+    mcac_group *g = nullptr;
+    StepRun *run = nullptr;
+    RunList l;
+    bool several = false;  // boxes in the call
+};
+
+int group_flush(Enqueue &e) {
+    RunList &l = e.l;
+    mcac_group *g = e.g;
     if (!l.open || l.n == 0) return 0;
     const int q = g->parity;
     const auto t0 = std::chrono::steady_clock::now();
@@ -1607,35 +1622,43 @@ int group_flush(mcac_group *g, RunList &l) {
     return 0;
 }
 
-// Launches the steps gathered in the group's run, or puts them on the list:
-// with several boxes in the call, runs whose windows one block per step can
-// sweep share a launch.
-int run_flush(mcac_group *g, RunList &l, bool several) {
-    StepRun &r = *g->run;
+// Launches the steps gathered, or puts them on the list: with several boxes in
+// the call, runs whose windows one block per step can sweep share a launch.
+int run_flush(Enqueue &e) {
+    StepRun &r = *e.run;
     if (r.n == 0) return 0;
+    RunList &l = e.l;
+    mcac_group *g = e.g;
     mcac_box *b = r.box;
     const int n = r.n;
     r.n = 0;
-    g->batched_steps += n;
-    if (!several || r.items > kBlockItems) {
+    if (g) g->batched_steps += n;
+    if (!e.several || r.items > kBlockItems) {
         if (l.last == b) {  // after the box's earlier steps
-            int rc = group_flush(g, l);
+            int rc = group_flush(e);
             if (rc) return rc;
         }
         const auto t0 = std::chrono::steady_clock::now();
-        r.set.b = b->d;
-        r.set.nj = n;
         int vg = 1;
         for (int q = 0; q < n; ++q) vg = std::max(vg, r.set.a[q].vg);
-        hipLaunchKernelGGL(k_steps, dim3(static_cast<unsigned>(vg), static_cast<unsigned>(n)), dim3(kBlock), 0,
-                           g->stream, r.set);
+        if (n == 1) {
+            hipLaunchKernelGGL(k_step, dim3(static_cast<unsigned>(vg)), dim3(kBlock), 0, bstream(b),
+                               StepOne{b->d, r.set.a[0]});
+        } else {
+            r.set.b = b->d;
+            r.set.nj = n;
+            hipLaunchKernelGGL(k_steps, dim3(static_cast<unsigned>(vg), static_cast<unsigned>(n)), dim3(kBlock), 0,
+                               bstream(b), r.set);
+        }
         HIP_TRY(hipGetLastError());
-        g->t_launch += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
-        g->launches += 1;
+        if (g) {
+            g->t_launch += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+            g->launches += 1;
+        }
         return 0;
     }
     if (l.open && (l.last == b || l.n >= g->cap)) {
-        int rc = group_flush(g, l);
+        int rc = group_flush(e);
         if (rc) return rc;
     }
     if (!l.open) {
@@ -1659,6 +1682,47 @@ int run_flush(mcac_group *g, RunList &l, bool several) {
     return 0;
 }
 
+// Adds one move of box b; first: the call's first move of it.
+int enqueue_move(Enqueue &e, mcac_box *b, bool first, int64_t agg, const double *dir, double lpm, double maxradius,
+                 uint64_t *ticket) {
+    StepRun &run = *e.run;
+    int rc = 0;
+    const bool valid = agg >= 0 && agg < b->n_aggs;
+    if (run.n > 0 && (run.box != b || run.n == kMaxSteps) && (rc = run_flush(e)) != 0) return rc;
+    auto timed = [&](auto &&work) {
+        const auto t0 = std::chrono::steady_clock::now();
+        const int r = work();
+        if (e.g) e.g->t_rebuild += std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
+        return r;
+    };
+    if (first && b->inflight == 0 && !b->inline_pending &&
+        (b->cells_stale || b->dirty_count + kMaxSteps + 3 >= rebuild_threshold(b))) {
+        // a rebuild that this call's moves would make due, run before the
+        // box's first move: nothing of the box is in flight, so it needs no
+        // drain, and its kernels run ahead of the box's steps on the stream
+        rc = timed([&] { return rebuild_cells(b); });
+        if (rc) return rc;
+    }
+    // a step launched on its own, or the cell-list rebuild that the enqueue
+    // launches, runs after the box's steps gathered or listed so far
+    double com[3];
+    const bool batch = valid && b->eng_blocks == 0 &&
+                       one_block_step(b, b->count[static_cast<size_t>(agg)], next_step_timed(b)) &&
+                       mover_position(b, static_cast<size_t>(agg), com);
+    const bool rebuild = rebuild_due(b) || b->cells_stale;
+    if (!batch || rebuild) {
+        if ((rc = run_flush(e)) != 0) return rc;
+        if (e.l.last == b && (rc = group_flush(e)) != 0) return rc;
+    }
+    unsigned long long t = 0;
+    auto work = [&] { return enqueue_search(b, agg, dir, lpm, maxradius, 1, 1, &t, batch ? &run : nullptr); };
+    rc = rebuild ? timed(work) : work();
+    if (rc) return rc;
+    *ticket = t;
+    if (!batch && e.g) e.g->single_steps += 1;
+    return 0;
+}
+
 }  // namespace
 
 int mcac_move_enqueue_group(mcac_group *g, mcac_box *const *boxes, const int64_t *aggs, const double *dirs,
@@ -1675,51 +1739,34 @@ int mcac_move_enqueue_group(mcac_group *g, mcac_box *const *boxes, const int64_t
         if (b->group_call == call) return MCAC_E_ARGUMENT;
         b->group_call = call;
     }
-    RunList l;
-    StepRun &run = *g->run;
-    run.n = 0;
-    bool several = false;
-    for (int i = 1; i < n; ++i) several = several || boxes[i] != boxes[0];
+    Enqueue e;
+    e.g = g;
+    e.run = g->run;
+    e.run->n = 0;
+    for (int i = 1; i < n; ++i) e.several = e.several || boxes[i] != boxes[0];
     int rc = 0;
-    for (int i = 0; i < n; ++i) {
-        mcac_box *b = boxes[i];
-        const int64_t agg = aggs[i];
-        const bool valid = agg >= 0 && agg < b->n_aggs;
-        if (run.n > 0 && (run.box != b || run.n == kMaxSteps) && (rc = run_flush(g, l, several)) != 0) break;
-        if ((i == 0 || boxes[i - 1] != b) && b->inflight == 0 && !b->inline_pending &&
-            (b->cells_stale || b->dirty_count + mcac_group::kMovesPerBox + 3 >= rebuild_threshold(b))) {
-            // a rebuild that this call's moves would make due, run before the
-            // box's first move: nothing of the box is in flight, so it needs no
-            // drain, and its kernels run ahead of the box's steps on the stream
-            const auto t_r = std::chrono::steady_clock::now();
-            rc = rebuild_cells(b);
-            g->t_rebuild += std::chrono::duration<double>(std::chrono::steady_clock::now() - t_r).count();
-            if (rc) break;
-        }
-        // a step launched on its own, or the cell-list rebuild that the
-        // enqueue launches, runs after the box's steps gathered or listed so far
-        double com[3];
-        const bool batch = valid && one_block_step(b, b->count[static_cast<size_t>(agg)], next_step_timed(b)) &&
-                           mover_position(b, static_cast<size_t>(agg), com);
-        const bool rebuild = rebuild_due(b) || b->cells_stale;
-        if (!batch || rebuild) {
-            if ((rc = run_flush(g, l, several)) != 0) break;
-            if (l.last == b && (rc = group_flush(g, l)) != 0) break;
-        }
-        unsigned long long t = 0;
-        const auto t_s = std::chrono::steady_clock::now();
-        rc = enqueue_search(b, agg, dirs + 3 * i, lpm[i], maxradius[i], 1, 1, &t, batch ? &run : nullptr);
-        if (rebuild) g->t_rebuild += std::chrono::duration<double>(std::chrono::steady_clock::now() - t_s).count();
-        if (rc) break;
-        tickets[i] = t;
-        if (!batch) g->single_steps += 1;
-    }
-    const int rrc = run_flush(g, l, several);
-    if (rc == 0) rc = rrc;
+    for (int i = 0; i < n && rc == 0; ++i)
+        rc = enqueue_move(e, boxes[i], i == 0 || boxes[i - 1] != boxes[i], aggs[i], dirs + 3 * i, lpm[i], maxradius[i],
+                          tickets + i);
     // the steps enqueued before a failing one still run: their results are read as usual
-    const int frc = group_flush(g, l);
+    const int rrc = run_flush(e), frc = group_flush(e);
     g->t_enqueue += std::chrono::duration<double>(std::chrono::steady_clock::now() - t_in).count();
-    return rc ? rc : frc;
+    return rc ? rc : (rrc ? rrc : frc);
+}
+
+int mcac_move_enqueue_run(mcac_box *b, const int64_t *aggs, const double *dirs, const double *lpm, double maxradius,
+                          int n, uint64_t *tickets) {
+    if (!b || n < 0 || (n > 0 && (!aggs || !dirs || !lpm || !tickets))) return MCAC_E_ARGUMENT;
+    if (!b->run) b->run.reset(new (std::nothrow) StepRun());
+    if (!b->run) return MCAC_E_CAPACITY;
+    Enqueue e;
+    e.run = b->run.get();
+    e.run->n = 0;
+    int rc = 0;
+    for (int i = 0; i < n && rc == 0; ++i)
+        rc = enqueue_move(e, b, i == 0, aggs[i], dirs + 3 * i, lpm[i], maxradius, tickets + i);
+    const int rrc = run_flush(e);
+    return rc ? rc : rrc;
 }
 
 int mcac_box_spare_moves(mcac_box *b) {
