@@ -23,6 +23,7 @@
 #include <memory>
 #include <mutex>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 #include "../../include/mcac_gpu.h"
@@ -120,7 +121,12 @@ struct mcac_box {
     size_t h_alpha_cap = 0;
     unsigned long long seq = 0;        // step tickets (searches)
     unsigned long long merge_seq = 0;  // merge records
-    std::vector<void *> allocs;
+    // every buffer of the box in one allocation: one call to make and one to
+    // free instead of some 75, and the box's pages lie together (a step touches
+    // forty buffers, each a translation of its own when they are scattered)
+    char *arena = nullptr;
+    int *moved_members = nullptr;    // the member pool once a compaction has replaced it
+    char *h_records = nullptr;       // pinned block of the records and the live-id staging
     int timing = 0;                  // 0 off; n >= 1: every n-th search is timed
     unsigned long long timing_base = 1;  // first ticket after timing was set: timed
     int slot_timed[kRing] = {0};     // 1 timed, 2 timed and consumed, events not read yet
@@ -182,16 +188,6 @@ namespace {
             return MCAC_E_DEVICE;                                                             \
         }                                                                                     \
     } while (0)
-
-template <class T> int dalloc(mcac_box *b, T **ptr, int64_t n) {
-    void *p = nullptr;
-    size_t bytes = static_cast<size_t>(n < 1 ? 1 : n) * sizeof(T);
-    HIP_TRY(hipMalloc(&p, bytes));
-    HIP_TRY(hipMemset(p, 0, bytes));
-    b->allocs.push_back(p);
-    *ptr = static_cast<T *>(p);
-    return 0;
-}
 
 // Brings the device copy of the box's descriptor up to date (at creation and
 // when a buffer has moved; nothing of the box may be running).
@@ -273,6 +269,10 @@ void engine_stop(mcac_box *b) {
 // to end first.
 hipStream_t bstream(mcac_box *b) {
     engine_stop(b);
+    // a box that joins a group before its first work never makes one
+    if (!b->stream && (hipSetDevice(b->p.device) != hipSuccess ||
+                       hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess))
+        b->stream = nullptr;
     return b->stream;
 }
 
@@ -398,7 +398,11 @@ int rebuild_cells(mcac_box *b) {
     b->n_rebuilds++;
     b->cells_stale = false;
     b->cstart_ok = false;
-    if (b->h_cstart && (b->eng_blocks > 0 || b->verify_cells)) {
+    const bool tables = (b->eng_blocks > 0 || b->verify_cells) && b->n_cells + 1 <= (1 << 20);
+    if (tables && !b->h_cstart)
+        HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&b->h_cstart), (static_cast<size_t>(b->n_cells) + 1) * sizeof(int),
+                              hipHostMallocDefault));
+    if (tables) {
         // the host passes the visited cells' bounds with each engine step:
         // counted here when the mirrors allow, else read back from the build
         const bool on_host = b->mirrors_exact && b->inflight == 0;
@@ -460,9 +464,8 @@ int compact_pool(mcac_box *b, int64_t need) {
     }
     HIP_TRY(hipMemcpy(b->d.astart, b->start.data(), b->start.size() * sizeof(int), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(b->d.acap, b->cap.data(), b->cap.size() * sizeof(int), hipMemcpyHostToDevice));
-    for (auto &p : b->allocs)
-        if (p == b->d.members) p = nm;
-    HIP_TRY(hipFree(b->d.members));
+    if (b->moved_members) HIP_TRY(hipFree(b->moved_members));
+    b->moved_members = nm;
     b->d.members = nm;
     b->pool_cap = cap;
     b->pool_used = used;
@@ -882,7 +885,7 @@ BoxSizes box_sizes(const mcac_box_params &p) {
     z.Na = p.max_aggregates;
     z.n_cells = p.n_div * p.n_div * p.n_div;
     z.cand_cap = p.candidate_capacity > 0 ? p.candidate_capacity : std::max<int64_t>(4096, std::min<int64_t>(z.Na, 1 << 20));
-    z.part_cap = std::max<int64_t>(z.cand_cap + 1024, 1 << 20);
+    z.part_cap = z.cand_cap + z.Ns / 64 + 1024;  // a minimum per candidate and tile of 64 spheres it lies in
     z.pool_cap = p.member_pool > 0 ? p.member_pool : 4 * z.Ns + 4096;
     return z;
 }
@@ -1069,43 +1072,45 @@ int mcac_box_create(const mcac_box_params *params, mcac_box **out) {
         return code;
     };
     if (hipSetDevice(params->device) != hipSuccess) return fail(MCAC_E_DEVICE);
-    if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) return fail(MCAC_E_DEVICE);
     const BoxSizes z = box_sizes(*params);
     b->n_cells = static_cast<int>(z.n_cells);
     b->cand_cap = z.cand_cap;
     b->part_cap = z.part_cap;
     b->pool_cap = z.pool_cap;
-    rc = box_buffers(b->d, z, params->volsurf, [&](auto *&ptr, int64_t n) { return dalloc(b, &ptr, n); });
-    if (rc == 0) rc = dalloc(b, &b->d_self, 1);
-    if (rc == 0) rc = copy_descriptor(b);
+    constexpr size_t kAlign = 256;
+    size_t bytes = 0;
+    auto room = [&](auto *&ptr, int64_t n) {
+        ptr = reinterpret_cast<std::remove_reference_t<decltype(ptr)>>(b->arena + bytes);
+        bytes += (static_cast<size_t>(n < 1 ? 1 : n) * sizeof(*ptr) + kAlign - 1) / kAlign * kAlign;
+        return 0;
+    };
+    auto lay_out = [&] {
+        bytes = 0;
+        box_buffers(b->d, z, params->volsurf, room);
+        room(b->d_self, 1);
+    };
+    lay_out();  // the size, then the addresses
+    if (hipMalloc(reinterpret_cast<void **>(&b->arena), bytes) != hipSuccess) return fail(MCAC_E_DEVICE);
+    lay_out();
+    if (hipMemset(b->arena, 0, bytes) != hipSuccess) return fail(MCAC_E_DEVICE);
+    rc = copy_descriptor(b);  // its wait covers the clearing before it
     if (rc) return fail(rc);
-    if (b->n_cells + 1 <= (1 << 20) &&
-        hipHostMalloc(reinterpret_cast<void **>(&b->h_cstart), (static_cast<size_t>(b->n_cells) + 1) * sizeof(int),
-                      hipHostMallocDefault) != hipSuccess)
-        return fail(MCAC_E_DEVICE);
     b->alive_cap = z.Na;
-    if (hipHostMalloc(reinterpret_cast<void **>(&b->h_alive), static_cast<size_t>(z.Na) * sizeof(int),
-                      hipHostMallocDefault) != hipSuccess ||
+    constexpr size_t kStepBytes = mcac_box::kRing * sizeof(StepRecord);
+    const size_t rec = (kStepBytes + sizeof(MergeRecord) + kAlign - 1) / kAlign * kAlign;
+    if (hipHostMalloc(reinterpret_cast<void **>(&b->h_records), rec + static_cast<size_t>(z.Na) * sizeof(int),
+                      hipHostMallocCoherent) != hipSuccess ||
         hipEventCreateWithFlags(&b->alive_read, hipEventDisableTiming) != hipSuccess)
         return fail(MCAC_E_DEVICE);
-    if (hipHostMalloc(reinterpret_cast<void **>(&b->h_step), mcac_box::kRing * sizeof(StepRecord),
-                      hipHostMallocCoherent) != hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void **>(&b->h_merge), sizeof(MergeRecord), hipHostMallocCoherent) != hipSuccess)
+    std::memset(b->h_records, 0, rec);
+    char *dev = nullptr;
+    if (hipHostGetDevicePointer(reinterpret_cast<void **>(&dev), b->h_records, 0) != hipSuccess)
         return fail(MCAC_E_DEVICE);
-    std::memset(b->h_step, 0, mcac_box::kRing * sizeof(StepRecord));
-    std::memset(b->h_merge, 0, sizeof(MergeRecord));
-    if (hipHostGetDevicePointer(reinterpret_cast<void **>(&b->d_step), b->h_step, 0) != hipSuccess ||
-        hipHostGetDevicePointer(reinterpret_cast<void **>(&b->d_merge), b->h_merge, 0) != hipSuccess)
-        return fail(MCAC_E_DEVICE);
-    if (hipHostMalloc(reinterpret_cast<void **>(&b->h_ring), kEngineRing * sizeof(EngineJob), hipHostMallocCoherent) !=
-            hipSuccess ||
-        hipHostMalloc(reinterpret_cast<void **>(&b->h_ctl), sizeof(EngineCtl), hipHostMallocCoherent) != hipSuccess)
-        return fail(MCAC_E_DEVICE);
-    std::memset(b->h_ring, 0, kEngineRing * sizeof(EngineJob));
-    std::memset(b->h_ctl, 0, sizeof(EngineCtl));
-    if (hipHostGetDevicePointer(reinterpret_cast<void **>(&b->dp_ring), b->h_ring, 0) != hipSuccess ||
-        hipHostGetDevicePointer(reinterpret_cast<void **>(&b->dp_ctl), b->h_ctl, 0) != hipSuccess)
-        return fail(MCAC_E_DEVICE);
+    b->h_step = reinterpret_cast<StepRecord *>(b->h_records);
+    b->d_step = reinterpret_cast<StepRecord *>(dev);
+    b->h_merge = reinterpret_cast<MergeRecord *>(b->h_records + kStepBytes);
+    b->d_merge = reinterpret_cast<MergeRecord *>(dev + kStepBytes);
+    b->h_alive = reinterpret_cast<int *>(b->h_records + rec);
     {
         int khz = 0;
         if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, params->device) != hipSuccess || khz <= 0)
@@ -1113,8 +1118,6 @@ int mcac_box_create(const mcac_box_params *params, mcac_box **out) {
         b->eng_clock_khz = khz;
         b->eng_idle_ticks = static_cast<unsigned long long>(khz) * 500ull;  // an idle grid ends after 0.5 s
     }
-    for (auto &e : b->ev)
-        if (hipEventCreate(&e) != hipSuccess) return fail(MCAC_E_DEVICE);
     *out = b;
     return 0;
 }
@@ -1122,12 +1125,11 @@ int mcac_box_create(const mcac_box_params *params, mcac_box **out) {
 int mcac_box_destroy(mcac_box *b) {
     if (!b) return 0;
     if (b->stream) (void)hipStreamSynchronize(bstream(b));  // a resident engine ends first
-    for (void *p : b->allocs) (void)hipFree(p);
-    if (b->h_step) (void)hipHostFree(b->h_step);
-    if (b->h_merge) (void)hipHostFree(b->h_merge);
+    if (b->arena) (void)hipFree(b->arena);
+    if (b->moved_members) (void)hipFree(b->moved_members);
+    if (b->h_records) (void)hipHostFree(b->h_records);
     if (b->h_alpha) (void)hipHostFree(b->h_alpha);
     if (b->h_cstart) (void)hipHostFree(b->h_cstart);
-    if (b->h_alive) (void)hipHostFree(b->h_alive);
     if (b->alive_read) (void)hipEventDestroy(b->alive_read);
     if (b->h_ring) (void)hipHostFree(b->h_ring);
     if (b->h_grow) (void)hipHostFree(b->h_grow);
@@ -1150,10 +1152,29 @@ int mcac_box_upload(mcac_box *b, int64_t ns, const double *x, const double *y, c
     if (!b || ns < 0 || na < 0 || ns > b->p.max_spheres || na > b->p.max_aggregates) return MCAC_E_ARGUMENT;
     const size_t S = static_cast<size_t>(ns), A = static_cast<size_t>(na);
     int rc = 0;
-    auto up = [&](double *dst, const double *src, size_t n) -> int {
-        if (n) HIP_TRY(hipMemcpy(dst, src, n * sizeof(double), hipMemcpyHostToDevice));
+    HIP_TRY(hipSetDevice(b->p.device));
+    if (!bstream(b)) return MCAC_E_DEVICE;
+    HIP_TRY(hipStreamSynchronize(b->stream));
+    // a small box's state goes up in a few copies, put together on the host (the
+    // buffers lie one behind the other); a large one's array by array
+    constexpr size_t kStageBytes = size_t(4) << 20;
+    struct Part {
+        char *lo = nullptr, *hi = nullptr;
+        std::vector<char> host;
+        bool holds(const void *p) const { return p >= lo && p < hi; }
+    };
+    Part parts[2];
+    auto put = [&](void *dst, const void *src, size_t bytes) -> int {
+        if (bytes == 0) return 0;
+        for (Part &q : parts)
+            if (q.holds(dst)) {
+                std::memcpy(q.host.data() + (static_cast<char *>(dst) - q.lo), src, bytes);
+                return 0;
+            }
+        HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, b->stream));
         return 0;
     };
+    auto up = [&](double *dst, const double *src, size_t n) -> int { return put(dst, src, n * sizeof(double)); };
     std::vector<double> hx(A), hy(A), hz(A), hrx(A), hry(A), hrz(A), c0(A), c1(A), c2(A), csr(A), cvr2(A);
     std::vector<int> cell(A, -1), cnt(A, 0), st(A, 0);
     std::vector<int> alive;
@@ -1204,8 +1225,21 @@ int mcac_box_upload(mcac_box *b, int64_t ns, const double *x, const double *y, c
         }
     }
     if (static_cast<int64_t>(pool.size()) > b->pool_cap) return MCAC_E_CAPACITY;
+    if (reinterpret_cast<char *>(b->d.acap + b->p.max_aggregates) - reinterpret_cast<char *>(b->d.sx) <=
+        static_cast<std::ptrdiff_t>(kStageBytes)) {
+        // spheres and aggregates up to the gyration radii (not part of the
+        // state), the merge caches and segments, the live ids
+        auto part = [](Part &q, auto *first, auto *end) {
+            q.lo = reinterpret_cast<char *>(first);
+            q.hi = reinterpret_cast<char *>(end);
+            q.host.resize(static_cast<size_t>(q.hi - q.lo));
+        };
+        part(parts[0], b->d.sx, b->d.asurf + A);
+        part(parts[1], b->d.csvx, b->d.acap + A);
+    }
+    std::vector<double> r3;
     if (b->p.volsurf == 2) {  // pow(r, 3) of the alphas sums (aggregat.cpp:402-403), host libm as the reference
-        std::vector<double> r3(S);
+        r3.resize(S);
         for (size_t s = 0; s < S; ++s) r3[s] = std::pow(r[s], 3.0);
         if ((rc = up(b->d.sr3, r3.data(), S))) return rc;
     }
@@ -1219,16 +1253,16 @@ int mcac_box_upload(mcac_box *b, int64_t ns, const double *x, const double *y, c
         (rc = up(b->d.csvx, c0.data(), A)) || (rc = up(b->d.csvy, c1.data(), A)) || (rc = up(b->d.csvz, c2.data(), A)) ||
         (rc = up(b->d.csr, csr.data(), A)) || (rc = up(b->d.csvr2, cvr2.data(), A)))
         return rc;
-    if (A) {
-        HIP_TRY(hipMemcpy(b->d.astart, st.data(), A * sizeof(int), hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(b->d.acount, cnt.data(), A * sizeof(int), hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(b->d.acell, cell.data(), A * sizeof(int), hipMemcpyHostToDevice));
-        HIP_TRY(hipMemcpy(b->d.acap, cnt.data(), A * sizeof(int), hipMemcpyHostToDevice));
-    }
-    if (!pool.empty()) HIP_TRY(hipMemcpy(b->d.members, pool.data(), pool.size() * sizeof(int), hipMemcpyHostToDevice));
-    if (!alive.empty()) HIP_TRY(hipMemcpy(b->d.alive, alive.data(), alive.size() * sizeof(int), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemset(b->d.ss, 0, sizeof(SearchState)));
-    HIP_TRY(hipDeviceSynchronize());
+    if ((rc = put(b->d.astart, st.data(), A * sizeof(int))) || (rc = put(b->d.acount, cnt.data(), A * sizeof(int))) ||
+        (rc = put(b->d.acell, cell.data(), A * sizeof(int))) || (rc = put(b->d.acap, cnt.data(), A * sizeof(int))) ||
+        (rc = put(b->d.members, pool.data(), pool.size() * sizeof(int))) ||
+        (rc = put(b->d.alive, alive.data(), alive.size() * sizeof(int))))
+        return rc;
+    for (Part &q : parts)
+        if (q.lo)
+            HIP_TRY(hipMemcpyAsync(q.lo, q.host.data(), q.host.size(), hipMemcpyHostToDevice, b->stream));
+    HIP_TRY(hipMemsetAsync(b->d.ss, 0, sizeof(SearchState), b->stream));
+    HIP_TRY(hipStreamSynchronize(b->stream));
     b->n_spheres = ns;
     b->n_aggs = na;
     b->count = cnt;
@@ -1576,8 +1610,10 @@ int mcac_group_destroy(mcac_group *g) {
 int mcac_group_add(mcac_group *g, mcac_box *b) {
     if (!g || !b || b->group || b->inflight || b->p.device != g->device) return MCAC_E_ARGUMENT;
     b->eng_blocks = 0;  // the group's launches take the box's steps
-    HIP_TRY(hipStreamSynchronize(bstream(b)));
-    if (b->own_stream) HIP_TRY(hipStreamDestroy(b->stream));
+    if (b->stream) {
+        HIP_TRY(hipStreamSynchronize(bstream(b)));
+        if (b->own_stream) HIP_TRY(hipStreamDestroy(b->stream));
+    }
     b->stream = g->stream;
     b->own_stream = false;
     b->group = g;
@@ -2039,6 +2075,22 @@ int mcac_box_grow(mcac_box *b, double dr, double *volume, double *surface, doubl
 int mcac_box_set_engine(mcac_box *b, int blocks) {
     if (!b || blocks < 0 || blocks > 255 || (blocks > 0 && b->group)) return MCAC_E_ARGUMENT;
     engine_stop(b);
+    if (blocks > 0 && !b->h_ring) {
+        HIP_TRY(hipSetDevice(b->p.device));
+        if (!bstream(b)) return MCAC_E_DEVICE;
+        EngineJob *ring = nullptr;
+        HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&ring), kEngineRing * sizeof(EngineJob), hipHostMallocCoherent));
+        std::memset(static_cast<void *>(ring), 0, kEngineRing * sizeof(EngineJob));
+        b->h_ring = ring;
+        HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void **>(&b->dp_ring), b->h_ring, 0));
+    }
+    if (blocks > 0 && !b->h_ctl) {
+        EngineCtl *ctl = nullptr;
+        HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&ctl), sizeof(EngineCtl), hipHostMallocCoherent));
+        std::memset(ctl, 0, sizeof(EngineCtl));
+        b->h_ctl = ctl;
+        HIP_TRY(hipHostGetDevicePointer(reinterpret_cast<void **>(&b->dp_ctl), b->h_ctl, 0));
+    }
     b->eng_blocks = blocks;
     return 0;
 }
@@ -2053,7 +2105,7 @@ int mcac_box_engine_stats(mcac_box *b, double out[8]) {
     out[2] = static_cast<double>(s.eng_steps);
     out[3] = static_cast<double>(s.eng_busy) / b->eng_clock_khz;  // ms
     out[4] = static_cast<double>(b->eng_relaunches);
-    out[5] = static_cast<double>(b->h_ctl->reason);
+    out[5] = b->h_ctl ? static_cast<double>(b->h_ctl->reason) : 0.0;
     out[6] = static_cast<double>(s.eng_idle) / b->eng_clock_khz;  // ms
     out[7] = static_cast<double>(b->eng_grid);
     return 0;
@@ -2061,7 +2113,10 @@ int mcac_box_engine_stats(mcac_box *b, double out[8]) {
 
 int mcac_box_set_timing(mcac_box *b, int enable) {
     if (!b) return MCAC_E_ARGUMENT;
-    if (enable > 0)  // the per-slot events of timed steps, made on first use
+    if (enable > 0)  // the events of timed merges and steps, made on first use
+        for (auto &e : b->ev)
+            if (!e) HIP_TRY(hipEventCreate(&e));
+    if (enable > 0)
         for (auto &row : b->sev)
             for (auto &e : row)
                 if (!e) HIP_TRY(hipEventCreate(&e));
