@@ -65,6 +65,7 @@ __global__ __launch_bounds__(kBlock) void k_cell_scatter(DevBox b, int n_alive) 
             b.cpy[pos] = b.ay[id];
             b.cpz[pos] = b.az[id];
             b.cpr[pos] = b.armax[id];
+            b.cinfo[pos] = entry_info(b, id);
             b.cf[pos] = make_float4(static_cast<float>(b.ax[id]), static_cast<float>(b.ay[id]),
                                     static_cast<float>(b.az[id]), static_cast<float>(b.armax[id]));
         }
@@ -132,6 +133,7 @@ __global__ __launch_bounds__(kBuildThreads) void k_cell_build_small(DevBox b, in
             b.cpy[pos] = b.ay[id];
             b.cpz[pos] = b.az[id];
             b.cpr[pos] = b.armax[id];
+            b.cinfo[pos] = entry_info(b, id);
             b.cf[pos] = make_float4(static_cast<float>(b.ax[id]), static_cast<float>(b.ay[id]),
                                     static_cast<float>(b.az[id]), static_cast<float>(b.armax[id]));
         }

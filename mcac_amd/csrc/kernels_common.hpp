@@ -155,6 +155,13 @@ __device__ __forceinline__ void mark_dirty(const DevBox &b, int id) {
     }
 }
 
+// Size and member segment of an aggregate as the search's packed entries hold
+// them: of one sphere, ~ that sphere.
+__device__ __forceinline__ int2 entry_info(const DevBox &b, int id) {
+    const int n = b.acount[id], st = b.astart[id];
+    return make_int2(n, n == 1 ? ~b.members[st] : st);
+}
+
 // Current CoM, rmax and cell of a dirty aggregate, read by the search.
 __device__ __forceinline__ void set_dirty_entry(const DevBox &b, int slot, double x, double y, double z, double r,
                                                 int cell) {

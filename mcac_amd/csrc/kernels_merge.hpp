@@ -84,6 +84,7 @@ __device__ __forceinline__ void store_merged(const DevBox &b, const MergeArgs &a
     b.dpy[b.dslot[k]] = com[1];
     b.dpz[b.dslot[k]] = com[2];
     b.dpcell[b.dslot[k]] = b.acell[k];
+    b.dinfo[b.dslot[k]] = make_int2(a.n_k + a.n_r, a.new_start);
     b.dpcell[b.dslot[a.rem]] = -1;
     b.cslot[a.rem] = -1;  // removed for good: no entry of a later build is its
 }
@@ -297,6 +298,7 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
         b.dpy[dsk] = com[1];
         b.dpz[dsk] = com[2];
         b.dpcell[dsk] = cell;
+        b.dinfo[dsk] = make_int2(n, a.new_start);
         b.dpcell[dsr] = -1;
         b.cslot[a.rem] = -1;
         for (int l = 0; l < 3; ++l) r[l] = rr[l];

@@ -24,7 +24,7 @@ namespace mcac_dev {
 struct BoxSink {
     const DevBox &b;
     int cap;
-    __device__ __forceinline__ void operator()(int id, int rank, double d) const {
+    __device__ __forceinline__ void operator()(int id, int rank, double d, int2, int) const {
         const unsigned int slot = atomicAdd(&b.ss->nfilt, 1u);
         if (slot < static_cast<unsigned int>(cap)) {
             b.cand_db[slot] = d;
@@ -47,6 +47,7 @@ struct Moved {
     int id[kMaxSteps], cell[kMaxSteps];
     double x[kMaxSteps], y[kMaxSteps], z[kMaxSteps], r[kMaxSteps];  // centre of mass and rmax
     double rx[kMaxSteps], ry[kMaxSteps], rz[kMaxSteps];             // centre - relative centre: its spheres' origin
+    int2 info[kMaxSteps];                                           // as DevBox::cinfo
 };
 
 // Positions of spheres as a step sees them: an aggregate with entry m >= 0 of
@@ -66,12 +67,13 @@ template <bool kMoved> struct Places {
             z = b.sz[sp];
         }
     }
-    __device__ __forceinline__ int entry(int id) const {
-        int e = -1;
-        if (kMoved)
-            for (int m = 0; m < mv->n; ++m)
-                if (mv->id[m] == id) e = m;
-        return e;
+    // the mover's sphere of this thread
+    template <class Sphere>
+    __device__ __forceinline__ void of(int m, const Sphere &s, double &x, double &y, double &z) const {
+        const bool moved = kMoved && m >= 0;
+        x = moved ? mv->rx[m] + s.rx : s.x;
+        y = moved ? mv->ry[m] + s.ry : s.y;
+        z = moved ? mv->rz[m] + s.rz : s.z;
     }
 };
 
@@ -142,6 +144,17 @@ __device__ __forceinline__ CellBounds load_cell_bounds(const DevBox &b, const Se
     return cb;
 }
 
+// Largest c of the n entries with pre[c] <= w (pre ascending from 0).
+template <class T> __device__ __forceinline__ int last_not_above(const T *pre, int n, T w) {
+    int lo = 0, hi = n;
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (pre[mid] <= w) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
 // Bounds of the visited cells in LDS.
 struct FilterLds {
     int win[6], nvisit;
@@ -151,7 +164,8 @@ struct FilterLds {
 
 // Filter work of block vb of the vg blocks on this step: the aggregates of the
 // reference's visited Verlet cells and the dirty list, bounding sweep,
-// survivors to `append` (shared by every form of the search).  With skip the
+// survivors to `append` (id, visit rank, bounding distance, cinfo, moved-set
+// entry; shared by every form of the search).  With skip the
 // work is read-only (a step behind a closed gate appends nothing).  nd: entries
 // of the dirty list.  kMoved: the aggregates of the moved set are taken from
 // there, by the first block.
@@ -289,7 +303,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
             cnt += 1;
             const double d = bounding(mv->x[m], mv->y[m], mv->z[m], mv->r[m]);
             if (d < a.lpm && !skip) {
-                append(mv->id[m], (oi * lj + oj) * lk + ok, d);
+                append(mv->id[m], (oi * lj + oj) * lk + ok, d, mv->info[m], m);
                 cnt += kAppendOne;
             }
         }
@@ -304,6 +318,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
         for (int w0 = gtid; w0 < total; w0 += kSweep * gstride) {
             int rk[kSweep] = {}, idv[kSweep];
             double xv[kSweep], yv[kSweep], zv[kSweep], rv[kSweep];
+            int pv[kSweep];
             for (int s = top; s > 0; s >>= 1) {  // largest v with pre[v] <= w, as above
 #pragma unroll
                 for (int u = 0; u < kSweep; ++u) {
@@ -317,8 +332,10 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
                 idv[u] = a.src;
                 xv[u] = yv[u] = zv[u] = 0.0;
                 rv[u] = -1.0;
+                pv[u] = 0;
                 if (w < total) {
                     const int pos = cbeg[rk[u]] + (w - pre[rk[u]]);
+                    pv[u] = pos;
                     idv[u] = b.citems[pos];
                     xv[u] = b.cpx[pos];
                     yv[u] = b.cpy[pos];
@@ -332,7 +349,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
                 cnt += 1;
                 const double d = bounding(xv[u], yv[u], zv[u], rv[u]);
                 if (d < a.lpm && !skip) {
-                    append(idv[u], rk[u], d);
+                    append(idv[u], rk[u], d, b.cinfo[pv[u]], -1);
                     cnt += kAppendOne;
                 }
             }
@@ -347,7 +364,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
             cnt += 1;
             const double d = bounding(b.dpx[i], b.dpy[i], b.dpz[i], b.dpr[i]);
             if (d < a.lpm && !skip) {
-                append(id, (oi * lj + oj) * lk + ok, d);
+                append(id, (oi * lj + oj) * lk + ok, d, b.dinfo[i], -1);
                 cnt += kAppendOne;
             }
         }
@@ -356,6 +373,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
     for (int w = gtid; w < total + nd; w += gstride) {
         int id, rank;
         double x, y, z, r;
+        int2 info;
         if (w < total) {
             int pos;
             if (V <= kMaxVisit) {
@@ -392,6 +410,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
             y = b.cpy[pos];
             z = b.cpz[pos];
             r = b.cpr[pos];
+            info = b.cinfo[pos];
             if (r < 0.0 || elsewhere(id)) continue;  // moved since the build, or the mover
             if (V > kMaxVisit) {
                 const int c = ref_cell(x, y, z, n, a.L);
@@ -408,6 +427,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
             y = b.dpy[i];
             z = b.dpz[i];
             r = b.dpr[i];
+            info = b.dinfo[i];
             if (c < 0 || elsewhere(id)) continue;
             int oi = window_offset(c / (n * n), b1i, n), oj = window_offset((c / n) % n, b1j, n),
                 ok = window_offset(c % n, b1k, n);
@@ -417,7 +437,7 @@ __device__ __forceinline__ unsigned long long filter_phase(const DevBox &b, cons
         cnt += 1;
         const double d = bounding(x, y, z, r);
         if (d < a.lpm && !skip) {
-            append(id, rank, d);
+            append(id, rank, d, info, -1);
             cnt += kAppendOne;
         }
     }
@@ -453,15 +473,19 @@ struct StepPick {
     int overflow;
     int src_slot;               // packed cell entry of the mover (-1: none)
     int handover;               // survivors left to the grid form: no contact known
+    int on, pad;                // size of the other aggregate
 };
 
 // Survivors of a one-launch step (at most kStepCands), kept in LDS by the
 // finishing block: bounding distance, visit rank, label, size and member
-// segment, moved-set entry, exact (d, pair) minimum, and the multimap order.
+// segment (or ~ its only sphere), moved-set entry, exact minimum, and the
+// multimap order.
 struct StepCands {
     double db[kStepCands], ex[kStepCands];
-    long long pair[kStepCands];
+    int ms[kStepCands], os[kStepCands];  // spheres of the minimum
     int rank[kStepCands], id[kStepCands], nk[kStepCands], sk[kStepCands], mv[kStepCands], order[kStepCands];
+    double mx[kThreadPairs], my[kThreadPairs], mz[kThreadPairs], mr[kThreadPairs];  // a small mover's spheres
+    int msp[kThreadPairs];
     int pre[kStepCands + 1];  // spheres before each survivor's
     unsigned int n;           // survivors of a search by one block (may exceed kStepCands)
 };
@@ -471,11 +495,12 @@ struct StepCands {
 struct MoverSphere {
     int loaded;  // the block loaded the mover (uniform)
     int sp;      // this thread's sphere, -1: none
-    double rx, ry, rz;
+    double rx, ry, rz;     // relative position
+    double x, y, z, r;     // position in the box, radius
 };
 
 __device__ __forceinline__ MoverSphere load_mover_sphere(const DevBox &b, const SearchArgs &a) {
-    MoverSphere m{a.apply && a.n_mov <= kBlock, -1, 0., 0., 0.};
+    MoverSphere m{a.n_mov <= kBlock, -1, 0., 0., 0., 0., 0., 0., 0.};
     if (m.loaded && static_cast<int>(threadIdx.x) < a.n_mov) {
         m.sp = b.members[a.start + threadIdx.x];
         m.rx = b.srx[m.sp];
@@ -522,6 +547,8 @@ struct SolveLds {
     // kept spheres of the tile: nearest image to the mover, stored position, radius
     double qx[kBlock], qy[kBlock], qz[kBlock], px[kBlock], py[kBlock], pz[kBlock], pr[kBlock];
     int cand[kBlock], idx[kBlock];                // their candidate (from the tile's first) and sphere number in it
+    int sp[kBlock], msp[kMoverTile];              // sphere indices
+    int bms[kBlock], bos[kBlock];                 // per candidate of the tile: spheres of pmin
     unsigned long long dmin[kBlock];              // per candidate of the tile: least distance (ordered bits)
     unsigned long long pmin[kBlock];              // and least pair index at it
     double rd[kBlock];                            // minimum of each kept sphere over the mover's
@@ -586,15 +613,24 @@ __device__ __forceinline__ void scan_candidates(const DevBox &b, unsigned int F,
         }
         pick.dist = closest;
         pick.ms = pick.os = pick.oagg = -1;
+        pick.on = 0;
         if (best >= 0) {
-            const long long p = lc ? lc->pair[best] : b.cand_pair[best];
-            const int k = lc ? lc->id[best] : b.cand_id[best];
-            const long long nk = lc ? lc->nk[best] : b.acount[k];
-            const int sk = lc ? lc->sk[best] : b.astart[k];
-            const long long i = p / nk, j = p - i * nk;
-            pick.ms = b.members[ssrc + i];
-            pick.os = b.members[sk + j];
-            pick.oagg = k;
+            if (lc) {
+                pick.ms = lc->ms[best];
+                pick.os = lc->os[best];
+                pick.oagg = lc->id[best];
+                pick.on = lc->nk[best];
+            } else {
+                const long long p = b.cand_pair[best];
+                const int k = b.cand_id[best];
+                const long long nk = b.acount[k];
+                const int sk = b.astart[k];
+                const long long i = p / nk, j = p - i * nk;
+                pick.ms = b.members[ssrc + i];
+                pick.os = b.members[sk + j];
+                pick.oagg = k;
+                pick.on = static_cast<int>(nk);
+            }
         }
     }
 }
@@ -612,9 +648,16 @@ __device__ __forceinline__ bool apply_step(const DevBox &b, const SearchArgs &a,
     __shared__ double s_ref[3];
     __shared__ StepRecord srec;  // assembled here, copied to host memory by one wave
     SearchState *s = b.ss;
+    int other_n = 0, other_start = 0, keep_cap = 0;  // of a contact's merge (thread 0)
     if (threadIdx.x == 0) {
         // every load of this thread comes before its stores (no reloads through global memory)
         const double closest = pick.dist;
+        if (pick.oagg >= 0 && closest <= a.lpm && a.automerge) {
+            const int o = static_cast<int>(pick.oagg);
+            other_n = pick.on;
+            other_start = b.astart[o];
+            keep_cap = b.acap[a.src < o ? a.src : o];
+        }
         // calcul.cpp:128-130 and aggregat.cpp:148-153
         const int contact = closest <= a.lpm;
         const double move = contact ? closest : a.lpm;
@@ -682,6 +725,7 @@ __device__ __forceinline__ bool apply_step(const DevBox &b, const SearchArgs &a,
                 }
             }
             set_dirty_entry(b, a.dirty_pos, ncom[0], ncom[1], ncom[2], rmax_src, ncell);
+            b.dinfo[a.dirty_pos] = make_int2(a.n_mov, a.n_mov == 1 && m.loaded ? ~m.sp : a.start);
         }
         if (a.gated && contact) s->gate = a.seq;  // the steps behind wait for the merge
         closed = a.gated && contact;
@@ -717,12 +761,12 @@ __device__ __forceinline__ bool apply_step(const DevBox &b, const SearchArgs &a,
             if (srec.contact) {
                 const int oagg = static_cast<int>(srec.oagg);
                 const int keep = a.src < oagg ? a.src : oagg, rem = a.src < oagg ? oagg : a.src;
-                const int nk = (keep == a.src) ? a.n_mov : b.acount[keep];
-                const int nr = (rem == a.src) ? a.n_mov : b.acount[rem];
-                const int start_k = (keep == a.src) ? a.start : b.astart[keep];
-                const int start_r = (rem == a.src) ? a.start : b.astart[rem];
+                const int nk = (keep == a.src) ? a.n_mov : other_n;
+                const int nr = (rem == a.src) ? a.n_mov : other_n;
+                const int start_k = (keep == a.src) ? a.start : other_start;
+                const int start_r = (rem == a.src) ? a.start : other_start;
                 const int n = nk + nr;
-                int new_start = start_k, new_cap = b.acap[keep];
+                int new_start = start_k, new_cap = keep_cap;
                 bool fits = n <= kSmallMerge;
                 if (fits && n > new_cap) {  // a fresh segment of twice the merged size
                     new_cap = (2 * n > 4) ? 2 * n : 4;
@@ -789,17 +833,26 @@ __device__ __forceinline__ double from_ordered_bits(unsigned long long u) {
 // that holds them (block-uniform).
 template <class Where>
 __device__ __forceinline__ double load_mover_tile(const DevBox &b, SolveLds &u, int ssrc, long long i0, int nt,
-                                                  const double centre[3], int self, const Where &where) {
+                                                  const double centre[3], int self, const Where &where,
+                                                  const MoverSphere *own = nullptr) {
     double far = 0.0;
     for (int t = threadIdx.x; t < nt; t += blockDim.x) {
-        const int sp = b.members[ssrc + i0 + t];
-        double x, y, z;
-        const double r = b.sr[sp];
-        where(self, sp, x, y, z);
+        double x, y, z, r;
+        int sp;
+        if (own) {  // the thread's sphere, loaded with the step's first loads
+            sp = own->sp;
+            r = own->r;
+            where.of(self, *own, x, y, z);
+        } else {
+            sp = b.members[ssrc + i0 + t];
+            r = b.sr[sp];
+            where(self, sp, x, y, z);
+        }
         u.mx[t] = x;
         u.my[t] = y;
         u.mz[t] = z;
         u.mr[t] = r;
+        u.msp[t] = sp;
         const double d0 = x - centre[0], d1 = y - centre[1], d2 = z - centre[2];
         const double f = __builtin_sqrt(d0 * d0 + d1 * d1 + d2 * d2) + r;
         far = !(f <= far) ? f : far;  // a NaN stays: nothing is pruned then
@@ -816,7 +869,8 @@ __device__ __forceinline__ double load_mover_tile(const DevBox &b, SolveLds &u, 
 }
 
 // One tile: thread t holds sphere number j of candidate cl (counted from the
-// tile's first; cl < 0: no sphere), listed at member slot m, of an aggregate
+// tile's first; cl < 0: no sphere), listed at member slot m (`member` itself
+// where that is known, else -1), of an aggregate
 // with moved-set entry `entry`, against the nt mover spheres in LDS (numbers i0 ...).  Returns whether some pair of the tile
 // has a finite distance: then u.dmin / u.pmin hold the minima of its ncl (at
 // most kBlock) candidates, candidate cl's for thread cl, where they are at most
@@ -825,12 +879,14 @@ __device__ __forceinline__ double load_mover_tile(const DevBox &b, SolveLds &u, 
 template <class Where, class Size>
 __device__ __forceinline__ bool solve_tile(const DevBox &b, const SearchArgs &a, const SweepTest &sw, SolveLds &u,
                                            const double centre[3], double reach, long long i0, int nt, int cl,
-                                           long long j, long long m, int entry, const Where &where, int ncl, double best,
+                                           long long j, long long m, int member, int entry, const Where &where, int ncl,
+                                           double best,
                                            Size &&nk) {
     double x = 0, y = 0, z = 0, r = 0, q0 = 0, q1 = 0, q2 = 0;
     bool keep = false;
+    int sp = -1;
     if (cl >= 0) {
-        const int sp = b.members[m];
+        sp = member >= 0 ? member : b.members[m];
         r = b.sr[sp];
         where(entry, sp, x, y, z);
         const double d0 = nearest_image(x - centre[0], sw.hx, sw), d1 = nearest_image(y - centre[1], sw.hy, sw),
@@ -871,6 +927,7 @@ __device__ __forceinline__ bool solve_tile(const DevBox &b, const SearchArgs &a,
         u.pr[e] = r;
         u.cand[e] = cl;
         u.idx[e] = static_cast<int>(j);
+        u.sp[e] = sp;
     }
     lds_barrier();
     // a kept sphere by g lanes, each over every g-th mover sphere
@@ -923,24 +980,17 @@ __device__ __forceinline__ bool solve_tile(const DevBox &b, const SearchArgs &a,
     }
     lds_barrier();
     if (!u.found) return false;
-    if (static_cast<int>(threadIdx.x) < kept) {
-        const int e = threadIdx.x;
-        if (u.rd[e] < kInf && ordered_bits(u.rd[e]) == u.dmin[u.cand[e]])
-            atomicMin(&u.pmin[u.cand[e]], static_cast<unsigned long long>(u.rp[e]));
+    // every thread passes the barriers
+    const int e = threadIdx.x;
+    const bool least = e < kept && u.rd[e] < kInf && ordered_bits(u.rd[e]) == u.dmin[u.cand[e]];
+    if (least) atomicMin(&u.pmin[u.cand[e]], static_cast<unsigned long long>(u.rp[e]));
+    lds_barrier();
+    if (least && u.pmin[u.cand[e]] == static_cast<unsigned long long>(u.rp[e])) {
+        u.bms[u.cand[e]] = u.msp[(u.rp[e] - u.idx[e]) / nk(u.cand[e]) - i0];
+        u.bos[u.cand[e]] = u.sp[e];
     }
     lds_barrier();
     return true;
-}
-
-// Largest c of the n entries with pre[c] <= w (pre ascending from 0).
-template <class T> __device__ __forceinline__ int last_not_above(const T *pre, int n, T w) {
-    int lo = 0, hi = n;
-    while (hi - lo > 1) {
-        const int mid = (lo + hi) >> 1;
-        if (pre[mid] <= w) lo = mid;
-        else hi = mid;
-    }
-    return lo;
 }
 
 // Pair solve of the survivors filtered for step a: the tiles of the candidates'
@@ -1016,7 +1066,7 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
             for (int q = 0; q < n_movers; ++q) {
                 mover_tile(q);
                 if (solve_tile(b, a, sw, u, centre, reach, static_cast<long long>(q) * kMoverTile, nt, cl, j, m,
-                               -1, where, c1 - c0 + 1, bd, [&](int e) { return cpre[c0 + e + 1] - cpre[c0 + e]; }) &&
+                               -1, -1, where, c1 - c0 + 1, bd, [&](int e) { return cpre[c0 + e + 1] - cpre[c0 + e]; }) &&
                     static_cast<int>(threadIdx.x) <= c1 - c0 && u.pmin[threadIdx.x] != ~0ull)
                     lexmin(bd, bp, from_ordered_bits(u.dmin[threadIdx.x]), static_cast<long long>(u.pmin[threadIdx.x]));
             }
@@ -1038,7 +1088,7 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
                 for (long long w0 = 0; w0 < nk; w0 += kBlock) {
                     const long long j = w0 + threadIdx.x;
                     if (solve_tile(b, a, sw, u, centre, reach, static_cast<long long>(q) * kMoverTile, nt,
-                                   j < nk ? 0 : -1, j, sk + j, -1, where, 1, bd, [&](int) { return nk; }) &&
+                                   j < nk ? 0 : -1, j, sk + j, -1, -1, where, 1, bd, [&](int) { return nk; }) &&
                         threadIdx.x == 0 && u.pmin[0] != ~0ull)
                         lexmin(bd, bp, from_ordered_bits(u.dmin[0]), static_cast<long long>(u.pmin[0]));
                 }
@@ -1095,7 +1145,7 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
         pick.tpairs = nsrc * T;
         pick.handover = 0;
     }
-    apply_step(b, a, pick, MoverSphere{0, -1, 0., 0., 0.}, true, lds.merge);
+    apply_step(b, a, pick, MoverSphere{0, -1, 0., 0., 0., 0., 0., 0., 0.}, true, lds.merge);
 }
 
 __global__ __launch_bounds__(kBlock) void k_solve(DevBox b, SearchArgs a) {
@@ -1147,19 +1197,23 @@ struct StepSink {
     const DevBox &b;
     StepCands &sc;
     int q, slots;  // the step's number and its share of the buffer (-1: LDS)
-    __device__ __forceinline__ void operator()(int id, int rank, double d) const {
+    __device__ __forceinline__ void operator()(int id, int rank, double d, int2 info, int entry) const {
         if (slots < 0) {
             const unsigned int c = atomicAdd(&sc.n, 1u);
             if (c >= static_cast<unsigned int>(kStepCands)) return;  // counted: left to the grid form
             sc.id[c] = id;
             sc.rank[c] = rank;
             sc.db[c] = d;
+            sc.nk[c] = info.x;
+            sc.sk[c] = info.y;
+            sc.mv[c] = entry;
         } else {
             const unsigned int c = atomicAdd(&b.ss->step_nfilt[q], 1u);
             if (c >= static_cast<unsigned int>(slots)) return;
             b.cand_id[q * slots + c] = id;
             b.cand_rank[q * slots + c] = rank;
             b.cand_db[q * slots + c] = d;
+            b.step_info[q * kStepCands + c] = make_int4(info.x, info.y, entry, 0);
         }
     }
 };
@@ -1183,7 +1237,7 @@ __device__ __forceinline__ int search_step(const DevBox &b, const SearchArgs &a,
     // independent loads first, so that their latencies overlap: the gate, the
     // mover's cell entry and sphere indices, the bounds of the visited cells
     const unsigned long long gate = (!gate_open && a.gated) ? b.ss->gate : 0ull;
-    const bool mload = a.apply && a.n_mov <= kBlock;
+    const bool mload = a.n_mov <= kBlock;
     int src_slot = -1, msp = -1;
     if (pre) {
         src_slot = pre->src_slot;
@@ -1194,13 +1248,18 @@ __device__ __forceinline__ int search_step(const DevBox &b, const SearchArgs &a,
     }
     const CellBounds cb = load_cell_bounds(b, a, ct);
     const bool skip = gate != 0ull && gate < a.seq && gate > a.released;
-    mover = MoverSphere{mload, msp, 0., 0., 0.};
-    if (pre) {
-        mover = pre->mover;
-    } else if (msp >= 0) {
-        mover.rx = b.srx[msp];
-        mover.ry = b.sry[msp];
-        mover.rz = b.srz[msp];
+    mover = MoverSphere{mload, msp, 0., 0., 0., 0., 0., 0., 0.};
+    if (pre) mover = pre->mover;
+    if (msp >= 0) {
+        if (!pre) {
+            mover.rx = b.srx[msp];
+            mover.ry = b.sry[msp];
+            mover.rz = b.srz[msp];
+        }
+        mover.x = b.sx[msp];
+        mover.y = b.sy[msp];
+        mover.z = b.sz[msp];
+        mover.r = b.sr[msp];
     }
     if (threadIdx.x == 0) sc.n = 0u;  // filter_phase appends behind a barrier
     const int share = a.cap / kMaxSteps < kStepCands ? a.cap / kMaxSteps : kStepCands;
@@ -1255,13 +1314,19 @@ __device__ __forceinline__ int search_step(const DevBox &b, const SearchArgs &a,
                 sc.id[c] = b.cand_id[q * share + c];
                 sc.db[c] = b.cand_db[q * share + c];
                 sc.rank[c] = b.cand_rank[q * share + c];
+                const int4 v = b.step_info[q * kStepCands + c];
+                sc.nk[c] = v.x;
+                sc.sk[c] = v.y;
+                sc.mv[c] = v.z;
             }
-            const int k = sc.id[c];
-            const int nk = b.acount[k];
-            tp += nsrc * nk;
-            sc.nk[c] = nk;
-            sc.sk[c] = b.astart[k];
-            sc.mv[c] = where.entry(k);
+            tp += nsrc * sc.nk[c];
+        }
+        if (mload && nsrc <= kThreadPairs && threadIdx.x < nsrc) {
+            // a small mover's spheres, loaded with the step's first loads
+            const int t = threadIdx.x;
+            sc.msp[t] = mover.sp;
+            sc.mr[t] = mover.r;
+            where.of(self, mover, sc.mx[t], sc.my[t], sc.mz[t]);
         }
         const long long tpairs = block_sum(tp);
         __shared__ int s_over;
@@ -1292,25 +1357,29 @@ __device__ __forceinline__ int search_step(const DevBox &b, const SearchArgs &a,
         // candidate: when every candidate has at most kThreadPairs pairs
         // (monomers), one thread walks a candidate's in (i, j) order (strict <
         // keeps the first minimum); else all candidates' spheres in tiles
-        if (s_most <= kThreadPairs) {
+        if (s_most <= kThreadPairs && mload) {
             if (threadIdx.x < F) {
                 const unsigned int c = threadIdx.x;
                 const int nk = sc.nk[c];  // this thread's own entries
                 const int sk = sc.sk[c];
                 double bd = kInf;
-                long long bp = 0x7fffffffffffffffLL;
-                for (long long p = 0; p < nsrc * nk; ++p) {
-                    const long long i = p / nk, j = p - i * nk;
-                    const int si = b.members[ssrc + i], sj = b.members[sk + j];
-                    double x1, y1, z1, x2, y2, z2;
-                    where(self, si, x1, y1, z1);
-                    where(sc.mv[c], sj, x2, y2, z2);
-                    const double d = swept_sphere(x1, y1, z1, b.sr[si], x2, y2, z2, b.sr[sj], a.dir[0], a.dir[1],
-                                                  a.dir[2], a.lpm, a.L);
-                    lexmin(bd, bp, d, p);
-                }
+                int bi = -1, bj = -1;
+                for (int i = 0; i < nsrc; ++i)
+                    for (int j = 0; j < nk; ++j) {
+                        const int sj = sk < 0 ? ~sk : b.members[sk + j];
+                        double x2, y2, z2;
+                        where(sc.mv[c], sj, x2, y2, z2);
+                        const double d = swept_sphere(sc.mx[i], sc.my[i], sc.mz[i], sc.mr[i], x2, y2, z2, b.sr[sj],
+                                                      a.dir[0], a.dir[1], a.dir[2], a.lpm, a.L);
+                        if (d < bd) {
+                            bd = d;
+                            bi = sc.msp[i];
+                            bj = sj;
+                        }
+                    }
                 sc.ex[c] = bd;
-                sc.pair[c] = (bd < kInf) ? bp : -1;
+                sc.ms[c] = bi;
+                sc.os[c] = bj;
             }
             lds_barrier();
         } else {
@@ -1321,29 +1390,39 @@ __device__ __forceinline__ int search_step(const DevBox &b, const SearchArgs &a,
             const int T = sc.pre[F];
             double bd = kInf;  // thread c: candidate c's minimum
             long long bp = 0x7fffffffffffffffLL;
+            int bi = -1, bj = -1;
             for (long long i0 = 0; i0 < nsrc; i0 += kMoverTile) {
                 const int nt = static_cast<int>(nsrc - i0 < kMoverTile ? nsrc - i0 : kMoverTile);
                 if (i0 > 0) lds_barrier();
-                const double reach = load_mover_tile(b, u, ssrc, i0, nt, centre, self, where);
+                const double reach = load_mover_tile(b, u, ssrc, i0, nt, centre, self, where, mload ? &mover : nullptr);
                 for (int w0 = 0; w0 < T; w0 += kBlock) {
                     const int w = w0 + static_cast<int>(threadIdx.x);
-                    int c = -1, j = 0, m = 0, e = -1;
+                    int c = -1, j = 0, m = 0, e = -1, one = -1;
                     if (w < T) {
                         c = last_not_above(sc.pre, static_cast<int>(F), w);
                         j = w - sc.pre[c];
                         m = sc.sk[c] + j;
                         e = sc.mv[c];
+                        if (sc.sk[c] < 0) one = ~sc.sk[c];
                     }
-                    if (solve_tile(b, a, sw, u, centre, reach, i0, nt, c, j, m, e, where, static_cast<int>(F), bd,
+                    if (solve_tile(b, a, sw, u, centre, reach, i0, nt, c, j, m, one, e, where, static_cast<int>(F), bd,
                                    [&](int k) { return static_cast<long long>(sc.nk[k]); }) &&
-                        threadIdx.x < F && u.pmin[threadIdx.x] != ~0ull)
-                        lexmin(bd, bp, from_ordered_bits(u.dmin[threadIdx.x]),
-                               static_cast<long long>(u.pmin[threadIdx.x]));
+                        threadIdx.x < F && u.pmin[threadIdx.x] != ~0ull) {
+                        const double d = from_ordered_bits(u.dmin[threadIdx.x]);
+                        const long long p = static_cast<long long>(u.pmin[threadIdx.x]);
+                        if (d < bd || (d == bd && p < bp)) {
+                            bd = d;
+                            bp = p;
+                            bi = u.bms[threadIdx.x];
+                            bj = u.bos[threadIdx.x];
+                        }
+                    }
                 }
             }
             if (threadIdx.x < F) {
                 sc.ex[threadIdx.x] = bd;
-                sc.pair[threadIdx.x] = (bd < kInf) ? bp : -1;
+                sc.ms[threadIdx.x] = bi;
+                sc.os[threadIdx.x] = bj;
             }
             lds_barrier();
         }
@@ -1445,6 +1524,7 @@ __device__ __forceinline__ void set_moved(Moved &mv, int q, int src, const Args 
         mv.rx[p] = e.nc_ref[0];
         mv.ry[p] = e.nc_ref[1];
         mv.rz[p] = e.nc_ref[2];
+        mv.info[p] = make_int2(e.n_mov, e.start);
     }
     if (threadIdx.x == 0) {
         int self = -1;
@@ -1470,9 +1550,11 @@ __device__ __forceinline__ void commit_steps(const DevBox &b, StepsLds &u, int n
         const SearchArgs &a = u.args[q];
         bool later = false;
         for (int p = q + 1; p < f; ++p) later = later || u.args[p].src == a.src;
+        int first_sphere = 0;  // lane 0's
         if (!later)
             for (int t = lane; t < a.n_mov; t += 64) {
                 const int sp = b.members[a.start + t];
+                if (t == 0) first_sphere = sp;
                 b.sx[sp] = a.nc_ref[0] + b.srx[sp];
                 b.sy[sp] = a.nc_ref[1] + b.sry[sp];
                 b.sz[sp] = a.nc_ref[2] + b.srz[sp];
@@ -1508,6 +1590,7 @@ __device__ __forceinline__ void commit_steps(const DevBox &b, StepsLds &u, int n
                 b.az[a.src] = a.nc_com[2];
                 b.acell[a.src] = a.nc_cell;
                 set_dirty_entry(b, a.dirty_pos, a.nc_com[0], a.nc_com[1], a.nc_com[2], a.srmax, a.nc_cell);
+                b.dinfo[a.dirty_pos] = make_int2(a.n_mov, a.n_mov == 1 ? ~first_sphere : a.start);
             }
         }
     }
@@ -1609,7 +1692,8 @@ struct BoxRun {
     int nj, pad;
     SearchArgs a[kMaxSteps];
 };
-constexpr int kMoveWords = static_cast<int>(offsetof(SearchArgs, n_mov) / sizeof(unsigned long long));
+constexpr int kMoveWords = static_cast<int>(offsetof(SearchArgs, known) / sizeof(unsigned long long));
+static_assert(offsetof(SearchArgs, known) % sizeof(unsigned long long) == 0, "move part in 8-byte words");
 
 __global__ __launch_bounds__(kBlock) void k_steps_group(const BoxRun *runs) {
     __shared__ StepsLds u;
@@ -1862,6 +1946,7 @@ __global__ void k_set_move(DevBox b, int src, double v0, double v1, double v2, i
     b.acell[src] = s->newcell;
     mark_dirty(b, src);
     set_dirty_entry(b, b.dslot[src], s->newcom[0], s->newcom[1], s->newcom[2], b.armax[src], s->newcell);
+    b.dinfo[b.dslot[src]] = entry_info(b, src);
 }
 
 __global__ void k_swept_batch(long long n, const double *p1, const double *r1, const double *p2, const double *r2,
