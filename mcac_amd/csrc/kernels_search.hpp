@@ -798,9 +798,8 @@ __device__ __forceinline__ bool apply_step(const DevBox &b, const SearchArgs &a,
         }
         lds_barrier();
         if (s_inline) {
-            // the merge takes the mover's sphere positions from s_ref, and the
-            // thread that placed a sphere of the mover also remaps it when the
-            // mover is removed: no wait for the placements above
+            // the merge takes the mover's sphere positions from s_ref: its
+            // loads do not wait for the placements above
             merge_small_block(b, s_ma, srec.merge, s_ref, u);
             if (threadIdx.x == 0) srec.merged_inline = 1;  // thread 0 also copies the record
         }
