@@ -79,7 +79,7 @@ struct MergeState {
     int ok, keep, rem, n_k, n_r, new_start, start_k, start_r;
     double diffpos[3], refpos[3], r[3];
     unsigned long long rmax_bits;
-    unsigned int row_overflow, pad;
+    unsigned int row_overflow, tiles_done;  // tiles_done: blocks of the last kernel that finished
     // list-order sums of the first alphas phase: V, S, Σ rel·vol (3), Σ r, Σ vol·r², Σ vol
     double sums[8];
     mcac_merge_result res;

@@ -1481,8 +1481,8 @@ int mcac_merge(mcac_box *b, const mcac_contact *c, mcac_merge_result *out) {
         const unsigned tiles = static_cast<unsigned>((n + kBlock - 1) / kBlock);
         hipLaunchKernelGGL(k_merge_prep, dim3(1), dim3(64), 0, bstream(b), b->d, a);
         hipLaunchKernelGGL(k_merge_lists, dim3(nb), dim3(kBlock), 0, bstream(b), b->d);
-        hipLaunchKernelGGL(k_overlap_pairs, dim3(tiles, tiles), dim3(kBlock), 0, bstream(b), b->d, 1);
-        hipLaunchKernelGGL(k_overlap_sum, dim3(1), dim3(kBlock), 0, bstream(b), b->d, a);
+        hipLaunchKernelGGL(k_overlap_pairs, dim3(tiles, tiles), dim3(kBlock), 0, bstream(b), b->d);
+        hipLaunchKernelGGL(k_overlap_sum, dim3(1), dim3(kBlock), 0, bstream(b), b->d);
         if (a.volsurf == 1) hipLaunchKernelGGL(k_caps_volumes, dim3(nb), dim3(kBlock), 0, bstream(b), b->d);
         else hipLaunchKernelGGL(k_arvo_volumes, dim3(nb), dim3(kBlock), 0, bstream(b), b->d);
         hipLaunchKernelGGL(k_caps_sums, dim3(1), dim3(kBlock), 0, bstream(b), b->d, a);
@@ -1510,8 +1510,8 @@ int mcac_merge(mcac_box *b, const mcac_contact *c, mcac_merge_result *out) {
         } else {
             hipLaunchKernelGGL(k_merge_prep, dim3(1), dim3(64), 0, bstream(b), b->d, a);
             hipLaunchKernelGGL(k_merge_lists, dim3(nb), dim3(kBlock), 0, bstream(b), b->d);
-            hipLaunchKernelGGL(k_overlap_pairs, dim3(tiles, tiles), dim3(kBlock), 0, bstream(b), b->d, 1);
-            hipLaunchKernelGGL(k_overlap_sum, dim3(1), dim3(kBlock), 0, bstream(b), b->d, a);
+            hipLaunchKernelGGL(k_overlap_pairs, dim3(tiles, tiles), dim3(kBlock), 0, bstream(b), b->d);
+            hipLaunchKernelGGL(k_overlap_sum, dim3(1), dim3(kBlock), 0, bstream(b), b->d);
             hipLaunchKernelGGL(k_alpha_walk, dim3(nb), dim3(kBlock), 0, bstream(b), b->d);
             hipLaunchKernelGGL(k_caps_sums, dim3(1), dim3(kBlock), 0, bstream(b), b->d, a);
         }
@@ -1544,12 +1544,10 @@ int mcac_merge(mcac_box *b, const mcac_contact *c, mcac_merge_result *out) {
         const int nb = std::min(4096, (n + kBlock - 1) / kBlock);
         hipLaunchKernelGGL(k_merge_prep, dim3(1), dim3(64), 0, bstream(b), b->d, a);
         hipLaunchKernelGGL(k_merge_lists, dim3(nb), dim3(kBlock), 0, bstream(b), b->d);
-        hipLaunchKernelGGL(k_merge_seq, dim3(1), dim3(kBlock), 0, bstream(b), b->d, a);
-        hipLaunchKernelGGL(k_merge_dc, dim3(nb), dim3(kBlock), 0, bstream(b), b->d);
-        hipLaunchKernelGGL(k_merge_rg, dim3(1), dim3(kBlock), 0, bstream(b), b->d, a);
         const unsigned tiles = static_cast<unsigned>((n + kBlock - 1) / kBlock);
-        hipLaunchKernelGGL(k_overlap_pairs, dim3(tiles, tiles), dim3(kBlock), 0, bstream(b), b->d, 0);
-        hipLaunchKernelGGL(k_overlap_sum, dim3(1), dim3(kBlock), 0, bstream(b), b->d, a);
+        const unsigned cols = static_cast<unsigned>((n + kPairCols - 1) / kPairCols);
+        hipLaunchKernelGGL(k_merge_pairs, dim3(cols, tiles + 1), dim3(kBlock), 0, bstream(b), b->d, a);
+        hipLaunchKernelGGL(k_merge_finish, dim3(tiles), dim3(kBlock), 0, bstream(b), b->d, a);
     }
     if (b->timing) HIP_TRY(hipEventRecord(b->ev[1], bstream(b)));
     HIP_TRY(hipGetLastError());
