@@ -163,7 +163,7 @@ struct SearchArgs {
     StepRecord *out;           // pinned host record
     unsigned long long seq;
     int gated;                 // pipelined step: closes the gate on contact, skipped behind it
-    int automerge;             // merge in the same launch on contact when small enough
+    int automerge;             // merge in the same launch on contact when small enough: 1 method none, 2 caps
     unsigned long long released;  // gate values up to this one are open for this step
     int prec;                  // 0 FP64; 1 FP32 capsule prune of cell entries; 2 as 1 plus miss count
     float margin32;            // FP32 prune margin added to the radius sum [m]

@@ -309,7 +309,7 @@ struct Simulation {
     // (calcul.cpp:156-160 always merges on contact) unless a growth step must
     // come first, and the persistent engine when asked for.
     int box_modes() {
-        int rc = mcac_box_set_auto_merge(box, pm.with_surface_reactions ? 0 : 1);
+        int rc = mcac_box_merge_in_launch(box, pm.with_surface_reactions ? 0 : 1);
         if (rc) return rc;
         if (pm.with_surface_reactions)
             for (auto *v : {&g_vol, &g_surf, &g_rsum, &g_rg, &g_rmax}) v->assign(n_ids, 0.0);

@@ -113,6 +113,12 @@ __device__ __forceinline__ void publish_merge(const MergeArgs &a, const mcac_mer
 // two waves.  Against one thread adding everything, on a dense 6000-sphere run:
 // k_step 26.6 -> 25.3 us, its grid form 144 -> 125 us, launches of several steps
 // 50.6 -> 42.8 us (mean); 99th percentile of a 2347-sphere run's 43.6 -> 36.9 us.
+// With spherical caps (kCaps) the rows hold the contacts with every sphere and
+// come first: each thread corrects its sphere's volume and surface, and the sums
+// run over the whole list.  In the step's launch, against the step (18.2 us) and
+// a merge launched when the host had seen the contact (23.3 us): 27.2 us, a run
+// of 3000 spheres 200 -> 132 ms.  Kernels of their own carry it: with the choice
+// made at run time, 500-sphere runs without caps took 3 % longer.
 constexpr int kRowWords = kSmallMerge / 32;
 struct MergeLds {
     double diffpos[3], refpos[3], r[3];
@@ -121,9 +127,13 @@ struct MergeLds {
     double vols[kSmallMerge], rads[kSmallMerge], surfs[kSmallMerge];
     double rlx[kSmallMerge], rly[kSmallMerge], rlz[kSmallMerge];
     double tx[kSmallMerge], ty[kSmallMerge], tz[kSmallMerge], t2[kSmallMerge];  // terms of the removed spheres; then arg
-    unsigned int row[kSmallMerge * kRowWords];  // contacts of sphere i with j > i
-    double over[kSmallMerge * 4];               // 2 c_ij in the reference's order
-    int wtot[kBlock / 64], contacts;
+    unsigned int row[kSmallMerge * kRowWords];  // contacts of sphere i with j > i (caps: with every j)
+    union {
+        double over[kSmallMerge * 4];  // 2 c_ij in the reference's order
+        unsigned char map[2][kSmallMerge][kOverlapSlots];  // caps, before: neighbour maps' orders and scratch
+    };
+    double cvol[kSmallMerge], csurf[kSmallMerge];  // caps: corrected
+    int wtot[kBlock / 64], long_row;
     double wmax[kBlock / 64];
     double V, svr2, arg, overlapping;
     mcac_merge_result res;
@@ -158,6 +168,78 @@ __device__ __forceinline__ double ordered_sum(double a, const double *t, int n) 
     return a;
 }
 
+// The contacts of sphere i with the spheres of word w above it (all: with every
+// sphere of the word but itself).
+__device__ __forceinline__ unsigned int merge_row_word(const MergeLds &u, int n, int i, int w, bool all) {
+    unsigned int bits = 0;
+    int j = 32 * w > i + 1 || all ? 32 * w : i + 1;
+    const int end = 32 * w + 32 < n ? 32 * w + 32 : n;
+    for (; j < end; ++j)
+        if (merge_touch(u, i, j)) bits |= 1u << (j & 31);
+    if (all && (i >> 5) == w) bits &= ~(1u << (i & 31));
+    return bits;
+}
+
+// Word w of sphere i's contacts, those with j > i.
+__device__ __forceinline__ unsigned int merge_row_above(const MergeLds &u, int i, int w) {
+    const unsigned int bits = u.row[i * kRowWords + w];
+    return w == (i >> 5) ? bits & (0xfffffffeu << (i & 31)) : bits;
+}
+
+// Spherical caps (aggregat.cpp:354-386): sphere t's corrected volume and surface
+// from its row, as caps_volumes_part below does from rows in memory.
+__device__ __forceinline__ void merge_small_caps(MergeLds &u, int t, int n, int n_k, double &vol, double &surf) {
+    const int words = (n + 31) >> 5;
+    int m = 0, prev = 0;
+    for (int w = 0; w < words; ++w) {
+        const unsigned int bits = u.row[t * kRowWords + w];
+        m += __popc(bits);
+        const int inside = n_k - 32 * w;  // spheres of this word in the keeper
+        prev += __popc(inside >= 32 ? bits : inside > 0 ? bits & ((1u << inside) - 1u) : 0u);
+    }
+    if (t >= n_k) prev = 0;
+    if (m > kOverlapSlots) {
+        u.long_row = 1;  // reported; the values are not used
+        m = kOverlapSlots;
+    }
+    unsigned char *const order = u.map[0][t];
+    int w = 0;
+    unsigned int bits = u.row[t * kRowWords];
+    auto next = [&]() {
+        while (bits == 0u) bits = u.row[t * kRowWords + ++w];
+        const int j = 32 * w + __ffs(static_cast<int>(bits)) - 1;
+        bits &= bits - 1u;
+        return j;
+    };
+    order_neighbours(prev, m, next, order, u.map[1][t]);
+    const double rt = u.rads[t], vt = u.vols[t], at = u.surfs[t];
+    vol = vt;
+    surf = at;
+    w = 0;
+    bits = u.row[t * kRowWords];
+    int lower = 0;  // neighbours before t
+    for (int v = 0; v <= t >> 5; ++v)
+        lower += __popc(v < t >> 5 ? u.row[t * kRowWords + v] : u.row[t * kRowWords + v] & ((1u << (t & 31)) - 1u));
+    if (lower > m) lower = m;
+    // the caps of the lower neighbours, ascending (this sphere is the second), then
+    // those of the higher ones in map order (this sphere is the first)
+    for (int y = -lower; y < m; ++y) {
+        const int j = y < 0 ? next() : static_cast<int>(order[y]);
+        if (y >= 0 && j <= t) continue;
+        const int i1 = y < 0 ? j : t, i2 = y < 0 ? t : j;
+        const double d0 = u.rlx[i1] - u.rlx[i2], d1 = u.rly[i1] - u.rly[i2], d2 = u.rlz[i1] - u.rlz[i2];
+        const double dist = __builtin_sqrt(d0 * d0 + d1 * d1 + d2 * d2);
+        double v1, s1, v2, s2;
+        caps_intersection(u.rads[i1], u.vols[i1], u.surfs[i1], u.rads[i2], u.vols[i2], u.surfs[i2], dist, &v1, &s1, &v2,
+                          &s2);
+        vol = vol - (y < 0 ? v2 : v1);
+        surf = surf - (y < 0 ? s2 : s1);
+    }
+    vol = smax(vol, 0.0);
+    surf = smax(surf, 0.0);
+}
+
+template <bool kCaps>
 __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeArgs &a, mcac_merge_result &res_out,
                                                   const double *mover_ref, MergeLds &u) {
     static_assert(kSmallMerge <= kBlock, "a thread per sphere");
@@ -173,7 +255,7 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
     double m4[4] = {0, 0, 0, 0}, o4[4] = {0, 0, 0, 0}, mrel[3] = {0, 0, 0}, orel[3] = {0, 0, 0};
     int sp = -1;
     if (t < n) sp = (t < a.n_k) ? b.members[a.start_k + t] : b.members[a.start_r + (t - a.n_k)];
-    if (t < 7) {
+    if (t < 7 && !kCaps) {
         const double *const sums[7] = {b.avol, b.asurf, b.csvx, b.csvy, b.csvz, b.csr, b.csvr2};
         const double *p = sums[0];
 #pragma unroll
@@ -181,6 +263,7 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
         c0 = p[k];
     }
     if (t == 0) {
+        u.long_row = 0;
         // the moving aggregate's contact sphere (ms) and the other's (os); "mine"
         // is the keeper's side (aggregat.cpp:496-509)
         const int ms = static_cast<int>(a.ms), os = static_cast<int>(a.os);
@@ -265,30 +348,50 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
         b.sx[sp] = rx + u.refpos[0];
         b.sy[sp] = ry + u.refpos[1];
         b.sz[sp] = rz + u.refpos[2];
-        u.tx[t] = rx * v;           // aggregat.cpp:439
-        u.ty[t] = ry * v;
-        u.tz[t] = rz * v;
-        u.t2[t] = v * (rad * rad);  // aggregat.cpp:477
     }
     if (t < n) {
         u.rlx[t] = rx;
         u.rly[t] = ry;
         u.rlz[t] = rz;
     }
-    lds_barrier();
     const int words = (n + 31) >> 5;
+    if constexpr (kCaps) {
+        lds_barrier();
+        for (int e = t; e < n * words; e += kBlock) {
+            const int w = e / n, i = e - w * n;
+            u.row[i * kRowWords + w] = merge_row_word(u, n, i, w, true);
+        }
+        lds_barrier();
+        if (t < n) {
+            double sf;
+            merge_small_caps(u, t, n, a.n_k, v, sf);
+            u.cvol[t] = v;
+            u.csurf[t] = sf;
+        }
+    }
+    if (t < n) {
+        u.tx[t] = rx * v;           // aggregat.cpp:439
+        u.ty[t] = ry * v;
+        u.tz[t] = rz * v;
+        u.t2[t] = v * (rad * rad);  // aggregat.cpp:477
+    }
+    lds_barrier();
     if (wave == 0) {
-        // the seven sums, continued from the keeper's (aggregat.cpp:388, 389, 439, 259, 477)
+        // the sums, continued from the keeper's (aggregat.cpp:388, 389, 439, 259, 477);
+        // the corrected volumes' from the start, with the spheres' own as the eighth
         double s = c0;
-        if (lane < 7) {
-            const double *const terms[7] = {u.vols, u.surfs, u.tx, u.ty, u.tz, u.rads, u.t2};
+        if (lane < (kCaps ? 8 : 7)) {
+            const double *const terms[8] = {kCaps ? u.cvol : u.vols, kCaps ? u.csurf : u.surfs, u.tx, u.ty, u.tz, u.rads,
+                                            u.t2, u.vols};
             const double *p = terms[0];
 #pragma unroll
-            for (int q = 1; q < 7; ++q) p = lane == q ? terms[q] : p;
-            s = ordered_sum(s, p + a.n_k, a.n_r);
+            for (int q = 1; q < 8; ++q) p = lane == q ? terms[q] : p;
+            const int first = kCaps ? 0 : a.n_k;
+            s = ordered_sum(s, p + first, n - first);
         }
         const double V = __shfl(s, 0, 64), S = __shfl(s, 1, 64), vx = __shfl(s, 2, 64), vy = __shfl(s, 3, 64),
-                     vz = __shfl(s, 4, 64), sr = __shfl(s, 5, 64), svr2 = __shfl(s, 6, 64);
+                     vz = __shfl(s, 4, 64), sr = __shfl(s, 5, 64), svr2 = __shfl(s, 6, 64),
+                     raw = __shfl(s, 7, 64);
         if (lane == 0) {
             const double rr[3] = {vx / V, vy / V, vz / V};  // aggregat.cpp:442
             const double com[3] = {periodic_position(u.refpos[0] + rr[0], a.L),
@@ -354,26 +457,21 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
             res.removed = a.rem;
             res.n = n;
             res.merged = 1;
-            res.status = (V <= 0 || S <= 0) ? MCAC_VOL_SURF_ERROR : 0;  // aggregat.cpp:427-429
+            res.status = (V <= 0 || S <= 0) ? MCAC_VOL_SURF_ERROR : (u.long_row ? MCAC_E_CAPACITY : 0);  // aggregat.cpp:427-429
             res.volume = V;
             res.surface = S;
-            res.sphere_volume = V;  // the sphere sum is the volume for method none
+            res.sphere_volume = kCaps ? raw : V;  // the sphere sum is the volume for method none
             res.radius_sum = sr;
             for (int l = 0; l < 3; ++l) {
                 res.com[l] = com[l];
                 res.rcm[l] = rr[l];
             }
         }
-    } else {
-        // contacts (aggregat.cpp:736-759) of sphere i with the spheres of word w after it
+    } else if (!kCaps) {
+        // contacts (aggregat.cpp:736-759)
         for (int e = t - 64; e < n * words; e += kBlock - 64) {
             const int w = e / n, i = e - w * n;
-            unsigned int bits = 0;
-            int j = 32 * w > i + 1 ? 32 * w : i + 1;
-            const int end = 32 * w + 32 < n ? 32 * w + 32 : n;
-            for (; j < end; ++j)
-                if (merge_touch(u, i, j)) bits |= 1u << (j & 31);
-            u.row[i * kRowWords + w] = bits;
+            u.row[i * kRowWords + w] = merge_row_word(u, n, i, w, false);
         }
     }
     lds_barrier();
@@ -386,7 +484,7 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
         const double dc = __builtin_sqrt(d0 * d0 + d1 * d1 + d2 * d2);
         far = smax(far, rad + dc);     // aggregat.cpp:462
         u.tx[t] = v * (dc * dc);       // aggregat.cpp:476
-        for (int w = t >> 5; w < words; ++w) mine += __popc(u.row[t * kRowWords + w]);
+        for (int w = t >> 5; w < words; ++w) mine += __popc(merge_row_above(u, t, w));
     }
     for (int off = 32; off > 0; off >>= 1) far = smax(far, __shfl_xor(far, off, 64));
     const int upto = wave_inclusive_scan(mine);
@@ -401,7 +499,7 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
     const bool listed = total <= kListed;
     if (listed && t < n)
         for (int w = t >> 5; w < words; ++w)
-            for (unsigned int bits = u.row[t * kRowWords + w]; bits != 0u; bits &= bits - 1u)
+            for (unsigned int bits = merge_row_above(u, t, w); bits != 0u; bits &= bits - 1u)
                 u.over[place++] = 2.0 * merge_overlap(u, t, 32 * w + __ffs(static_cast<int>(bits)) - 1);  // aggregat.cpp:755
     lds_barrier();
     if (t == 64) u.arg = ordered_sum(0., u.tx, n);
@@ -412,7 +510,7 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
         } else {  // spheres grown into very many neighbours
             for (int i = 0; i < n; ++i)
                 for (int w = i >> 5; w < words; ++w)
-                    for (unsigned int bits = u.row[i * kRowWords + w]; bits != 0u; bits &= bits - 1u)
+                    for (unsigned int bits = merge_row_above(u, i, w); bits != 0u; bits &= bits - 1u)
                         overlapping += 2.0 * merge_overlap(u, i, 32 * w + __ffs(static_cast<int>(bits)) - 1);
         }
         u.overlapping = overlapping;
@@ -440,10 +538,10 @@ __device__ __forceinline__ void merge_small_block(const DevBox &b, const MergeAr
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_merge_small(DevBox b, MergeArgs a) {
+template <bool kCaps> __global__ __launch_bounds__(kBlock) void k_merge_small(DevBox b, MergeArgs a) {
     __shared__ mcac_merge_result res;
     __shared__ MergeLds u;
-    merge_small_block(b, a, res, nullptr, u);
+    merge_small_block<kCaps>(b, a, res, nullptr, u);
     if (threadIdx.x == 0) publish_merge(a, res);
 }
 

@@ -640,8 +640,10 @@ __device__ __forceinline__ void scan_candidates(const DevBox &b, unsigned int F,
 // publishes later) and resets the search counters.  pick is read by thread 0
 // only.  Returns (in thread 0) whether the step closed the gate for the steps
 // queued behind it.
+template <bool kCaps>
 __device__ __forceinline__ bool apply_step(const DevBox &b, const SearchArgs &a, const StepPick &pick,
                                            const MoverSphere &m, bool publish, MergeLds &u) {
+    constexpr int kAutomerge = kCaps ? 2 : 1;  // the merges this kernel carries
     bool closed = false;
     const long long nsrc = a.n_mov;
     const int ssrc = a.start;
@@ -652,7 +654,7 @@ __device__ __forceinline__ bool apply_step(const DevBox &b, const SearchArgs &a,
     if (threadIdx.x == 0) {
         // every load of this thread comes before its stores (no reloads through global memory)
         const double closest = pick.dist;
-        if (pick.oagg >= 0 && closest <= a.lpm && a.automerge) {
+        if (pick.oagg >= 0 && closest <= a.lpm && a.automerge == kAutomerge) {
             const int o = static_cast<int>(pick.oagg);
             other_n = pick.on;
             other_start = b.astart[o];
@@ -753,7 +755,7 @@ __device__ __forceinline__ bool apply_step(const DevBox &b, const SearchArgs &a,
     }
     // merge in the same launch (AggregatList::merge, aggregat_list.cpp:367-410)
     // when the merged aggregate is small and its member segment fits
-    if (a.automerge && a.apply && a.translate_in_finish) {
+    if (a.automerge == kAutomerge && a.apply && a.translate_in_finish) {
         __shared__ MergeArgs s_ma;
         __shared__ int s_inline;
         if (threadIdx.x == 0) {
@@ -788,6 +790,7 @@ __device__ __forceinline__ bool apply_step(const DevBox &b, const SearchArgs &a,
                     m.start_r = start_r;
                     m.n_div = a.n_div;
                     m.cap_k = new_cap;
+                    m.volsurf = kCaps ? 1 : 0;
                     m.L = a.L;
                     s_ma = m;
                     s_inline = 1;
@@ -800,7 +803,7 @@ __device__ __forceinline__ bool apply_step(const DevBox &b, const SearchArgs &a,
         if (s_inline) {
             // the merge takes the mover's sphere positions from s_ref: its
             // loads do not wait for the placements above
-            merge_small_block(b, s_ma, srec.merge, s_ref, u);
+            merge_small_block<kCaps>(b, s_ma, srec.merge, s_ref, u);
             if (threadIdx.x == 0) srec.merged_inline = 1;  // thread 0 also copies the record
         }
     }
@@ -1144,7 +1147,7 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
         pick.tpairs = nsrc * T;
         pick.handover = 0;
     }
-    apply_step(b, a, pick, MoverSphere{0, -1, 0., 0., 0., 0., 0., 0., 0.}, true, lds.merge);
+    apply_step<false>(b, a, pick, MoverSphere{0, -1, 0., 0., 0., 0., 0., 0., 0.}, true, lds.merge);
 }
 
 __global__ __launch_bounds__(kBlock) void k_solve(DevBox b, SearchArgs a) {
@@ -1449,6 +1452,7 @@ __device__ __forceinline__ void hand_over(const DevBox &b, const SearchArgs &a, 
 // writes its body and the caller publishes the sequence number later, after a
 // system-scope fence).  Returns (in thread 0) whether the step closed the gate.
 // role (optional, LDS, set by thread 0): as search_step's result.
+template <bool kCaps>
 __device__ __forceinline__ bool step_body(const DevBox &b, const SearchArgs &a, unsigned vb, unsigned vg,
                                           bool gate_open, const CellTable *ct, bool publish, int *role = nullptr,
                                           const StepPrefetch *pre = nullptr) {
@@ -1463,7 +1467,7 @@ __device__ __forceinline__ bool step_body(const DevBox &b, const SearchArgs &a, 
         if (threadIdx.x == 0) hand_over(b, a, publish);
         return a.gated != 0;
     }
-    return apply_step(b, a, pick, mover, publish, lds.merge);
+    return apply_step<kCaps>(b, a, pick, mover, publish, lds.merge);
 }
 
 // Kernel arguments read where the launch put them, in constant memory, when
@@ -1479,9 +1483,9 @@ struct StepOne {
     DevBox b;
     SearchArgs a;
 };
-__global__ __launch_bounds__(kBlock) void k_step(StepOne) {
+template <bool kCaps> __global__ __launch_bounds__(kBlock) void k_step(StepOne) {
     const StepOne &k = kernel_arguments<StepOne>();
-    step_body(k.b, k.a, blockIdx.x, gridDim.x, false, nullptr, true);
+    step_body<kCaps>(k.b, k.a, blockIdx.x, gridDim.x, false, nullptr, true);
 }
 
 // Several consecutive queued steps of a box in one launch (at most kMaxSteps).
@@ -1536,7 +1540,7 @@ __device__ __forceinline__ void set_moved(Moved &mv, int q, int src, const Args 
 
 // Carries out the nj searched steps in u.args / u.picks in order up to the first
 // contact or hand-over and publishes their records (whole block).
-__device__ __forceinline__ void commit_steps(const DevBox &b, StepsLds &u, int nj) {
+template <bool kCaps> __device__ __forceinline__ void commit_steps(const DevBox &b, StepsLds &u, int nj) {
     SearchState *s = b.ss;
     int f = 0;
     while (f < nj && !u.picks[f].handover && !(u.picks[f].dist <= u.args[f].lpm)) ++f;
@@ -1617,13 +1621,13 @@ __device__ __forceinline__ void commit_steps(const DevBox &b, StepsLds &u, int n
         return;
     }
     const MoverSphere mover = load_mover_sphere(b, u.args[f]);
-    apply_step(b, u.args[f], u.picks[f], mover, true, u.lds.merge);
+    apply_step<kCaps>(b, u.args[f], u.picks[f], mover, true, u.lds.merge);
 }
 
 // The rest of a step's launch once its arguments are known: args(p) gives those
 // of step p <= q, fetch(p) loads all of step p's into LDS (for p < nj, when
 // every step has finished its search).
-template <class Args, class Fetch>
+template <bool kCaps, class Args, class Fetch>
 __device__ __forceinline__ void run_steps(const DevBox &b, StepsLds &u, const SearchArgs &a, int q, int nj,
                                           int nd, unsigned vb, unsigned vg, const Args &args, const Fetch &fetch) {
     set_moved(u.mv, q, a.src, args);
@@ -1651,7 +1655,7 @@ __device__ __forceinline__ void run_steps(const DevBox &b, StepsLds &u, const Se
     }
     fetch();
     __syncthreads();
-    commit_steps(b, u, nj);
+    commit_steps<kCaps>(b, u, nj);
 }
 
 constexpr int kArgWords = static_cast<int>(sizeof(SearchArgs) / sizeof(unsigned long long));
@@ -1665,14 +1669,14 @@ struct StepSet {
 };
 
 // Steps of one box, blockIdx.y the step and blockIdx.x its block.
-__global__ __launch_bounds__(kBlock) void k_steps(StepSet) {
+template <bool kCaps> __global__ __launch_bounds__(kBlock) void k_steps(StepSet) {
     __shared__ StepsLds u;
     const StepSet &set = kernel_arguments<StepSet>();
     const int q = static_cast<int>(blockIdx.y);
     const SearchArgs &a = set.a[q];
     const unsigned vg = static_cast<unsigned>(a.vg);
     if (blockIdx.x >= vg) return;
-    run_steps(set.b, u, a, q, set.nj, a.run_dirty, blockIdx.x, vg,
+    run_steps<kCaps>(set.b, u, a, q, set.nj, a.run_dirty, blockIdx.x, vg,
               [&](int p) -> const SearchArgs & { return set.a[p]; },
               [&] {
                   for (int i = threadIdx.x; i < set.nj * kArgWords; i += blockDim.x)
@@ -1724,7 +1728,7 @@ __global__ __launch_bounds__(kBlock) void k_steps_group(const BoxRun *runs) {
             reinterpret_cast<unsigned long long *>(&b.sargs[q])[i] =
                 reinterpret_cast<const unsigned long long *>(&u.args[q])[i];
     const SearchArgs &a = u.args[q];
-    run_steps(b, u, a, q, nj, a.run_dirty, 0u, 1u, [&](int p) -> const SearchArgs & { return u.args[p]; },
+    run_steps<false>(b, u, a, q, nj, a.run_dirty, 0u, 1u, [&](int p) -> const SearchArgs & { return u.args[p]; },
               [&] {
                   if (nj > 1)
                       for (int i = threadIdx.x; i < nj * kArgWords; i += blockDim.x)
@@ -1877,7 +1881,7 @@ __global__ __launch_bounds__(kBlock) void k_step_engine(DevBox b, const EngineJo
         const CellTable *ct = job.cells.n > 0 ? &job.cells : nullptr;
         int role = 0;
         __shared__ int s_role;
-        const bool closed = step_body(b, a, blockIdx.x, vg, true, ct, false, &s_role, &pre);
+        const bool closed = step_body<false>(b, a, blockIdx.x, vg, true, ct, false, &s_role, &pre);
         __syncthreads();
         role = s_role;
         if (role == 2 && threadIdx.x == 0) {

@@ -88,7 +88,7 @@ struct mcac_box {
     bool gate_closed = false;        // a consumed queued step found a contact; not released yet
     unsigned long long released = 0; // gate values the steps enqueued from now on ignore
     unsigned long long last_gate = 0;  // seq of the last consumed step that closed the gate
-    int automerge = 0;               // queued moves merge in the same launch on contact
+    int automerge = 0;               // queued moves merge in the same launch on contact (SearchArgs::automerge)
     int fused_merge = 1;             // overlap-correction merges of <= kFusedMerge spheres in one launch
     bool inline_pending = false;     // a contact merged in its launch; mcac_merge not called yet
     StepRecord inline_rec{};
@@ -536,6 +536,9 @@ bool fits_one_launch(const mcac_box *b, int n_mov) {
     return n_mov <= kStepMover && (worst <= kStepWorst || (n_mov <= kStepNarrow && worst <= kStepNarrowWorst));
 }
 
+// The one-launch form of a box's steps, with the merge that it carries.
+auto step_kernel(const mcac_box *b) { return b->automerge == 2 ? k_step<true> : k_step<false>; }
+
 // A step that one block can take whole: the one-launch form (small mover, few
 // sphere pairs possible), the mover moved by the finishing block, not timed.
 bool one_block_step(const mcac_box *b, int n_mov, bool timed) {
@@ -658,7 +661,7 @@ int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, do
     a.seq = seq;
     a.gated = gated;
     a.released = b->released;
-    a.automerge = (b->automerge && gated && apply) ? 1 : 0;
+    a.automerge = (gated && apply) ? b->automerge : 0;
     // FP32 broad phase only where the minimum image decides (sweep + radii < 0.4 L)
     a.prec = (b->p.precision > 0 && a.known && lpm + a.srmax + maxradius < 0.4 * b->p.box_length)
                  ? static_cast<int>(std::min<int32_t>(b->p.precision, 2))
@@ -724,8 +727,9 @@ int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, do
         if (rc) return rc;
         engine_post(b, &a, &ct, std::min(grid, b->eng_blocks));
     } else if (fused) {
-        if (timed) hipExtLaunchKernelGGL(k_step, dim3(grid), dim3(kBlock), 0, bstream(b), ev[0], ev[1], 0, StepOne{b->d, a});
-        else hipLaunchKernelGGL(k_step, dim3(grid), dim3(kBlock), 0, bstream(b), StepOne{b->d, a});
+        const auto step = step_kernel(b);
+        if (timed) hipExtLaunchKernelGGL(step, dim3(grid), dim3(kBlock), 0, bstream(b), ev[0], ev[1], 0, StepOne{b->d, a});
+        else hipLaunchKernelGGL(step, dim3(grid), dim3(kBlock), 0, bstream(b), StepOne{b->d, a});
     } else if (b->grid_solve) {
         const int g2 = grid_form_blocks(b, grid);
         if (timed) hipExtLaunchKernelGGL(k_step_grid, dim3(g2), dim3(kBlock), 0, bstream(b), ev[0], ev[1], 0, b->d, a);
@@ -1472,7 +1476,9 @@ int mcac_merge(mcac_box *b, const mcac_contact *c, mcac_merge_result *out) {
     const int n = nk + nr;
     if (b->timing) HIP_TRY(hipEventRecord(b->ev[0], bstream(b)));
     const bool fused = b->fused_merge && a.volsurf != 0 && n <= kFusedMerge;
-    if (fused && a.volsurf != 2) {
+    if (fused && a.volsurf == 1 && n <= kSmallMerge) {
+        hipLaunchKernelGGL(k_merge_small<true>, dim3(1), dim3(kBlock), 0, bstream(b), b->d, a);
+    } else if (fused && a.volsurf != 2) {
         hipLaunchKernelGGL(k_merge_fused, dim3(1), dim3(kBlock), 0, bstream(b), b->d, a);
     } else if (a.volsurf == 1 || a.volsurf == 3) {
         // spherical caps or arvo: the two-way contact rows first, then the
@@ -1539,7 +1545,7 @@ int mcac_merge(mcac_box *b, const mcac_contact *c, mcac_merge_result *out) {
             }
         }
     } else if (n <= kSmallMerge) {
-        hipLaunchKernelGGL(k_merge_small, dim3(1), dim3(kBlock), 0, bstream(b), b->d, a);
+        hipLaunchKernelGGL(k_merge_small<false>, dim3(1), dim3(kBlock), 0, bstream(b), b->d, a);
     } else {
         const int nb = std::min(4096, (n + kBlock - 1) / kBlock);
         hipLaunchKernelGGL(k_merge_prep, dim3(1), dim3(64), 0, bstream(b), b->d, a);
@@ -1685,13 +1691,13 @@ int run_flush(Enqueue &e) {
             vg = std::max(vg, r.set.a[q].vg);
         }
         if (n == 1) {
-            hipLaunchKernelGGL(k_step, dim3(static_cast<unsigned>(vg)), dim3(kBlock), 0, bstream(b),
+            hipLaunchKernelGGL(step_kernel(b), dim3(static_cast<unsigned>(vg)), dim3(kBlock), 0, bstream(b),
                                StepOne{b->d, r.set.a[0]});
         } else {
             r.set.b = b->d;
             r.set.nj = n;
-            hipLaunchKernelGGL(k_steps, dim3(static_cast<unsigned>(vg), static_cast<unsigned>(n)), dim3(kBlock), 0,
-                               bstream(b), r.set);
+            hipLaunchKernelGGL(b->automerge == 2 ? k_steps<true> : k_steps<false>,
+                               dim3(static_cast<unsigned>(vg), static_cast<unsigned>(n)), dim3(kBlock), 0, bstream(b), r.set);
         }
         HIP_TRY(hipGetLastError());
         if (g) {
@@ -1862,8 +1868,15 @@ int mcac_release(mcac_box *b) {
 
 int mcac_box_set_auto_merge(mcac_box *b, int enable) {
     if (!b || b->inflight) return MCAC_E_ARGUMENT;
-    b->automerge = (enable && b->p.volsurf == 0) ? 1 : 0;  // caps merges run their own kernel sequence
+    b->automerge = (enable && b->p.volsurf == 0) ? 1 : 0;
     return 0;
+}
+
+int mcac_box_merge_in_launch(mcac_box *b, int enable) {
+    const int rc = mcac_box_set_auto_merge(b, enable);
+    // alphas needs the host's powers, and an arvo ball more registers than a step has to spare
+    if (!rc && enable && b->p.volsurf == 1 && b->fused_merge) b->automerge = 2;
+    return rc;
 }
 
 int mcac_arvo_part(int k, const double *x, const double *y, const double *z, const double *r, double out[2]) {

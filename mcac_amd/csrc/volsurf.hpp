@@ -12,6 +12,8 @@
 #pragma once
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "device_math.hpp"
 
 namespace mcac_dev {
@@ -34,10 +36,11 @@ __host__ __device__ inline unsigned umap_next_bkt(unsigned n) {
 // Inserts key at the front of its bucket's run in list l of len keys (a new
 // bucket goes to the front of the list): _Hashtable::_M_insert_bucket_begin,
 // also the order _M_rehash_aux rebuilds the list in.
-__host__ __device__ inline void umap_link(int64_t *l, int len, int64_t key, unsigned nb) {
-    const int64_t b = key % static_cast<int64_t>(nb);
+template <class K> __host__ __device__ inline void umap_link(K *l, int len, K key, unsigned nb) {
+    using Mod = std::conditional_t<(sizeof(K) < 4), unsigned, int64_t>;
+    const Mod n = static_cast<Mod>(nb), b = static_cast<Mod>(key) % n;
     int p = 0;
-    while (p < len && l[p] % static_cast<int64_t>(nb) != b) ++p;
+    while (p < len && static_cast<Mod>(l[p]) % n != b) ++p;
     if (p == len) p = 0;
     for (int q = len; q > p; --q) l[q] = l[q - 1];
     l[p] = key;
@@ -50,11 +53,11 @@ __host__ __device__ inline void umap_link(int64_t *l, int len, int64_t key, unsi
 // libstdc++ with the identity hash and max load factor 1: reserve sets
 // next_bkt(max(1, prev)) buckets; inserting the (c+1)-th key into c keys and
 // nb buckets with c + 1 > nb first rehashes to next_bkt(max(c + 2, 2 nb)).
-// out receives the m keys; returns 0, or -1 when m > kMapKeys.
-__host__ __device__ inline int neighbour_order(int prev, const int64_t *keys, int m, int64_t *out) {
-    if (m > kMapKeys || m < 0) return -1;
+// out receives the m keys (m <= kMapKeys), tmp is scratch of the same length;
+// next() gives the keys one after the other.
+template <class K, class Next>
+__host__ __device__ inline void order_neighbours(int prev, int m, Next next, K *out, K *tmp) {
     unsigned nb = umap_next_bkt(prev > 1 ? static_cast<unsigned>(prev) : 1u);
-    int64_t tmp[kMapKeys];
     for (int c = 0; c < m; ++c) {
         if (static_cast<unsigned>(c + 1) > nb) {
             const unsigned want = static_cast<unsigned>(c + 2) > 2 * nb ? static_cast<unsigned>(c + 2) : 2 * nb;
@@ -63,8 +66,14 @@ __host__ __device__ inline int neighbour_order(int prev, const int64_t *keys, in
             for (int q = 0; q < c; ++q) umap_link(out, q, tmp[q], nb2);
             nb = nb2;
         }
-        umap_link(out, c, keys[c], nb);
+        umap_link(out, c, static_cast<K>(next()), nb);
     }
+}
+// The same from an array; returns 0, or -1 when m > kMapKeys.
+__host__ __device__ inline int neighbour_order(int prev, const int64_t *keys, int m, int64_t *out) {
+    if (m > kMapKeys || m < 0) return -1;
+    int64_t tmp[kMapKeys];
+    order_neighbours(prev, m, [&]() { return *keys++; }, out, tmp);
     return 0;
 }
 
