@@ -6,10 +6,10 @@
 //                                (:321-390, sphere sums), compute_mass_center
 //                                (:431-452), compute_max_radius (:453-464),
 //                                compute_giration_radius (:465-483)
-// One wave per live aggregate walks its member list in 64-sphere chunks; every
-// lane adds the chunk's terms in list order (broadcast by shuffles), so each
-// sum is the reference's sequential FP64 sum.  The merge caches (sums the next
-// merge continues) are rewritten from the grown spheres.
+// A wave, or eight lanes of one, walk an aggregate's member list in chunks of as
+// many spheres; every lane adds the chunk's terms in list order (broadcast by
+// shuffles), so each sum is the reference's sequential FP64 sum.  The merge
+// caches (sums the next merge continues) are rewritten from the grown spheres.
 #pragma once
 #include "kernels_common.hpp"
 
@@ -18,38 +18,42 @@ namespace mcac_dev {
 constexpr double kVolumeFactorD = 4 * kPi / 3;  // constants.hpp:114
 constexpr double kSurfaceFactorD = 4 * kPi;     // constants.hpp:115
 
-// ids[0..n_ids) may hold dead ids (count 0): skipped.  Outputs by position in
-// ids: volume, surface, list-order radius sum, Rg and rmax of each live aggregate.
-// The contact search's copies of CoM and rmax follow in place: a dirty
-// aggregate's dirty-list entry, or the packed cell entry of one still in the
-// cell it was built in; *o_left counts the aggregates whose growth took them
-// out of their built cell (their entries are stale: the cell list must be
-// rebuilt before the next search).
-// With grow = 0 the spheres keep their radii, volumes and surfaces (the update
-// alone); o_flag[wave] gets 1 when a sphere of the aggregate is at or below
-// rp_min after growing (oxidation removes it).
-__global__ __launch_bounds__(kBlock) void k_grow_update(DevBox b, const int *ids, int n_ids, double dr, int grow,
-                                                       double rp_min, double L, int n_div, double *o_vol,
-                                                       double *o_surf, double *o_rsum, double *o_rg, double *o_rmax,
-                                                       int *o_left, int *o_flag) {
-    const int wave = static_cast<int>((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const int lane = static_cast<int>(threadIdx.x & 63);
-    if (wave >= n_ids) return;
-    const int id = ids[wave];
-    const int n = b.acount[id];
-    if (n <= 0) return;
-    const int st = b.astart[id];
+struct GrowOut {
+    double *vol, *surf, *rsum, *rg, *rmax;  // by position in ids
+    int *flag;
+};
+constexpr int kGrowSmall = 1, kGrowSplit = 2, kGrowLeft = 4;
+
+// One aggregate by kLanes lanes (aligned, all active): id at position at, with n > 0
+// spheres in the segment st.  The contact search's copies of CoM and rmax follow
+// in place: a dirty aggregate's dirty-list entry, or the packed cell entry of one
+// still in the cell it was built in; kGrowLeft tells that its growth took it out of
+// its built cell (the entry is stale: the cell list must be rebuilt before the
+// next search).  With grow = 0 the spheres keep their radii, volumes and surfaces
+// (the update alone); kGrowSmall tells that a sphere of the aggregate is at or
+// below rp_min after growing (oxidation removes it).
+template <int kLanes>
+__device__ __forceinline__ void grow_one(const DevBox &b, int at, int id, int n, int st, double dr, int grow,
+                                         double rp_min, double L, int n_div, const GrowOut &o) {
+    const int lane = static_cast<int>(threadIdx.x & (kLanes - 1));
     // grow, then volume, surface, sum of vol * relative position, radius sum
     // and sum of vol * r^2 in list order
     double V = 0.0, S = 0.0, vx = 0.0, vy = 0.0, vz = 0.0, rs = 0.0, brg = 0.0;
-    int small = 0;
-    for (int c0 = 0; c0 < n; c0 += 64) {
+    double r = 0.0, vol = 0.0, rx = 0.0, ry = 0.0, rz = 0.0;
+    int small = 0, s0 = 0;
+    for (int c0 = 0; c0 < n; c0 += kLanes) {
         const int i = c0 + lane;
-        double r = 0.0, vol = 0.0, surf = 0.0, rx = 0.0, ry = 0.0, rz = 0.0;
+        double surf = 0.0;
+        r = vol = rx = ry = rz = 0.0;
         if (i < n) {
             const int s = b.members[st + i];
+            if (c0 == 0) s0 = s;
+            r = b.sr[s];
+            rx = b.srx[s];
+            ry = b.sry[s];
+            rz = b.srz[s];
             if (grow) {
-                r = b.sr[s] + dr;  // PhysicalModel::grow: r + u_sg * dt, dr = u_sg * dt
+                r = r + dr;  // PhysicalModel::grow: r + u_sg * dt, dr = u_sg * dt
                 const double r2 = r * r;
                 const double r3 = r2 * r;
                 vol = kVolumeFactorD * r3;
@@ -58,102 +62,141 @@ __global__ __launch_bounds__(kBlock) void k_grow_update(DevBox b, const int *ids
                 b.svol[s] = vol;
                 b.ssurf[s] = surf;
             } else {
-                r = b.sr[s];
                 vol = b.svol[s];
                 surf = b.ssurf[s];
             }
             small |= (r <= rp_min) ? 1 : 0;
-            rx = b.srx[s];
-            ry = b.sry[s];
-            rz = b.srz[s];
         }
-        const int m = (n - c0 < 64) ? n - c0 : 64;
+        const double tx = rx * vol, ty = ry * vol, tz = rz * vol, t2 = vol * (r * r);
+        const int m = (n - c0 < kLanes) ? n - c0 : kLanes;
         for (int j = 0; j < m; ++j) {
-            const double vj = __shfl(vol, j, 64), rj = __shfl(r, j, 64);
-            V = V + vj;
-            S = S + __shfl(surf, j, 64);
-            vx = vx + __shfl(rx, j, 64) * vj;
-            vy = vy + __shfl(ry, j, 64) * vj;
-            vz = vz + __shfl(rz, j, 64) * vj;
-            rs = rs + rj;
-            brg = brg + vj * (rj * rj);
+            V = V + __shfl(vol, j, kLanes);
+            S = S + __shfl(surf, j, kLanes);
+            vx = vx + __shfl(tx, j, kLanes);
+            vy = vy + __shfl(ty, j, kLanes);
+            vz = vz + __shfl(tz, j, kLanes);
+            rs = rs + __shfl(r, j, kLanes);
+            brg = brg + __shfl(t2, j, kLanes);
         }
     }
     const double cx = vx / V, cy = vy / V, cz = vz / V;  // r /= agregat_volume
     // distances to the centre of mass, rmax and sum of vol * dc^2 in list order
     double rmax = 0.0, arg = 0.0;
-    for (int c0 = 0; c0 < n; c0 += 64) {
+    for (int c0 = 0; c0 < n; c0 += kLanes) {
         const int i = c0 + lane;
-        double dc = 0.0, r = 0.0, vol = 0.0;
-        if (i < n) {
-            const int s = b.members[st + i];
-            const double dx = b.srx[s] - cx, dy = b.sry[s] - cy, dz = b.srz[s] - cz;
-            dc = __builtin_sqrt(dx * dx + dy * dy + dz * dz);
-            r = b.sr[s];  // written above by this lane
-            vol = b.svol[s];
+        if (n > kLanes) {  // else still in registers
+            r = vol = rx = ry = rz = 0.0;
+            if (i < n) {
+                const int s = b.members[st + i];
+                rx = b.srx[s];
+                ry = b.sry[s];
+                rz = b.srz[s];
+                r = b.sr[s];  // written above by this lane
+                vol = b.svol[s];
+            }
         }
-        const int m = (n - c0 < 64) ? n - c0 : 64;
+        const double dx = rx - cx, dy = ry - cy, dz = rz - cz;
+        const double dc = __builtin_sqrt(dx * dx + dy * dy + dz * dz);
+        const double far = r + dc, term = vol * (dc * dc);
+        const int m = (n - c0 < kLanes) ? n - c0 : kLanes;
         for (int j = 0; j < m; ++j) {
-            const double dj = __shfl(dc, j, 64);
-            rmax = smax(rmax, __shfl(r, j, 64) + dj);
-            arg = arg + __shfl(vol, j, 64) * (dj * dj);
+            rmax = smax(rmax, __shfl(far, j, kLanes));
+            arg = arg + __shfl(term, j, kLanes);
         }
     }
     const double rg = __builtin_sqrt(__builtin_fabs((arg + 3. / 5. * brg) / V));
-    if (lane == 0) {
-        // set_position(sphere 0 + r_cm) wraps into the box (aggregat.cpp:109-118)
-        const int s0 = b.members[st];
-        const double px = periodic_position(b.sx[s0] + cx, L);
-        const double py = periodic_position(b.sy[s0] + cy, L);
-        const double pz = periodic_position(b.sz[s0] + cz, L);
-        b.avol[id] = V;
-        b.asurf[id] = S;
-        b.csvx[id] = vx;
-        b.csvy[id] = vy;
-        b.csvz[id] = vz;
-        b.csr[id] = rs;
-        b.csvr2[id] = brg;
-        b.arx[id] = cx;
-        b.ary[id] = cy;
-        b.arz[id] = cz;
-        b.ax[id] = px;
-        b.ay[id] = py;
-        b.az[id] = pz;
-        const int cell = ref_cell(px, py, pz, n_div, L);
-        const int built = b.acell[id];
-        b.acell[id] = cell;
-        b.armax[id] = rmax;
-        if (b.dirty[id]) {
-            set_dirty_entry(b, b.dslot[id], px, py, pz, rmax, cell);
-        } else {
-            const int cs = b.cslot[id];
-            if (cs >= 0 && cell == built) {
-                b.cpx[cs] = px;
-                b.cpy[cs] = py;
-                b.cpz[cs] = pz;
-                b.cpr[cs] = rmax;
-                b.cf[cs] = make_float4(static_cast<float>(px), static_cast<float>(py), static_cast<float>(pz),
-                                       static_cast<float>(rmax));
-            } else {
-                atomicAdd(o_left, 1);
-            }
-        }
-        b.arg[id] = rg;
-        o_vol[wave] = V;
-        o_surf[wave] = S;
-        o_rsum[wave] = rs;
-        o_rg[wave] = rg;
-        o_rmax[wave] = rmax;
+    int flag = 0;
+    {
+        const int base = static_cast<int>(threadIdx.x & 63) & ~(kLanes - 1);
+        const unsigned long long mine = kLanes == 64 ? ~0ull : ((1ull << (kLanes & 63)) - 1ull) << base;
+        if (__ballot(small) & mine) flag = kGrowSmall;
     }
-    const bool any_small = __any(small);
-    if (lane == 0) o_flag[wave] = any_small ? 1 : 0;
+    if (lane != 0) return;
+    // set_position(sphere 0 + r_cm) wraps into the box (aggregat.cpp:109-118)
+    const double px = periodic_position(b.sx[s0] + cx, L);
+    const double py = periodic_position(b.sy[s0] + cy, L);
+    const double pz = periodic_position(b.sz[s0] + cz, L);
+    b.avol[id] = V;
+    b.asurf[id] = S;
+    b.csvx[id] = vx;
+    b.csvy[id] = vy;
+    b.csvz[id] = vz;
+    b.csr[id] = rs;
+    b.csvr2[id] = brg;
+    b.arx[id] = cx;
+    b.ary[id] = cy;
+    b.arz[id] = cz;
+    b.ax[id] = px;
+    b.ay[id] = py;
+    b.az[id] = pz;
+    const int cell = ref_cell(px, py, pz, n_div, L);
+    const int built = b.acell[id];
+    b.acell[id] = cell;
+    b.armax[id] = rmax;
+    if (b.dirty[id]) {
+        set_dirty_entry(b, b.dslot[id], px, py, pz, rmax, cell);
+    } else {
+        const int cs = b.cslot[id];
+        if (cs >= 0 && cell == built) {
+            b.cpx[cs] = px;
+            b.cpy[cs] = py;
+            b.cpz[cs] = pz;
+            b.cpr[cs] = rmax;
+            b.cf[cs] = make_float4(static_cast<float>(px), static_cast<float>(py), static_cast<float>(pz),
+                                   static_cast<float>(rmax));
+        } else {
+            flag |= kGrowLeft;
+        }
+    }
+    b.arg[id] = rg;
+    o.vol[at] = V;
+    o.surf[at] = S;
+    o.rsum[at] = rs;
+    o.rg[at] = rg;
+    o.rmax[at] = rmax;
+    o.flag[at] = flag;
+}
+
+// ids[0..n_ids) may hold dead ids (count 0): their outputs are not written.
+// kLanes lanes an aggregate.  What bounds it is the chain of loads from an id to its
+// spheres, so the more aggregates are under way the better: a wave for each while
+// the chip holds them all at once (kGrowPacked), eight lanes beyond that if the
+// aggregates are small (kGrowPackedMean spheres on average); those of more than
+// kGrowWide spheres are left to the whole wave afterwards (else one large
+// aggregate would end long after the rest).  A call's time, a wave each -> eight
+// lanes: 100000 aggregates of 8 spheres 454 -> 307 us, 30000 of 16 224 -> 141,
+// 10000 of 16 139 -> 139, 25000 of 32 269 -> 277, 9000 of 32 138 -> 281.
+constexpr int kGrowPacked = 8192;  // aggregates: 256 compute units with 32 waves each
+constexpr int kGrowPackedMean = 16;
+constexpr int kGrowWide = 32;
+template <int kLanes>
+__global__ __launch_bounds__(kBlock) void k_grow_update(DevBox b, const int *ids, int n_ids, double dr, int grow,
+                                                       double rp_min, double L, int n_div, GrowOut o) {
+    const int at = static_cast<int>((blockIdx.x * blockDim.x + threadIdx.x) / kLanes);
+    int id = 0, n = 0, st = 0;
+    if (at < n_ids) {
+        id = ids[at];
+        n = b.acount[id];
+        st = b.astart[id];
+    }
+    if constexpr (kLanes == 64) {
+        if (n > 0) grow_one<64>(b, at, id, n, st, dr, grow, rp_min, L, n_div, o);
+    } else {
+        if (n > 0 && n <= kGrowWide) grow_one<kLanes>(b, at, id, n, st, dr, grow, rp_min, L, n_div, o);
+        unsigned long long wide = __ballot(n > kGrowWide && (threadIdx.x & (kLanes - 1)) == 0);
+        for (; wide != 0ull; wide &= wide - 1ull) {
+            const int l = __ffsll(static_cast<long long>(wide)) - 1;
+            grow_one<64>(b, __shfl(at, l, 64), __shfl(id, l, 64), __shfl(n, l, 64), __shfl(st, l, 64), dr, grow, rp_min,
+                         L, n_div, o);
+        }
+    }
 }
 
 // Aggregate::split's question (aggregat.cpp:553-584) for each aggregate of
 // ids: are its spheres one connected set under the contact test
 // (sphere_distances.cpp:81-90)?  One wave per aggregate of at most 64
 // spheres: lane i builds sphere i's contact bits, and the set reached from
-// sphere 0 grows by wave-wide ORs until it stops.  o_flag[wave] |= 2 when the
+// sphere 0 grows by wave-wide ORs until it stops.  o_flag[wave] |= kGrowSplit when the
 // aggregate falls apart, or when it has more than 64 spheres (left to the host).
 __global__ __launch_bounds__(kBlock) void k_connected(DevBox b, const int *ids, int n_ids, double L, int *o_flag) {
     const int wave = static_cast<int>((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
@@ -163,7 +206,7 @@ __global__ __launch_bounds__(kBlock) void k_connected(DevBox b, const int *ids, 
     const int n = b.acount[id];
     if (n <= 1) return;
     if (n > 64) {
-        if (lane == 0) o_flag[wave] |= 2;
+        if (lane == 0) o_flag[wave] |= kGrowSplit;
         return;
     }
     const int st = b.astart[id];
@@ -193,7 +236,7 @@ __global__ __launch_bounds__(kBlock) void k_connected(DevBox b, const int *ids, 
         if (next == reached) break;
         reached = next;
     }
-    if (lane == 0 && (reached & all) != all) o_flag[wave] |= 2;
+    if (lane == 0 && (reached & all) != all) o_flag[wave] |= kGrowSplit;
 }
 
 }  // namespace mcac_dev

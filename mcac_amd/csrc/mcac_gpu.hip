@@ -2028,13 +2028,15 @@ int mcac_box_grow_ids(mcac_box *b, const int64_t *ids, int64_t n_ids, double dr,
         return MCAC_E_ARGUMENT;
     const int64_t n = ids ? n_ids : static_cast<int64_t>(b->alive_ids.size());
     if (n == 0) return 0;
+    int64_t spheres = ids ? 0 : b->n_spheres;
     if (ids)
-        for (int64_t i = 0; i < n; ++i)
+        for (int64_t i = 0; i < n; ++i) {
             if (ids[i] < 0 || ids[i] >= b->n_aggs || b->count[static_cast<size_t>(ids[i])] <= 0) return MCAC_E_ARGUMENT;
-    // layout: five outputs per aggregate (doubles), its flags, the ids (ints), the
-    // count of aggregates that left their cell
+            spheres += b->count[static_cast<size_t>(ids[i])];
+        }
+    // layout: five outputs per aggregate (doubles), its flags, the ids (ints)
     const size_t N = static_cast<size_t>(n);
-    auto bytes_for = [](size_t m) { return 5 * m * sizeof(double) + 2 * m * sizeof(int) + sizeof(double); };
+    auto bytes_for = [](size_t m) { return 5 * m * sizeof(double) + 2 * m * sizeof(int); };
     if (b->grow_cap < n) {
         if (b->h_grow) HIP_TRY(hipHostFree(b->h_grow));
         if (b->d_grow) HIP_TRY(hipFree(b->d_grow));
@@ -2048,7 +2050,6 @@ int mcac_box_grow_ids(mcac_box *b, const int64_t *ids, int64_t n_ids, double dr,
     double *g = b->d_grow;
     int *d_flag = reinterpret_cast<int *>(g + 5 * N);
     int *d_ids = d_flag + N;
-    int *left = d_ids + N;
     hipStream_t st = bstream(b);
     const int *idp = b->d.alive;
     if (ids) {
@@ -2057,19 +2058,19 @@ int mcac_box_grow_ids(mcac_box *b, const int64_t *ids, int64_t n_ids, double dr,
         HIP_TRY(hipMemcpyAsync(d_ids, h_ids, N * sizeof(int), hipMemcpyHostToDevice, st));
         idp = d_ids;
     }
-    HIP_TRY(hipMemsetAsync(left, 0, sizeof(int), st));
+    const GrowOut out{g, g + N, g + 2 * N, g + 3 * N, g + 4 * N, d_flag};
+    const int lanes = n > kGrowPacked && spheres <= kGrowPackedMean * n ? 8 : 64;
+    hipLaunchKernelGGL(lanes == 8 ? k_grow_update<8> : k_grow_update<64>,
+                       dim3(static_cast<unsigned>((n * lanes + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, b->d, idp,
+                       static_cast<int>(n), dr, grow ? 1 : 0, rp_min, b->p.box_length, static_cast<int>(b->p.n_div), out);
     const unsigned blocks = static_cast<unsigned>((n * 64 + kBlock - 1) / kBlock);
-    hipLaunchKernelGGL(k_grow_update, dim3(blocks), dim3(kBlock), 0, st, b->d, idp, static_cast<int>(n), dr,
-                       grow ? 1 : 0, rp_min, b->p.box_length, static_cast<int>(b->p.n_div), g, g + N, g + 2 * N,
-                       g + 3 * N, g + 4 * N, left, d_flag);
     if (check_split)
         hipLaunchKernelGGL(k_connected, dim3(blocks), dim3(kBlock), 0, st, b->d, idp, static_cast<int>(n),
                            b->p.box_length, d_flag);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipMemcpyAsync(b->h_grow, g, 5 * N * sizeof(double) + N * sizeof(int), hipMemcpyDeviceToHost, st));
-    int n_left = 0;
-    HIP_TRY(hipMemcpyAsync(&n_left, left, sizeof(int), hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
+    int all = 0;  // every aggregate's flags
     const int *h_flag = reinterpret_cast<const int *>(b->h_grow + 5 * N);
     for (size_t w = 0; w < N; ++w) {
         const int id = ids ? static_cast<int>(ids[w]) : b->alive_ids[w];
@@ -2079,9 +2080,10 @@ int mcac_box_grow_ids(mcac_box *b, const int64_t *ids, int64_t n_ids, double dr,
         radius_sum[id] = b->h_grow[2 * N + w];
         rg[id] = b->h_grow[3 * N + w];
         rmax[id] = b->h_grow[4 * N + w];
-        if (flags) flags[id] = h_flag[w];
+        all |= h_flag[w];
+        if (flags) flags[id] = h_flag[w] & (kGrowSmall | kGrowSplit);
     }
-    if (n_left > 0) b->cells_stale = true;  // else the search's copies were refreshed in place
+    if (all & kGrowLeft) b->cells_stale = true;  // else the search's copies were refreshed in place
     b->mirrors_exact = false;
     return 0;
 }
