@@ -177,8 +177,8 @@ int mcac_neighbour_order(int prev, const int64_t *keys, int m, int64_t *out);
  * per-sphere step the device kernel runs, exposed for host checks. */
 int mcac_arvo_part(int k, const double *x, const double *y, const double *z, const double *r, double out[2]);
 
-/* Groups of boxes: one queued move of each of many boxes in a single launch
- * (one workgroup per box).  No counterpart in the reference, which runs one box
+/* Groups of boxes: queued moves of many boxes in a single launch (one
+ * workgroup per move).  No counterpart in the reference, which runs one box
  * per process (src/main.cpp); for ensembles of small boxes, whose steps are
  * bound by launch and memory latency rather than by work.  A box joins a group
  * with no step in flight and then works on the group's stream (its own stream
@@ -190,9 +190,9 @@ int mcac_group_add(mcac_group *group, mcac_box *box);
 /* mcac_move_enqueue for n moves of boxes of the group: the moves of one box
  * are contiguous, in the order they are to run (at most 16 in flight per
  * box; past 8 of a box in one call the list goes to a further launch),
- * n <= 8 * max_boxes.  One launch takes every move that fits one workgroup,
- * one workgroup running each box's moves in order; the others take their
- * usual launches on the group stream, in order with the rest.  dirs holds 3
+ * n <= 8 * max_boxes.  One launch takes every move that fits one workgroup;
+ * a box's moves are searched side by side and carried out in order; the others
+ * take their usual launches on the group stream, in order with the rest.  dirs holds 3
  * doubles per move.  Results are read per box with mcac_move_result, contacts
  * and skipped moves handled as for mcac_move_enqueue.  On an error the moves
  * enqueued before the failing one keep their tickets and run. */

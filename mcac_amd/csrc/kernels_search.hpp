@@ -12,7 +12,10 @@
 //            runs the reference early-exit scan (aggregat_list.cpp:459-482),
 //            moves the aggregate (aggregat.cpp:148-161) when it is small, and
 //            publishes the result to pinned host memory.
-// k_step     both in one launch for small movers with few survivors.
+// k_step     both in one launch for small movers with few survivors; k_steps and
+//            k_steps_group do so for several consecutive steps of one box or of
+//            many, searched side by side and carried out in order by the block
+//            that finishes last.  k_step_grid: both in one launch for the others.
 // k_translate moves the spheres of a large mover.
 #pragma once
 #include "kernels_common.hpp"

@@ -7,9 +7,11 @@
 //               merge caches, member segment, reference Verlet cell (-1 dead)
 //   members     pool of sphere indices; aggregate a owns [start, start+cap)
 //   cell list   CSR by reference Verlet cell + dirty list (kernels_cells.hpp)
-// One MC step is two launches (k_filter, k_solve; plus k_translate for movers
-// of more than 1024 spheres) and no copy: the last block publishes a small
-// record into pinned host memory, which the host polls by sequence number.
+// Up to eight MC steps of a box share a launch (k_steps; k_steps_group for many
+// boxes, k_step for a single step); large movers take k_step_grid, and movers of
+// more than 1024 spheres k_translate besides.  No copy: the last block publishes
+// a small record per step into pinned host memory, which the host polls by
+// sequence number.
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
 
