@@ -18,6 +18,7 @@
 //            that finishes last.  k_step_grid: both in one launch for the others.
 // k_translate moves the spheres of a large mover.
 #pragma once
+#include "grid_form.hpp"
 #include "kernels_common.hpp"
 #include "kernels_merge.hpp"
 
@@ -998,6 +999,25 @@ __device__ __forceinline__ bool solve_tile(const DevBox &b, const SearchArgs &a,
     return true;
 }
 
+// The counters of a search's grid (grid_form.hpp).
+constexpr unsigned long long kGridWaitTicks = 2000000;  // 20 ms of the 100 MHz constant clock
+struct SearchGrid {
+    SearchState *s;
+    unsigned long long since = 0;
+    __device__ __forceinline__ void publish() const { release_to_device(); }
+    __device__ __forceinline__ void arrive() {
+        atomicAdd(&s->grid_bar, 1u);
+        since = wall_clock64();
+    }
+    __device__ __forceinline__ bool out_of_time() const { return wall_clock64() - since > kGridWaitTicks; }
+    __device__ __forceinline__ unsigned arrived() const {
+        return __hip_atomic_load(&s->grid_bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __device__ __forceinline__ void pause() const { __builtin_amdgcn_s_sleep(1); }
+    __device__ __forceinline__ void give_up() const { atomicExch(&s->grid_fail, 1u); }
+    __device__ __forceinline__ unsigned ticket() const { return atomicAdd(&s->done_solve, 1u); }
+};
+
 // Pair solve of the survivors filtered for step a: the tiles of the candidates'
 // spheres over the blocks of the grid, and the last block to finish reduces the
 // tiles' minima per candidate and finishes the step.
@@ -1048,12 +1068,9 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
     const long long W = want >= kBlock ? kBlock : (want <= 64 ? 64 : (want + 63) / 64 * 64);
     const long long tiles = (T + W - 1) / W;
     const bool planned = fits && tiles + F <= a.part_cap;
-    long long P;
     if (planned) {
         block_exclusive_scan(cpre, static_cast<int>(F));
-        P = (tiles < gridDim.x) ? (tiles > 0 ? tiles : 1) : gridDim.x;
-        if (blockIdx.x >= P) return;
-        for (long long g = blockIdx.x; g < tiles; g += P) {
+        for (long long g = blockIdx.x; g < tiles; g += gridDim.x) {
             const long long w0 = g * W, w = w0 + threadIdx.x, w1 = w0 + W < T ? w0 + W : T;
             const int c0 = last_not_above(cpre, static_cast<int>(F), w0);
             const int c1 = last_not_above(cpre, static_cast<int>(F), w1 - 1);
@@ -1081,9 +1098,7 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
             }
         }
     } else {  // very many survivors (or partials): a candidate at a time by a block
-        P = F < gridDim.x ? (F > 0 ? F : 1) : gridDim.x;
-        if (blockIdx.x >= P) return;
-        for (unsigned int c = blockIdx.x; c < F; c += static_cast<unsigned int>(P)) {
+        for (unsigned int c = blockIdx.x; c < F; c += gridDim.x) {
             const int k = b.cand_id[c];
             const long long nk = b.acount[k], sk = b.astart[k];
             double bd = kInf;
@@ -1106,9 +1121,8 @@ __device__ __forceinline__ void solve_phase(const DevBox &b, const SearchArgs &a
     }
     __syncthreads();  // the block's partials are written
     if (threadIdx.x == 0) {
-        release_to_device();
-        unsigned int ticket = atomicAdd(&b.ss->done_solve, 1u);
-        last = (ticket == static_cast<unsigned int>(P) - 1u);
+        SearchGrid grid{b.ss};
+        last = grid_part(grid, gridDim.x, blockIdx.x < (planned ? tiles : static_cast<long long>(F)));
     }
     __syncthreads();
     if (!last) return;
@@ -1166,7 +1180,6 @@ __global__ __launch_bounds__(kBlock) void k_solve(DevBox b, SearchArgs a) {
 // the CUs; one box stream, launches in order); a block that waits past kGridWaitTicks at the
 // barrier gives up and sets grid_fail, the step then publishes no record and
 // the host reports a device error instead of waiting without end.
-constexpr unsigned long long kGridWaitTicks = 2000000;  // 20 ms of the 100 MHz constant clock
 __global__ __launch_bounds__(kBlock) void k_step_grid(DevBox b, SearchArgs a) {
     if (behind_gate(b, a)) return;  // every block reads the same gate: the host knows it is skipped
     __shared__ StepLds lds;
@@ -1176,19 +1189,8 @@ __global__ __launch_bounds__(kBlock) void k_step_grid(DevBox b, SearchArgs a) {
     __shared__ int s_ok;
     if (threadIdx.x == 0) {
         if (tot) atomicAdd(&b.ss->nquery, tot);
-        release_to_device();  // this block's candidates and counts before its arrival
-        atomicAdd(&b.ss->grid_bar, 1u);
-        const unsigned long long t0 = wall_clock64();
-        int ok = 0;
-        while (wall_clock64() - t0 <= kGridWaitTicks) {
-            if (__hip_atomic_load(&b.ss->grid_bar, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= gridDim.x) {
-                ok = 1;
-                break;
-            }
-            __builtin_amdgcn_s_sleep(1);
-        }
-        if (!ok) atomicExch(&b.ss->grid_fail, 1u);
-        s_ok = ok;
+        SearchGrid grid{b.ss};
+        s_ok = grid_meet(grid, gridDim.x) ? 1 : 0;
     }
     __syncthreads();
     if (!s_ok) return;
