@@ -1298,7 +1298,8 @@ __device__ __forceinline__ int search_step(const DevBox &b, const SearchArgs &a,
     }
     const unsigned long long total = s_total;
     const unsigned int nfilt = static_cast<unsigned int>((total >> 32) & 0xffffffull);
-    const unsigned int most = vg > 1 ? static_cast<unsigned int>(share) : static_cast<unsigned int>(kStepCands);
+    // past the box's candidate capacity the grid form reports it
+    const unsigned int most = static_cast<unsigned int>(vg > 1 ? share : (a.cap < kStepCands ? a.cap : kStepCands));
     const unsigned int F = nfilt < most ? nfilt : most;
     const long long nsrc = a.n_mov;
     const int ssrc = a.start;
