@@ -1548,11 +1548,14 @@ __device__ __forceinline__ void set_moved(Moved &mv, int q, int src, const Args 
 // contact or hand-over and publishes their records (whole block).
 template <bool kCaps> __device__ __forceinline__ void commit_steps(const DevBox &b, StepsLds &u, int nj) {
     SearchState *s = b.ss;
-    int f = 0;
-    while (f < nj && !u.picks[f].handover && !(u.picks[f].dist <= u.args[f].lpm)) ++f;
+    // a step whose move the host does not know (the only one of its launch) is
+    // carried out as one with a contact; a lane looks at a step
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const bool stops = lane < nj && (!u.args[lane].nc_ok || u.picks[lane].handover || u.picks[lane].dist <= u.args[lane].lpm);
+    const unsigned long long stop = __ballot(stops);
+    const int f = stop ? __ffsll(static_cast<long long>(stop)) - 1 : nj;
     constexpr int kHead = static_cast<int>(offsetof(StepRecord, merge) / sizeof(unsigned long long));
     static_assert(offsetof(StepRecord, merge) % sizeof(unsigned long long) == 0, "record head in 8-byte words");
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     // moves without contact: a wave per step; a mover that moves again later in
     // the launch is placed by its last move
     for (int q = wave; q < f; q += kBlock / 64) {

@@ -590,9 +590,34 @@ bool mover_position(const mcac_box *b, size_t A, double com[3]) {
     return false;
 }
 
+// Brings the host mirrors up to date (surface growth moves every aggregate's
+// centre of mass); nothing of the box is in flight.
+int refresh_mirrors(mcac_box *b) {
+    const size_t A = static_cast<size_t>(b->n_aggs);
+    const double *const dev[7] = {b->d.ax, b->d.ay, b->d.az, b->d.arx, b->d.ary, b->d.arz, b->d.armax};
+    // the seven arrays lie one behind the other
+    std::vector<char> host(static_cast<size_t>(reinterpret_cast<const char *>(dev[6] + A) - reinterpret_cast<const char *>(dev[0])));
+    HIP_TRY(hipMemcpyAsync(host.data(), dev[0], host.size(), hipMemcpyDeviceToHost, bstream(b)));
+    HIP_TRY(hipStreamSynchronize(bstream(b)));
+    auto at = [&](int q, size_t a) {
+        double v;
+        std::memcpy(&v, host.data() + (reinterpret_cast<const char *>(dev[q] + a) - reinterpret_cast<const char *>(dev[0])), sizeof v);
+        return v;
+    };
+    for (size_t a = 0; a < A; ++a) {
+        Mirror &m = b->mir[a];
+        m.x = at(0, a), m.y = at(1, a), m.z = at(2, a);
+        m.rx = at(3, a), m.ry = at(4, a), m.rz = at(5, a);
+        m.rmax = at(6, a);
+    }
+    b->mirrors_exact = true;
+    return 0;
+}
+
 // Picks the launch of one step and enqueues it.  With run (given only for a
-// step that takes the one-launch form, known to the host and not timed) the
-// step is added there instead, for a launch by the caller.
+// step that takes the one-launch form and is not timed; the only one of its run
+// unless the host knows where its mover is) the step is added there instead, for
+// a launch by the caller.
 int enqueue_search(mcac_box *b, int64_t agg, const double dir[3], double lpm, double maxradius, int apply, int gated,
                    unsigned long long *ticket, StepRun *run = nullptr) {
     if (agg < 0 || agg >= b->n_aggs || b->count[static_cast<size_t>(agg)] <= 0) return MCAC_E_ARGUMENT;
@@ -1733,9 +1758,9 @@ int run_flush(Enqueue &e) {
     return 0;
 }
 
-// Adds one move of box b; first: the call's first move of it.
-int enqueue_move(Enqueue &e, mcac_box *b, bool first, int64_t agg, const double *dir, double lpm, double maxradius,
-                 uint64_t *ticket) {
+// Adds one move of box b; first: the call's first move of it; more: not its last.
+int enqueue_move(Enqueue &e, mcac_box *b, bool first, bool more, int64_t agg, const double *dir, double lpm,
+                 double maxradius, uint64_t *ticket) {
     StepRun &run = *e.run;
     int rc = 0;
     const bool valid = agg >= 0 && agg < b->n_aggs;
@@ -1754,13 +1779,21 @@ int enqueue_move(Enqueue &e, mcac_box *b, bool first, int64_t agg, const double 
         rc = timed([&] { return rebuild_cells(b); });
         if (rc) return rc;
     }
+    // steps side by side need the moves of those before them, so a box that has
+    // grown is read back for several; a single one reads its mover on the device
+    // (growth runs, one step a box between growths)
+    if (first && more && !b->mirrors_exact && b->inflight == 0 && (rc = refresh_mirrors(b)) != 0) return rc;
     // a step launched on its own, or the cell-list rebuild that the enqueue
     // launches, runs after the box's steps gathered or listed so far
     double com[3];
-    const bool batch = valid && b->eng_blocks == 0 &&
-                       one_block_step(b, b->count[static_cast<size_t>(agg)], next_step_timed(b)) &&
-                       mover_position(b, static_cast<size_t>(agg), com);
+    const bool one_block = valid && b->eng_blocks == 0 &&
+                           one_block_step(b, b->count[static_cast<size_t>(agg)], next_step_timed(b));
+    const bool known = one_block && mover_position(b, static_cast<size_t>(agg), com);
+    const bool alone = one_block && !known && e.several &&
+                       window_items(b, b->mir[static_cast<size_t>(agg)].rmax + maxradius + lpm) <= kBlockItems;
+    const bool batch = known || alone;
     const bool rebuild = rebuild_due(b) || b->cells_stale;
+    if (alone && (rc = run_flush(e)) != 0) return rc;
     if (!batch || rebuild) {
         if ((rc = run_flush(e)) != 0) return rc;
         if (e.l.last == b && (rc = group_flush(e)) != 0) return rc;
@@ -1771,7 +1804,7 @@ int enqueue_move(Enqueue &e, mcac_box *b, bool first, int64_t agg, const double 
     if (rc) return rc;
     *ticket = t;
     if (!batch && e.g) e.g->single_steps += 1;
-    return 0;
+    return alone ? run_flush(e) : 0;
 }
 
 }  // namespace
@@ -1797,8 +1830,8 @@ int mcac_move_enqueue_group(mcac_group *g, mcac_box *const *boxes, const int64_t
     for (int i = 1; i < n; ++i) e.several = e.several || boxes[i] != boxes[0];
     int rc = 0;
     for (int i = 0; i < n && rc == 0; ++i)
-        rc = enqueue_move(e, boxes[i], i == 0 || boxes[i - 1] != boxes[i], aggs[i], dirs + 3 * i, lpm[i], maxradius[i],
-                          tickets + i);
+        rc = enqueue_move(e, boxes[i], i == 0 || boxes[i - 1] != boxes[i], i + 1 < n && boxes[i + 1] == boxes[i], aggs[i],
+                          dirs + 3 * i, lpm[i], maxradius[i], tickets + i);
     // the steps enqueued before a failing one still run: their results are read as usual
     const int rrc = run_flush(e), frc = group_flush(e);
     g->t_enqueue += std::chrono::duration<double>(std::chrono::steady_clock::now() - t_in).count();
@@ -1815,7 +1848,7 @@ int mcac_move_enqueue_run(mcac_box *b, const int64_t *aggs, const double *dirs, 
     e.run->n = 0;
     int rc = 0;
     for (int i = 0; i < n && rc == 0; ++i)
-        rc = enqueue_move(e, b, i == 0, aggs[i], dirs + 3 * i, lpm[i], maxradius, tickets + i);
+        rc = enqueue_move(e, b, i == 0, i + 1 < n, aggs[i], dirs + 3 * i, lpm[i], maxradius, tickets + i);
     const int rrc = run_flush(e);
     return rc ? rc : rrc;
 }
