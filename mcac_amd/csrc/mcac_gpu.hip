@@ -123,11 +123,11 @@ struct mcac_box {
     size_t h_alpha_cap = 0;
     unsigned long long seq = 0;        // step tickets (searches)
     unsigned long long merge_seq = 0;  // merge records
-    // every buffer of the box in one allocation: one call to make and one to
-    // free instead of some 75, and the box's pages lie together (a step touches
-    // forty buffers, each a translation of its own when they are scattered)
+    // every buffer of the box but the member pool (which a compaction replaces)
+    // in one allocation: one call to make and one to free instead of some 75, and
+    // the box's pages lie together (a step touches forty buffers, each a
+    // translation of its own when they are scattered)
     char *arena = nullptr;
-    int *moved_members = nullptr;    // the member pool once a compaction has replaced it
     char *h_records = nullptr;       // pinned block of the records and the live-id staging
     int timing = 0;                  // 0 off; n >= 1: every n-th search is timed
     unsigned long long timing_base = 1;  // first ticket after timing was set: timed
@@ -466,8 +466,7 @@ int compact_pool(mcac_box *b, int64_t need) {
     }
     HIP_TRY(hipMemcpy(b->d.astart, b->start.data(), b->start.size() * sizeof(int), hipMemcpyHostToDevice));
     HIP_TRY(hipMemcpy(b->d.acap, b->cap.data(), b->cap.size() * sizeof(int), hipMemcpyHostToDevice));
-    if (b->moved_members) HIP_TRY(hipFree(b->moved_members));
-    b->moved_members = nm;
+    HIP_TRY(hipFree(b->d.members));
     b->d.members = nm;
     b->pool_cap = cap;
     b->pool_used = used;
@@ -923,9 +922,10 @@ BoxSizes box_sizes(const mcac_box_params &p) {
     return z;
 }
 
-// Every device buffer of a box, in allocation order: f(pointer, entries) is
-// called once per buffer (mcac_box_create allocates through it,
-// mcac_box_device_bytes adds the sizes up).  Returns the first non-zero f.
+// Every device buffer of a box but its member pool and the descriptor's copy, in
+// the order of the arena: f(pointer, entries) is called once per buffer
+// (mcac_box_create lays out through it, mcac_box_device_bytes adds the sizes up).
+// Returns the first non-zero f.
 template <class F> int box_buffers(DevBox &d, const BoxSizes &z, int volsurf, F &&f) {
     const int64_t Ns = z.Ns, Na = z.Na;
     int rc = 0;
@@ -937,7 +937,6 @@ template <class F> int box_buffers(DevBox &d, const BoxSizes &z, int volsurf, F 
     ALLOC(d.armax, Na); ALLOC(d.avol, Na); ALLOC(d.asurf, Na); ALLOC(d.arg, Na);
     ALLOC(d.csvx, Na); ALLOC(d.csvy, Na); ALLOC(d.csvz, Na); ALLOC(d.csr, Na); ALLOC(d.csvr2, Na);
     ALLOC(d.astart, Na); ALLOC(d.acount, Na); ALLOC(d.acell, Na); ALLOC(d.acap, Na);
-    ALLOC(d.members, z.pool_cap);
     ALLOC(d.alive, Na);
     ALLOC(d.cstart, z.n_cells + 1); ALLOC(d.citems, Na); ALLOC(d.ccursor, z.n_cells + 1);
     ALLOC(d.cpx, Na); ALLOC(d.cpy, Na); ALLOC(d.cpz, Na); ALLOC(d.cpr, Na); ALLOC(d.cslot, Na); ALLOC(d.cf, Na);
@@ -1079,8 +1078,9 @@ int64_t mcac_box_device_bytes(const mcac_box_params *params) {
         params->n_div > 1290 || params->volsurf < 0 || params->volsurf > 3)
         return -1;
     DevBox d{};
-    int64_t bytes = 0;
-    box_buffers(d, box_sizes(*params), params->volsurf, [&](auto *&ptr, int64_t n) {
+    const BoxSizes z = box_sizes(*params);
+    int64_t bytes = z.pool_cap * static_cast<int64_t>(sizeof(*d.members)) + static_cast<int64_t>(sizeof(DevBox));
+    box_buffers(d, z, params->volsurf, [&](auto *&ptr, int64_t n) {
         bytes += (n < 1 ? 1 : n) * static_cast<int64_t>(sizeof(*ptr));
         return 0;
     });
@@ -1126,6 +1126,10 @@ int mcac_box_create(const mcac_box_params *params, mcac_box **out) {
     lay_out();  // the size, then the addresses
     if (hipMalloc(reinterpret_cast<void **>(&b->arena), bytes) != hipSuccess) return fail(MCAC_E_DEVICE);
     lay_out();
+    if (hipMalloc(reinterpret_cast<void **>(&b->d.members), static_cast<size_t>(z.pool_cap) * sizeof(int)) != hipSuccess) {
+        b->d.members = nullptr;
+        return fail(MCAC_E_DEVICE);
+    }
     if (hipMemset(b->arena, 0, bytes) != hipSuccess) return fail(MCAC_E_DEVICE);
     rc = copy_descriptor(b);  // its wait covers the clearing before it
     if (rc) return fail(rc);
@@ -1160,7 +1164,7 @@ int mcac_box_destroy(mcac_box *b) {
     if (!b) return 0;
     if (b->stream) (void)hipStreamSynchronize(bstream(b));  // a resident engine ends first
     if (b->arena) (void)hipFree(b->arena);
-    if (b->moved_members) (void)hipFree(b->moved_members);
+    if (b->d.members) (void)hipFree(b->d.members);
     if (b->h_records) (void)hipHostFree(b->h_records);
     if (b->h_alpha) (void)hipHostFree(b->h_alpha);
     if (b->h_cstart) (void)hipHostFree(b->h_cstart);
