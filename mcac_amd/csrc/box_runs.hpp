@@ -5,6 +5,8 @@
 #include "../../include/mcac_gpu.h"
 
 extern "C" {
+// mcac_box_create and mcac_group_add in one, without a stream of the box's own.
+int mcac_box_create_in_group(const mcac_box_params *params, mcac_group *group, mcac_box **out);
 // mcac_move_enqueue for n moves of a box, in the order they are to run.  Moves
 // that take the one-launch form share launches of up to eight; the others take
 // their usual launches, in order with the rest.  On an error the moves enqueued

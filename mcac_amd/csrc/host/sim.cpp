@@ -300,10 +300,7 @@ struct Simulation {
         bp.device = device;
         bp.precision = precision;
         bp.volsurf = pm.volsurf;
-        int rc = mcac_box_create(&bp, &box);
-        if (rc) return rc;
-        if (group) rc = mcac_group_add(group, box);
-        return rc;
+        return group ? mcac_box_create_in_group(&bp, group, &box) : mcac_box_create(&bp, &box);
     }
     // Launch modes of an uploaded box: merges in the contact step's launch
     // (calcul.cpp:156-160 always merges on contact) unless a growth step must

@@ -271,10 +271,6 @@ void engine_stop(mcac_box *b) {
 // to end first.
 hipStream_t bstream(mcac_box *b) {
     engine_stop(b);
-    // a box that joins a group before its first work never makes one
-    if (!b->stream && (hipSetDevice(b->p.device) != hipSuccess ||
-                       hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess))
-        b->stream = nullptr;
     return b->stream;
 }
 
@@ -990,6 +986,10 @@ int scratch_address(int device, double **out) {
 }
 }  // namespace
 
+// A box on a stream of its own, or in a group from the start on the group's (no
+// stream is made only to be given up).
+static int create_box(const mcac_box_params *params, mcac_group *group, mcac_box **out);
+
 extern "C" {
 
 int mcac_swept_sphere_batch(int64_t n, const double *p1, const double *r1, const double *p2, const double *r2,
@@ -1087,8 +1087,14 @@ int64_t mcac_box_device_bytes(const mcac_box_params *params) {
     return bytes;
 }
 
-int mcac_box_create(const mcac_box_params *params, mcac_box **out) {
-    if (!params || !out) return MCAC_E_ARGUMENT;
+int mcac_box_create(const mcac_box_params *params, mcac_box **out) { return create_box(params, nullptr, out); }
+
+int mcac_box_create_in_group(const mcac_box_params *params, mcac_group *group, mcac_box **out) {
+    return group ? create_box(params, group, out) : MCAC_E_ARGUMENT;
+}
+
+static int create_box(const mcac_box_params *params, mcac_group *group, mcac_box **out) {
+    if (!params || !out || (group && group->device != params->device)) return MCAC_E_ARGUMENT;
     if (params->box_length <= 0 || params->n_div < 1 || params->n_div > 1290 || params->max_spheres < 1 ||
         params->max_aggregates < 1 || params->max_spheres > INT32_MAX / 2 || params->max_aggregates > INT32_MAX / 2 ||
         params->volsurf < 0 || params->volsurf > 3)
@@ -1106,6 +1112,14 @@ int mcac_box_create(const mcac_box_params *params, mcac_box **out) {
         return code;
     };
     if (hipSetDevice(params->device) != hipSuccess) return fail(MCAC_E_DEVICE);
+    if (group) {
+        b->stream = group->stream;
+        b->own_stream = false;
+        b->group = group;
+    } else if (hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) != hipSuccess) {
+        b->stream = nullptr;
+        return fail(MCAC_E_DEVICE);
+    }
     const BoxSizes z = box_sizes(*params);
     b->n_cells = static_cast<int>(z.n_cells);
     b->cand_cap = z.cand_cap;
@@ -1191,8 +1205,7 @@ int mcac_box_upload(mcac_box *b, int64_t ns, const double *x, const double *y, c
     const size_t S = static_cast<size_t>(ns), A = static_cast<size_t>(na);
     int rc = 0;
     HIP_TRY(hipSetDevice(b->p.device));
-    if (!bstream(b)) return MCAC_E_DEVICE;
-    HIP_TRY(hipStreamSynchronize(b->stream));
+    HIP_TRY(hipStreamSynchronize(bstream(b)));
     // a small box's state goes up in a few copies, put together on the host (the
     // buffers lie one behind the other); a large one's array by array
     constexpr size_t kStageBytes = size_t(4) << 20;
@@ -1648,10 +1661,8 @@ int mcac_group_destroy(mcac_group *g) {
 int mcac_group_add(mcac_group *g, mcac_box *b) {
     if (!g || !b || b->group || b->inflight || b->p.device != g->device) return MCAC_E_ARGUMENT;
     b->eng_blocks = 0;  // the group's launches take the box's steps
-    if (b->stream) {
-        HIP_TRY(hipStreamSynchronize(bstream(b)));
-        if (b->own_stream) HIP_TRY(hipStreamDestroy(b->stream));
-    }
+    HIP_TRY(hipStreamSynchronize(bstream(b)));
+    if (b->own_stream) HIP_TRY(hipStreamDestroy(b->stream));
     b->stream = g->stream;
     b->own_stream = false;
     b->group = g;
@@ -2138,7 +2149,6 @@ int mcac_box_set_engine(mcac_box *b, int blocks) {
     engine_stop(b);
     if (blocks > 0 && !b->h_ring) {
         HIP_TRY(hipSetDevice(b->p.device));
-        if (!bstream(b)) return MCAC_E_DEVICE;
         EngineJob *ring = nullptr;
         HIP_TRY(hipHostMalloc(reinterpret_cast<void **>(&ring), kEngineRing * sizeof(EngineJob), hipHostMallocCoherent));
         std::memset(static_cast<void *>(ring), 0, kEngineRing * sizeof(EngineJob));

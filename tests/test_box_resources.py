@@ -73,3 +73,25 @@ assert fake.fake_device_bytes() - before == 4 * (4 * pool - pool), (fake.fake_de
 box.close()
 assert fake.fake_device_bytes() == 0
 """)
+
+
+def test_a_stream_that_cannot_be_made_fails_the_creation(run):
+    run("""
+fake.fake_fail_streams(1)
+try:
+    m.Box(1e-6, 4, 8, 8)
+    raise SystemExit("created without a stream")
+except m.MCACError as e:
+    assert "status 32" in str(e)
+assert fake.fake_device_bytes() == 0 and fake.fake_streams() == 0
+fake.fake_fail_streams(0)
+box = m.Box(1e-6, 4, 8, 8)
+assert fake.fake_streams() == 1
+L, group = m.load_gpu(), ctypes.c_void_p()
+assert L.mcac_group_create(0, 2, ctypes.byref(group)) == 0 and fake.fake_streams() == 2
+assert L.mcac_group_add(group, box.h) == 0 and fake.fake_streams() == 1
+box.close()
+assert fake.fake_streams() == 1
+L.mcac_group_destroy(group)
+assert fake.fake_streams() == 0
+""")
