@@ -2184,13 +2184,15 @@ int mcac_box_engine_stats(mcac_box *b, double out[8]) {
 
 int mcac_box_set_timing(mcac_box *b, int enable) {
     if (!b) return MCAC_E_ARGUMENT;
-    if (enable > 0)  // the events of timed merges and steps, made on first use
+    if (enable > 0) {
+        HIP_TRY(hipSetDevice(b->p.device));  // an event belongs to the current device
+        // the events of timed merges and steps, made on first use
         for (auto &e : b->ev)
             if (!e) HIP_TRY(hipEventCreate(&e));
-    if (enable > 0)
         for (auto &row : b->sev)
             for (auto &e : row)
                 if (!e) HIP_TRY(hipEventCreate(&e));
+    }
     b->timing = enable < 0 ? 0 : enable;
     b->timing_base = b->seq + 1;  // the next search is the first timed one
     for (int k = 0; k < mcac_box::kRing; ++k) b->slot_timed[k] = 0;

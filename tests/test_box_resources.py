@@ -95,3 +95,13 @@ assert fake.fake_streams() == 1
 L.mcac_group_destroy(group)
 assert fake.fake_streams() == 0
 """)
+
+
+def test_timing_events_belong_to_the_box_device(run):
+    run("""
+far = m.Box(1e-6, 4, 8, 8, device=1)
+near = m.Box(1e-6, 4, 8, 8, device=0)
+before = [fake.fake_events(d) for d in range(2)]
+far.set_timing(1)
+assert fake.fake_events(0) == before[0] and fake.fake_events(1) > before[1]
+""")
