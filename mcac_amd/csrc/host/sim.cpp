@@ -141,7 +141,7 @@ struct Simulation {
     bool trace_steps = false, trace_merges = false;
     std::vector<mcac_step_rec> steps;
     std::vector<mcac_merge_rec> merge_recs;
-    double q_query = 0, q_filtered = 0, q_pairs = 0, n_ties = 0;
+    double q_query = 0, q_filtered = 0, q_pairs = 0, n_ties = 0, n_runs = 0;
     double t_pick = 0, t_merge_host = 0, t_device = 0, t_init = 0;
     double t_tie = 0, t_enqueue = 0, t_wait = 0, t_merge_call = 0, t_drain = 0;
     bool initialized = false;
@@ -698,15 +698,28 @@ struct Simulation {
         return true;
     }
 
+    // A pick among equal keys looks at every aggregate (17 ns each: 9 us at 500, 344
+    // us at 20000), and a contact of a step in flight takes it back.  It is made
+    // ahead of those as long as that is expected to cost less than the ~10 us that
+    // the device idles when it waits (boxes of equal monomers, where every pick is
+    // one); one that takes longer than a step waits for the launch of those gathered.
+    static constexpr double kTieWorth = 600.0;  // aggregates looked at in 10 us
+    bool tie_now(bool gathered) const {
+        const double n = static_cast<double>(live.size());
+        return n * (1.0 - std::pow(1.0 - p_contact, static_cast<double>(flight.size()))) < kTieWorth &&
+               !(gathered && n > kTieWorth);
+    }
+
     // The mover and move of the next step to issue (calcul.cpp:99-127).  Without
-    // settle a pick among equal keys is left open (num -1).
-    Pending pick_move(bool settle = true) {
+    // settle a pick among equal keys that should wait is left open (num -1);
+    // gathered: steps picked before it are not launched yet.
+    Pending pick_move(bool settle = true, bool gathered = false) {
         auto t0 = Clock::now();
         const Draw &d = draw_at(flight.size());
         size_t tie_pos = 0;
         int num = pick.pick_fast(d.u, &tie_pos);  // aggregat_list.cpp:59-66
         bool tie = false;
-        if (num < 0 && !settle) {
+        if (num < 0 && !settle && !tie_now(gathered)) {
             t_pick += ms_since(t0);
             return {0, -1, true, 0.0, d};
         }
@@ -747,10 +760,9 @@ struct Simulation {
         r_dirs.clear();
         r_lpm.clear();
         while (r_aggs.size() < most && !finished() && can_issue(consumed, max_steps)) {
-            // a pick among equal keys waits until nothing is in flight: it costs a sort of
-            // all keys, which a contact of a step before it would take back (10^6
-            // aggregates: ties took 6.0 us a step, now 1.9)
-            const Pending P = pick_move(flight.empty());
+            // a pick among equal keys may wait until nothing is in flight (10^6
+            // aggregates, one in 2000 steps: ties took 6.0 us a step made ahead, 1.9 so)
+            const Pending P = pick_move(false, !r_aggs.empty());
             if (P.num < 0) break;
             flight.push_back(P);
             r_aggs.push_back(P.num);
@@ -764,6 +776,7 @@ struct Simulation {
         int rc = mcac_move_enqueue_run(box, r_aggs.data(), r_dirs.data(), r_lpm.data(), maxradius, static_cast<int>(k),
                                        r_tickets.data());
         t_enqueue += ms_since(te0);
+        ++n_runs;
         if (rc) return rc;
         for (size_t q = 0; q < k; ++q) flight[flight.size() - k + q].ticket = r_tickets[q];
         return 0;
@@ -1610,6 +1623,7 @@ double mcac_sim_scalar(mcac_sim *sim, const char *name) {
     if (n == "filtered") return s.q_filtered;
     if (n == "pairs") return s.q_pairs;
     if (n == "ties") return s.n_ties;
+    if (n == "step_runs") return s.n_runs;
     if (n == "t_host_pick_ms") return s.t_pick;
     if (n == "t_host_merge_ms") return s.t_merge_host;
     if (n == "t_device_ms") return s.t_device;
