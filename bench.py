@@ -428,7 +428,8 @@ def main() -> int:
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS if achieved else None, "traffic": traffic,
                      "bytes_per_launch": bytes_per_launch, "avg_launch_ms": filt_ms,
                      "timed_launches": int(tm["n_search"]),
-                     "note": None if achieved else "no search was timed (events on every n-th search)"},
+                     "note": "timed: single steps in launches of their own on a drained queue; the others share k_steps "
+                             "launches" if achieved else "no search was timed (events on every n-th search)"},
         "candidate_pair_tests_per_s": pair_tests / elapsed,
         "breakdown": {"init_s": t_init, "host_pick_ms_per_step": d["t_host_pick_ms"] / steps,
                       "host_merge_ms_per_step": d["t_host_merge_ms"] / steps,

@@ -116,9 +116,11 @@ typedef struct mcac_merge_result {
 
 int mcac_box_create(const mcac_box_params *params, mcac_box **out);
 /* Device memory (bytes) mcac_box_create allocates for these parameters: the
- * sum of its buffer sizes, before the allocator's rounding (host computation,
- * no GPU call); -1 for invalid parameters.  No reference counterpart: it lets
- * a driver admit boxes by an HBM budget. */
+ * sum of its buffer sizes, before rounding (each of some 80 buffers to 256 bytes,
+ * and the allocator's own; host computation, no GPU call); -1 for invalid
+ * parameters.  A member pool that a compaction enlarges and the results of
+ * mcac_box_grow come on top when they are first needed.  No reference
+ * counterpart: it lets a driver admit boxes by an HBM budget. */
 int64_t mcac_box_device_bytes(const mcac_box_params *params);
 int mcac_box_destroy(mcac_box *box);
 
@@ -213,9 +215,10 @@ int mcac_group_times(mcac_group *group, double out[4]);
 int mcac_box_spare_moves(mcac_box *box);
 /* 1 when a move of the box whose sweep reaches `reach` (the mover's rmax +
  * maxradius + lpm) around its centre would currently run in one workgroup of
- * a group launch (its cell window holds few enough aggregates), else 0.  No
- * counterpart in the reference; lets a driver choose between group launches
- * and one launch per move. */
+ * a group launch (by the aggregates its cell window holds on average), else 0.
+ * The library asks the same of a mover whose position the host does not know
+ * (after surface growth).  No counterpart in the reference; lets a driver choose
+ * between group launches and one launch per move. */
 int mcac_box_block_steps(mcac_box *box, double reach);
 
 int mcac_box_download_spheres(mcac_box *box, double *x, double *y, double *z, double *rx, double *ry,

@@ -120,7 +120,7 @@ struct Simulation {
     bool rounds = true;               // several steps per launch (mcac_move_enqueue_run), else one launch each
     int engine_blocks = 0;            // persistent step engine grid (mcac_box_set_engine), 0: off
     std::vector<int64_t> r_aggs;      // scratch of issue_run
-    std::vector<double> r_dirs, r_lpm, r_maxr;
+    std::vector<double> r_dirs, r_lpm;
     std::vector<uint64_t> r_tickets;
     // spheres (index order) — host copy of the initial state only
     size_t N = 0;              // spheres in the box
@@ -750,7 +750,13 @@ struct Simulation {
     // probability of at least kWorth, by the rate p_contact of the last steps
     // (one at the rates of a dense box, eight below a fifth).  While the steps in
     // flight are more likely than not to run without a contact a second launch
-    // queues behind them, so that the picks overlap the device's work.
+    // queues behind them, so that the picks overlap the device's work.  Runs in ms,
+    // kWorth at 0.05 / 0.2 / 0.6: 500 monomers 30.7 / 30.9 / 29.6, 2347 111 / 115 /
+    // 124, 1500 at a volume fraction of 0.02 69 / 72 / 75, a dense box of 6000 302 /
+    // 292 / 291; kRate from 1/64 to 1/8 within 3 %; a second launch from a chance of
+    // 0.2 / 0.5 / never: 25.5 / 30.9 / 32.8, 115 / 115 / 116, 73 / 72 / 72, 292 / 292 /
+    // 292, and 50000 monomers from the start 31.3 / 36.8 / 37.6 (0.5 was taken unmeasured;
+    // lower is better where contacts are rare).
     static constexpr size_t kRunSteps = 8;
     static constexpr double kWorth = 0.2, kRate = 1.0 / 32.0;
     double p_contact = 0.0;

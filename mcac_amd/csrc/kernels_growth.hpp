@@ -164,8 +164,9 @@ __device__ __forceinline__ void grow_one(const DevBox &b, int at, int id, int n,
 // aggregates are small (kGrowPackedMean spheres on average); those of more than
 // kGrowWide spheres are left to the whole wave afterwards (else one large
 // aggregate would end long after the rest).  A call's time, a wave each -> eight
-// lanes: 100000 aggregates of 8 spheres 454 -> 307 us, 30000 of 16 224 -> 141,
-// 10000 of 16 139 -> 139, 25000 of 32 269 -> 277, 9000 of 32 138 -> 281.
+// lanes: 100000 aggregates of 8 spheres 436 -> 307 us (this kernel 44 us of it, the
+// copy back 79), 30000 of 16 201 -> 130, 10000 of 16 84 -> 59, 25000 of 32 244 ->
+// 263, 9000 of 32 109 -> 143.
 constexpr int kGrowPacked = 8192;  // aggregates: 256 compute units with 32 waves each
 constexpr int kGrowPackedMean = 16;
 constexpr int kGrowWide = 32;

@@ -1178,8 +1178,9 @@ __global__ __launch_bounds__(kBlock) void k_solve(DevBox b, SearchArgs a) {
 // blocks; the same arithmetic in the same order, so the same step.  The grid
 // is small enough to be resident at once (at most kFilterBlocks blocks, half
 // the CUs; one box stream, launches in order); a block that waits past kGridWaitTicks at the
-// barrier gives up and sets grid_fail, the step then publishes no record and
-// the host reports a device error instead of waiting without end.
+// barrier gives up and sets grid_fail, the step then publishes no record (the block
+// takes no ticket, so none is the last) and the host reports a device error instead
+// of waiting without end.
 __global__ __launch_bounds__(kBlock) void k_step_grid(DevBox b, SearchArgs a) {
     if (behind_gate(b, a)) return;  // every block reads the same gate: the host knows it is skipped
     __shared__ StepLds lds;
@@ -1503,7 +1504,11 @@ template <bool kCaps> __global__ __launch_bounds__(kBlock) void k_step(StepOne) 
 // finish carries the steps out in order up to the first contact (or hand-over),
 // behind which the others do nothing, as they would behind the gate.  Every
 // step sees the very values it would see in launches of its own.
-// Eight steps take about as long as one, plus one ticket between blocks.
+// A launch of up to eight takes 23.4 us on average (2347 monomers; a single step's
+// 7.6): the searches, a ticket among a step's blocks and one among the steps, then
+// the moves, their records and, on a contact, the merge, by one block.  Against
+// eight launches of one that is less than half; how the 16 us beyond a step divide
+// has not been measured.
 struct StepsLds {
     StepLds lds;
     StepCands sc;

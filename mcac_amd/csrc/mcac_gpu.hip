@@ -113,8 +113,8 @@ struct mcac_box {
     int slot_fused[kRing] = {0};
     int slot_solving[kRing] = {0};   // its grid form was launched before a cell-list rebuild
     int max_count = 0;               // upper bound of the aggregate sizes
-    int64_t n_handover = 0;          // k_step searches finished by k_solve
-    int64_t n_fused = 0, n_split = 0;  // searches launched as k_step / k_filter + k_solve
+    int64_t n_handover = 0;          // searches that a block left to the grid form
+    int64_t n_fused = 0, n_split = 0;  // searches launched for a block to finish / in the grid form
     int64_t n_compactions = 0;
     MergeRecord *h_merge = nullptr, *d_merge = nullptr;
     // alphas: the merge state and the merged aggregate's neighbour-map walk
@@ -476,11 +476,10 @@ int compact_pool(mcac_box *b, int64_t need) {
 
 int harvest_timing(mcac_box *b, int slot);
 
-// Blocks of the grid form for a mover of n_mov spheres: the filter grid,
-// widened to the sphere tiles that four survivors as large as the largest
-// aggregate would bring, at most grid_blocks (a block of it holds 75 KB of LDS;
-// all of them are resident together for its barrier, whose arrivals are
-// atomics on one counter).
+// Blocks of the grid form: the filter grid, widened to the sphere tiles that four
+// survivors as large as the largest aggregate would bring, at most grid_blocks (a
+// block of it holds 79 KB of LDS, two to a CU; all of them are resident together
+// for its barrier, whose arrivals are atomics on one counter).
 int grid_form_blocks(const mcac_box *b, int filter_grid) {
     const double tiles = std::ceil(4.0 * static_cast<double>(b->max_count) / 64);
     return std::min(b->grid_blocks, std::max(filter_grid, static_cast<int>(std::min<double>(kFilterBlocks, tiles))));
@@ -525,9 +524,17 @@ int settle_handovers(mcac_box *b) {
 // The one-launch form: the finishing block solves the survivors itself.  Its
 // solve takes about 2 us per 256 spheres of survivors and 64 spheres of mover,
 // so a narrow mover may meet large partners; a wide mover among wide partners
-// is spread over a grid (searches of 100-sphere movers among 150-sphere
-// aggregates: 11 us in one block, 24 us as a grid with its barrier; 700 x 700:
-// 109 us as a grid).
+// is spread over a grid.  A search in one block / as a grid with its barrier, us,
+// 1 to 8 survivors of the partners' size on the way:
+//   mover of     32      64      128     192     256     512 spheres
+//   partners 64  27/45   33/44   43/47   64/55   76/64
+//   256          22/36   32/40   37/44   81/51   64/63   99/83
+//   512          27/38   36/41   33/41   50/46   59/51   101/86
+//   1024         34/43   31/37   48/41   48/43   64/51   69/56
+//   4096         35/35   44/38   48/40   56/44   55/44   61/49
+// (from 192 spheres up most of the block's searches are handed over).  The grid is
+// the better one from 192 spheres; at 128 or fewer among partners past 1024 the two
+// lie within 8 us of each other.
 bool fits_one_launch(const mcac_box *b, int n_mov) {
     const long long worst = static_cast<long long>(n_mov) * b->max_count;
     return n_mov <= kStepMover && (worst <= kStepWorst || (n_mov <= kStepNarrow && worst <= kStepNarrowWorst));
