@@ -1,6 +1,6 @@
 """Grouped moves of boxes whose spheres have grown (the host no longer knows where
 their aggregates are) share launches, and give what the same moves give one at a
-time, bit for bit."""
+time, bit for bit; beside boxes that have not, and up to a move that is refused."""
 import ctypes
 
 import numpy as np
@@ -45,9 +45,9 @@ def test_grown_boxes_share_launches(sizes, k, n_boxes):
             t = enqueue(L, m, group, [p[0] for p in pairs for _ in range(k)], aggs.ravel(), dirs.reshape(-1, 3),
                         lpm.ravel(), maxr)
             assert L.mcac_group_stats(group, m._ip(stats)) == 0
-            if n_boxes > 1 or k > 1:
-                launches += 1
-                assert (stats[0], stats[1], stats[2]) == (launches, launches * n_boxes * k, 0)
+            launches += k  # a move of each box a launch
+            if n_boxes > 1:
+                assert (stats[0], stats[1], stats[2]) == (launches, launches * n_boxes, 0)
             for i, (box, one, _) in enumerate(pairs):
                 stopped = False
                 for q in range(k):
@@ -71,3 +71,49 @@ def test_grown_boxes_share_launches(sizes, k, n_boxes):
             box.close()
             one.close()
         L.mcac_group_destroy(group)
+
+
+@pytest.mark.parametrize("bad", [None, 2, 9, 13])
+def test_grown_boxes_beside_others(bad):
+    """Four boxes with four moves each, every other one grown: all run, or those before
+    the move that is refused do."""
+    import mcac_amd as m
+    print(f"case: grown boxes beside others, refused move {bad}", flush=True)
+    L, group, k, n = m.load_gpu(), ctypes.c_void_p(), 4, 30
+    side = 2e-6
+    assert L.mcac_group_create(0, 4, ctypes.byref(group)) == 0
+    pairs = []
+    for i in range(4):
+        made = [make_box((1,) * n, side, np.random.default_rng(i), 0) for _ in range(2)]
+        pairs.append((made[0][0], made[1][0], made[0][3]))
+        assert L.mcac_group_add(group, made[0][0].h) == 0
+        if i % 2:
+            for b in pairs[-1][:2]:
+                grow(L, m, b, 1e-10)
+    maxr = 1.1 * max(p[2] for p in pairs)
+    rng = np.random.default_rng(3)
+    aggs = rng.integers(0, n, 4 * k)
+    dirs = rng.normal(size=(4 * k, 3))
+    dirs /= np.linalg.norm(dirs, axis=1)[:, None]
+    lpm = np.full(4 * k, 1e-9)
+    if bad is not None:
+        aggs[bad] = n
+    arr = (ctypes.c_void_p * (4 * k))(*[pairs[i // k][0].h for i in range(4 * k)])
+    t = (ctypes.c_uint64 * (4 * k))()
+    rc = L.mcac_move_enqueue_group(group, arr, m._ip(aggs), m._dp(dirs.ravel()), m._dp(lpm), m._dp(np.full(4 * k, maxr)),
+                                   4 * k, t)
+    assert rc == (0 if bad is None else 34)
+    for i in range(4 * k if bad is None else bad):
+        box, one, _ = pairs[i // k]
+        got, skipped = box.move_result(t[i])
+        assert skipped == 0
+        ref = one.next_contact(int(aggs[i]), dirs[i], float(lpm[i]), maxr, move=True)
+        assert got["distance"] == ref["distance"] and got["contact"] == ref["contact"] == 0
+    for box, one, _ in pairs:
+        if bad is not None:  # nothing else is in flight
+            assert L.mcac_box_spare_moves(box.h) == 16
+        for f, v in one.spheres().items():
+            assert np.array_equal(v, box.spheres()[f]), f
+        box.close()
+        one.close()
+    L.mcac_group_destroy(group)
