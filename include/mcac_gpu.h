@@ -193,7 +193,8 @@ int mcac_group_add(mcac_group *group, mcac_box *box);
  * are contiguous, in the order they are to run (at most 16 in flight per
  * box; past 8 of a box in one call the list goes to a further launch),
  * n <= 8 * max_boxes.  One launch takes every move that fits one workgroup;
- * a box's moves are searched side by side and carried out in order; the others
+ * a box's moves are searched side by side and carried out in order (after
+ * surface growth one move of a box per launch); the others
  * take their usual launches on the group stream, in order with the rest.  dirs holds 3
  * doubles per move.  Results are read per box with mcac_move_result, contacts
  * and skipped moves handled as for mcac_move_enqueue.  On an error the moves
